@@ -95,7 +95,7 @@ int tfsm_version(void);
  * Any mesh of >= 2 points per axis is accepted (the reference transforms any length,
  * mesh.py:481-491).  The fused step kernels cover 1D powers of two 32..4096 and 48, 96, 100, 112,
  * 192, 200, 384, 400, 768, 800 points; 2D axes of powers of two 16..1024 and 48, 96, 100, 112, 192,
- * 200; 3D axes of powers of two 16..128 and cubic 48, 96, 100 meshes.  Other plans (other sizes,
+ * 200; 3D axes of powers of two 16..256 and cubic 48, 96, 100 meshes.  Other plans (other sizes,
  * ConservativeConvection in 3D, a complex L with a product term in 2D / 3D, NSPressureConvection
  * with an external force, tfsm_plan_add_force) step through the
  * unfused path: separate field, product and stage launches with general-length FFTs (Stockham with
@@ -137,7 +137,7 @@ int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int
  * NSPressureConvection (16 samples from B = 32, 8 at B = 16..31) and 256^2 VorticityConvection
  * and Convection (16 samples, B >= 32; four streams from B = 64); 3D: radix-4
  * z rows from 64 points, and for Convection and NSPressureConvection sub-batches of 2 on two
- * streams at 128^3 with 4 or more samples, on four streams at 64^3 with 8 or more).
+ * streams at 128^3 with 4 or more samples and at 256^3 with 2 or more, on four streams at 64^3 with 8 or more).
  * (No reference counterpart: launch configuration.) */
 int tfsm_plan_get_tuning(const tfsm_plan* plan, int32_t* out);
 

@@ -723,8 +723,8 @@ hipError_t launch_col3d(const Col3Args& a, int nb, int stage, int col_var, hipSt
 hipError_t launch_yinv3d(const Yinv3Args& a, int col_var, hipStream_t st);
 hipError_t launch_row3d(const Row3Args& a, int row_var, hipStream_t st);
 bool step3d_supported(int n0, int n1, int n2);
-// radix-plan variant used by the 3D kernels for an axis of length n
-inline int var3(int n) { return n == 128 ? 2 : 0; }
+// radix-plan variant used by the 3D kernels for an axis of length n (128 and 256: 8 values per thread)
+constexpr int var3(int n) { return n == 128 ? 2 : (n == 256 ? 1 : 0); }
 hipError_t launch_linear_symbol(const LinArgs& a, hipStream_t st);
 hipError_t launch_axis_row(float* kv, int n, float s, hipStream_t st);
 hipError_t launch_coefs(const CoefArgs& a, hipStream_t st);

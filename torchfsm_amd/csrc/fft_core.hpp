@@ -223,6 +223,7 @@ template <> struct FftPlan<16, 3> { static constexpr int RMAX = 4; static conste
 template <> struct FftPlan<32, 3> { static constexpr int RMAX = 4; static constexpr int NST = 3; static constexpr int R[5] = {4, 4, 2, 0, 0}; };
 template <> struct FftPlan<64, 3> { static constexpr int RMAX = 4; static constexpr int NST = 3; static constexpr int R[5] = {4, 4, 4, 0, 0}; };
 template <> struct FftPlan<128, 3> { static constexpr int RMAX = 4; static constexpr int NST = 4; static constexpr int R[5] = {4, 4, 4, 2, 0}; };
+template <> struct FftPlan<256, 3> { static constexpr int RMAX = 4; static constexpr int NST = 4; static constexpr int R[5] = {4, 4, 4, 4, 0}; };
 
 template <int N, int VAR = 0>
 struct Fft {

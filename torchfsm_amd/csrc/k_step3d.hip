@@ -405,6 +405,7 @@ __global__ void __launch_bounds__((Fft<N2, VAR>::NT * ROWS)) k3_row(Row3Args a) 
     case 32: { constexpr int NN = 32; __VA_ARGS__ }    \
     case 64: { constexpr int NN = 64; __VA_ARGS__ }    \
     case 128: { constexpr int NN = 128; __VA_ARGS__ }  \
+    case 256: { constexpr int NN = 256; __VA_ARGS__ }  \
     case 48: { constexpr int NN = 48; __VA_ARGS__ }  \
     case 96: { constexpr int NN = 96; __VA_ARGS__ }  \
     case 100: { constexpr int NN = 100; __VA_ARGS__ }  \
@@ -412,10 +413,10 @@ __global__ void __launch_bounds__((Fft<N2, VAR>::NT * ROWS)) k3_row(Row3Args a) 
   }
 
 // Convection column kernels also compiled per ETDRK2 / SETDRK2 and SETDRK4 stage (and for the
-// field pass of the initial state): the 64- and 128-point x columns with the default radix plan
+// field pass of the initial state): the 64-, 128- and 256-point x columns with the default radix plan
 template <int NN, int VR>
 struct Col3StageKernels {
-  static constexpr bool value = (NN == 64 || NN == 128) && VR == (NN == 128 ? 2 : 0);
+  static constexpr bool value = (NN == 64 || NN == 128 || NN == 256) && VR == var3(NN);
 };
 
 template <int NN, int VR>
@@ -464,7 +465,7 @@ hipError_t launch_col3d(const Col3Args& a, int nb, int stage, int col_var, hipSt
     if constexpr (!is_mixed_size(NN)) {
       if (col_var == 1) return launch_col3d_t<NN, 3>(a, nb, stage, st);
     }
-    return launch_col3d_t<NN, (NN == 128 ? 2 : 0)>(a, nb, stage, st);
+    return launch_col3d_t<NN, var3(NN)>(a, nb, stage, st);
   })
 }
 
@@ -473,7 +474,7 @@ hipError_t launch_yinv3d(const Yinv3Args& a, int col_var, hipStream_t st) {
     if constexpr (!is_mixed_size(NN)) {
       if (col_var == 1) return launch_yinv3d_t<NN, 3>(a, st);
     }
-    return launch_yinv3d_t<NN, (NN == 128 ? 2 : 0)>(a, st);
+    return launch_yinv3d_t<NN, var3(NN)>(a, st);
   })
 }
 
@@ -511,13 +512,15 @@ hipError_t launch_row3d(const Row3Args& a, int row_var, hipStream_t st) {
     if constexpr (!is_mixed_size(NN)) {
       if (row_var == 1) return launch_row3d_t<NN, 3>(a, st);
     }
-    return launch_row3d_t<NN, (NN == 128 ? 2 : 0)>(a, st);
+    return launch_row3d_t<NN, var3(NN)>(a, st);
   })
 }
 
-// powers of two 16..128 per axis, or a cubic mesh of one of the mixed-radix 3D sizes
+// Powers of two 16..256 per axis (the 256-point column tiles hold 512 threads of 8 values; Burgers
+// 256^3 ETDRK2 takes 1.64 ms/step here against 5.1 on the unfused path, which moves about 3.5 times
+// the bytes; 4 values per thread in the columns: 1.77, 8 in the z rows: 1.82), or a cubic mesh of one of the mixed-radix 3D sizes
 bool step3d_supported(int n0, int n1, int n2) {
-  auto ok = [](int n) { return n == 16 || n == 32 || n == 64 || n == 128; };
+  auto ok = [](int n) { return n == 16 || n == 32 || n == 64 || n == 128 || n == 256; };
   if (ok(n0) && ok(n1) && ok(n2)) return true;
   return n0 == n1 && n1 == n2 && is_mixed_size_3d(n0);
 }
