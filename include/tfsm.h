@@ -94,7 +94,8 @@ int tfsm_version(void);
 /* Compile an operator on a mesh into a plan: symbols, dealias limits, twiddle tables, L.
  * Any mesh of >= 2 points per axis is accepted (the reference transforms any length,
  * mesh.py:481-491).  The fused step kernels cover 1D powers of two 32..4096 and 48, 96, 100, 112,
- * 192, 200, 384, 400, 768, 800 points; 2D axes of powers of two 16..1024 and 48, 96, 100, 112, 192,
+ * 192, 200, 384, 400, 768, 800 points, and 1D products above 4096 of two of those lengths from 64 to
+ * 1024 (Convection and ConservativeConvection with a real L); 2D axes of powers of two 16..1024 and 48, 96, 100, 112, 192,
  * 200; 3D axes of powers of two 16..256 and cubic 48, 96, 100 meshes.  Other plans (other sizes,
  * ConservativeConvection in 3D, a complex L with a product term in 2D / 3D, NSPressureConvection
  * with an external force, tfsm_plan_add_force) step through the

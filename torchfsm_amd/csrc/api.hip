@@ -146,6 +146,9 @@ struct tfsm_plan {
   size_t off_A1 = 0, off_A2 = 0, off_P = 0, off_G = 0, off_G2 = 0, ws_bytes = 0;
   size_t off_DC = 0;              // KSConvection: batch mean of the product DC (one complex value)
   size_t off_S = 0, off_N = 0;    // 1D KSConvection: stage spectrum and raw product spectrum
+  // long 1D meshes (k_long1d.hip): N = l1 l2, field and product pitch PF
+  int l1 = 0, l2 = 0;
+  float2 *ltw1 = nullptr, *ltw2 = nullptr, *ltw4 = nullptr;
   std::vector<void*> allocs;
   // adjoint (tfsm_adjoint_prepare)
   float* dcoef = nullptr;  // [Bc][3][modes]
@@ -263,6 +266,29 @@ int build_twiddles(tfsm_plan* p, int d) {
     if (rc) return rc;
     HIP_TRY(hipMemcpy(p->tw[d][var], h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice), "twiddle upload");
   }
+  return TFSM_OK;
+}
+
+// tables of a long 1D mesh: stage twiddles of both factors and the four-step twiddles of the kept columns
+int build_long1d(tfsm_plan* p) {
+  const int len[2] = {p->l1, p->l2};
+  float2** dst[2] = {&p->ltw1, &p->ltw2};
+  for (int i = 0; i < 2; ++i) {
+    std::vector<float2> h;
+    if (!twiddle_table(len[i], long1d_var(len[i]), h)) return fail(TFSM_E_INVALID, "no radix plan for this length");
+    int rc = dev_alloc(p, dst[i], h.size(), "twiddle table");
+    if (rc) return rc;
+    HIP_TRY(hipMemcpy(*dst[i], h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice), "twiddle upload");
+  }
+  std::vector<float2> h((size_t)p->l1 * p->PF, make_float2(0.f, 0.f));
+  for (int x1 = 0; x1 < p->l1; ++x1)
+    for (int q2 = 0; q2 <= p->l2 / 2; ++q2) {
+      const double ang = -2.0 * M_PI * (double)((long long)x1 * q2) / (double)p->n[0];
+      h[(size_t)x1 * p->PF + q2] = make_float2((float)std::cos(ang), (float)std::sin(ang));
+    }
+  int rc = dev_alloc(p, &p->ltw4, h.size(), "four-step twiddles");
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(p->ltw4, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice), "twiddle upload");
   return TFSM_OK;
 }
 
@@ -680,6 +706,40 @@ int run3d_eval(tfsm_plan* p, float2* U, char* ws, int stage, int b0, int nb, hip
   return TFSM_OK;
 }
 
+// one nonlinear evaluation of a long 1D mesh (row pass, then column pass with the stage combine)
+int run_long1d(tfsm_plan* p, float2* U, char* ws, int stage, hipStream_t st) {
+  Long1Args a;
+  a.B = p->B * p->C;
+  a.N = p->n[0];
+  a.L1 = p->l1;
+  a.L2 = p->l2;
+  a.P = p->P;
+  a.PG = p->PF;
+  a.kmax = p->kmax[0];
+  a.coef_t = p->coef_t;
+  a.scale = (float)(1.0 / p->n[0]);
+  a.tw1 = p->ltw1;
+  a.tw2 = p->ltw2;
+  a.tw4 = p->ltw4;
+  a.ax = p->kv[0];
+  a.ax_bstride = p->kv_bstride;
+  a.U = U;
+  a.A1 = (float2*)(ws + p->off_A1);
+  a.A2 = (float2*)(ws + p->off_A2);
+  a.cpk = p->cpk;
+  a.cpk_bstride = p->Bc > 1 ? 2 * p->modes : 0;
+  a.c5t = p->c5t;
+  a.src = p->src;
+  a.src_bstride = p->src_bstride();
+  a.Pr = (const float2*)(ws + p->off_P);
+  a.Pw = (float2*)(ws + p->off_P);
+  a.G = (float2*)(ws + p->off_G);
+  a.cons = p->term == TERM_CONS ? 1 : 0;
+  if (stage != ST_PRO) HIP_TRY(launch_long1d_row(a, st), "1D row launch");
+  HIP_TRY(launch_long1d_col(a, stage, st), "1D column launch");
+  return TFSM_OK;
+}
+
 int run_eval(tfsm_plan* p, float2* U, char* ws, int stage, int b0, int nb, hipStream_t st, StepMask m = StepMask()) {
   return p->D == 3 ? run3d_eval(p, U, ws, stage, b0, nb, st, 15, m) : run2d_eval(p, U, ws, stage, b0, nb, st, m);
 }
@@ -748,6 +808,18 @@ int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* tra
         if (dc) HIP_TRY(launch_ks_dc(Nr, a.B, (size_t)p->P, 1, 0, dc, st), "batch-mean launch");
         HIP_TRY(launch_k1_stage(a, scheme_stage(p->scheme, e), Nr, dc, S, st), "1D stage launch");
       }
+    }
+    if (rec_slot) HIP_TRY(launch_record(U, (float2*)traj, rec_slot, nsteps, p->B, per, T, st), "record launch");
+    return TFSM_OK;
+  }
+  if (p->D == 1 && p->l1) {
+    const int nev = scheme_evals(p->scheme);
+    const size_t per = (size_t)p->C * p->modes;
+    if (int rc = run_long1d(p, U, (char*)ws, ST_PRO, st)) return rc;
+    for (int i = 0; i < nsteps; ++i) {
+      if (rec_slot) HIP_TRY(launch_record(U, (float2*)traj, rec_slot, i, p->B, per, T, st), "record launch");
+      for (int e = 0; e < nev; ++e)
+        if (int rc = run_long1d(p, U, (char*)ws, scheme_stage(p->scheme, e), st)) return rc;
     }
     if (rec_slot) HIP_TRY(launch_record(U, (float2*)traj, rec_slot, nsteps, p->B, per, T, st), "record launch");
     return TFSM_OK;
@@ -925,6 +997,10 @@ int adj_jt(tfsm_plan* p, const float2* U, const float2* V, float2* W, char* wsa,
 // N(U) -> workspace A1
 int eval_nonlinear(tfsm_plan* p, float2* U, char* ws, hipStream_t st) {
   if (p->general) return gen_stage(p, U, U, ws, ST_EVAL, StepMask(), st);
+  if (p->l1) {
+    int rc = run_long1d(p, U, ws, ST_PRO, st);
+    return rc ? rc : run_long1d(p, U, ws, ST_EVAL, st);
+  }
   if (p->D == 1) {
     Run1Args r = run1_args(p, U, ws);
     r.eval_only = 1;
@@ -1189,6 +1265,11 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
   bool fused = fused_sizes && !(term == TERM_CONS && D == 3) && !(cplx && term != TERM_NONE && D > 1);
   if (fused && D == 3 && term != TERM_NONE && term != TERM_CONS)
     fused = step3d_supported(geom->n[0], geom->n[1], geom->n[2]);
+  // long 1D meshes that split into two fixed-size lengths (k_long1d.hip)
+  int l1 = 0, l2 = 0;
+  if (D == 1 && !fused_sizes && !cplx && geom->channels == 1 && (term == TERM_CONV || term == TERM_CONS) &&
+      geom->n[0] > 4096 && long1d_split(geom->n[0], &l1, &l2))
+    fused = true;
   if (terms->n_linear > 0 && !terms->linear_coef) return fail(TFSM_E_INVALID, "linear coefficients missing");
   const int Bc = terms->coef_batch < 1 ? 1 : terms->coef_batch;
   if (Bc != 1 && Bc != geom->batch) return fail(TFSM_E_INVALID, "coef_batch must be 1 or the batch size");
@@ -1226,6 +1307,8 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
   p->cplx = cplx;
   p->fused_ok = fused;
   p->general = !fused && term != TERM_NONE;
+  p->l1 = l1;
+  p->l2 = l2;
   p->per_len = D == 1 && geom->length_per_sample;
   p->Bc = Bc;
   int rc = TFSM_OK;
@@ -1239,6 +1322,10 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     if (rc) break;
   }
   if (!rc) rc = build_gaxes(p);
+  if (!rc && p->l1) {
+    p->PF = (int)roundup((size_t)p->l2 / 2 + 1, 16);
+    rc = build_long1d(p);
+  }
   // axis wavenumber tables
   if (!rc) {
     for (int d = 0; d < D && !rc; ++d) {
@@ -1342,6 +1429,11 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
       // ConservativeConvection keeps two product planes per channel
       p->off_G = p->off_P + roundup(term == TERM_CONS ? 2 * sb : sb, 256);
       p->ws_bytes = p->off_G + roundup((size_t)p->B * p->NF * p->n[0] * p->PF * sizeof(float2), 256);
+    } else if (p->l1) {
+      const size_t plane = (size_t)p->B * p->l1 * p->PF * sizeof(float2);
+      p->off_P = p->off_A2 + roundup(sb, 256);
+      p->off_G = p->off_P + roundup(plane, 256);
+      p->ws_bytes = p->off_G + roundup((term == TERM_CONS ? 1 : 2) * plane, 256);
     } else {
       p->ws_bytes = p->off_A2 + roundup(sb, 256);
       if (term == TERM_KS) {
@@ -1864,6 +1956,8 @@ int tfsm_apply(tfsm_plan* p, const void* uh, void* out, void* ws, void* stream) 
     if (!ws) return fail(TFSM_E_INVALID, "workspace pointer is null");
     if (p->general) {
       if (int rc = gen_stage(p, U, U, (char*)ws, ST_EVAL, StepMask(), st)) return rc;
+    } else if (p->l1) {
+      if (int rc = eval_nonlinear(p, U, (char*)ws, st)) return rc;
     } else if (p->D == 1 && p->term == TERM_KS) {
       Run1Args a = run1_args(p, U, (char*)ws);
       float2* Nr = (float2*)((char*)ws + p->off_N);
@@ -2003,6 +2097,7 @@ int tfsm_launch_pass(tfsm_plan* p, void* uh, void* ws, int32_t pass_id, int32_t 
   if (p->D == 1 && pass_id == 2) {
     if (p->scheme < 0) return fail(TFSM_E_STATE, "no scheme set on the plan");
     if (p->term == TERM_KS) return fail(TFSM_E_INVALID, "1D KSConvection steps stage by stage (tfsm_step)");
+    if (p->l1) return fail(TFSM_E_INVALID, "long 1D meshes step stage by stage (tfsm_step)");
     Run1Args a = run1_args(p, (float2*)uh, (char*)ws);
     a.nsteps = 1;
     HIP_TRY(launch_run1d(a, st), "1D stepper launch");

@@ -639,6 +639,26 @@ struct Run1Args {
 };
 
 
+// long 1D meshes (k_long1d.hip): N = L1 L2, columns q2 = 0..L2/2 at pitch PG
+struct Long1Args {
+  int B, N, L1, L2, P, PG, kmax;
+  float coef_t, scale;
+  const float2 *tw1, *tw2;    // stage twiddles of L1 and L2
+  const float2* tw4;          // [L1][PG] exp(-2 pi i q2 x1 / N)
+  const float* ax;
+  size_t ax_bstride;
+  float2 *U, *A1, *A2;
+  const float4* cpk;
+  size_t cpk_bstride;
+  const float* c5t;
+  const float2* src;
+  size_t src_bstride;
+  const float2* Pr;           // product rows [B][L1][PG] (read by the column pass)
+  float2* Pw;                 // the same, written by the row pass
+  float2* G;                  // fields [B][NF][L1][PG]
+  int cons = 0;               // ConservativeConvection (one field)
+};
+
 enum LinKind : int { LIN_LAP = 1, LIN_BIHARM = 2, LIN_UNIT = 3, LIN_DERIV = 4 };
 
 struct LinArgs {
@@ -719,6 +739,11 @@ hipError_t launch_k1_stage(const Run1Args& a, int stage, const float2* Nraw, con
 // out = (1/B) sum_b sum_x P[b * bstride + x * xstride]: the DC of the product spectra averaged over
 // the batch (KSConvection's remove_mean subtracts the mean over batch and space)
 hipError_t launch_ks_dc(const float2* P, int B, size_t bstride, int nx, size_t xstride, float2* out, hipStream_t st);
+// long 1D meshes: the split of N (false: none), the radix-plan variant of a factor, and the passes
+bool long1d_split(int n, int* l1, int* l2);
+int long1d_var(int n);
+hipError_t launch_long1d_row(const Long1Args& a, hipStream_t st);
+hipError_t launch_long1d_col(const Long1Args& a, int stage, hipStream_t st);
 hipError_t launch_col3d(const Col3Args& a, int nb, int stage, int col_var, hipStream_t st);
 hipError_t launch_yinv3d(const Yinv3Args& a, int col_var, hipStream_t st);
 hipError_t launch_row3d(const Row3Args& a, int row_var, hipStream_t st);
