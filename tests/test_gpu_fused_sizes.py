@@ -137,3 +137,46 @@ def test_long_1d_recorder_and_gradient(dev):
         op.integrate(x, dt=2e-4, step=5).square().sum().backward()
         grads.append(x.grad)
     assert _rel(grads[0], grads[1]) <= TOL
+
+
+@pytest.mark.parametrize("n,batch", [(32, 1), (64, 5), (96, 9), (100, 13), (112, 3), (128, 3), (256, 2), (512, 2), (768, 1), (800, 2),
+                                     (1024, 2), (2048, 3), (4096, 1)])
+def test_1d_stepper_lengths_and_batches(dev, n, batch):
+    """The persistent 1D stepper at every kind of radix plan and at batches that leave part of a workgroup
+    idle: Convection (SETDRK3) and ConservativeConvection (SETDRK4) with per-sample coefficients and a
+    source, per-sample step counts, and a complex L, against the oracle."""
+    from oracle import refpath
+    from torchfsm_amd.engine import SpectralPlan
+
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.arange(n, device=dev) / n
+    amp = torch.rand(batch, 1, 1, generator=g, device=dev)
+    u = (amp * torch.sin(2 * math.pi * x) + 0.3 + 0.02 * torch.randn(batch, 1, n, generator=g, device=dev)).contiguous()
+    src = torch.randn(1, 1, n, generator=g, device=dev)
+    dt, mi = 0.1 / n, [(0, 1.0, n)]
+    nus = [0.02 + 0.01 * b for b in range(batch)]
+    for kind, scheme in (("conv", "SETDRK3"), ("cons", "SETDRK4")):
+        plan = SpectralPlan(mi, batch, 1, nonlinear=kind, nonlinear_coef=-1.0,
+                            linear=[("lap", nus if batch > 1 else nus[0])], device=dev)
+        plan.add_source(src, 0.2)
+        plan.set_scheme(scheme, dt)
+        uh = plan.forward(u)
+        plan.step(uh, 6)
+        out = plan.inverse(uh)
+        counts = torch.arange(batch, device=dev, dtype=torch.int32)
+        uv = plan.forward(u)
+        plan.step_varying(uv, counts, 6)
+        part = plan.inverse(uv)
+        for b in range(0, batch, 2):
+            terms = [(nus[b], "lap", None), (-1, kind, None), (0.2, "src", src)]
+            assert _rel(out[b:b + 1], refpath.integrate(terms, mi, u[b:b + 1], dt, 6, scheme=scheme)) <= TOL
+            if 0 < b <= 6:
+                assert _rel(part[b:b + 1], refpath.integrate(terms, mi, u[b:b + 1], dt, b, scheme=scheme)) <= TOL
+        assert _rel(part[:1], u[:1]) <= TOL
+    plan = SpectralPlan(mi, batch, 1, nonlinear="conv", nonlinear_coef=-1.0, linear=[(("deriv", 0, 3), -1e-4), ("lap", 0.02)],
+                        device=dev)
+    plan.set_scheme("SETDRK4", dt)
+    uh = plan.forward(u)
+    plan.step(uh, 5)
+    terms = [(-1e-4, "deriv", (0, 3)), (0.02, "lap", None), (-1, "conv", None)]
+    assert _rel(plan.inverse(uh), refpath.integrate(terms, mi, u, dt, 5, scheme="SETDRK4")) <= TOL

@@ -251,6 +251,8 @@ bool twiddle_table(int n, int var, std::vector<float2>& h) {
     case 256: twiddle_table_t<256, 1>(h); return true;
     case 512: twiddle_table_t<512, 1>(h); return true;
     case 1024: twiddle_table_t<1024, 1>(h); return true;
+    case 2048: twiddle_table_t<2048, 1>(h); return true;
+    case 4096: twiddle_table_t<4096, 1>(h); return true;
     default: return false;
   }
 }
@@ -755,6 +757,7 @@ Run1Args run1_args(tfsm_plan* p, float2* U, char* ws) {
   a.scale = (float)(1.0 / p->n[0]);
   a.scheme = p->scheme;
   a.tw = p->tw[0][0];
+  a.tw_run = p->tw[0][var1(p->n[0])];
   a.ax = p->kv[0];
   a.ax_bstride = p->kv_bstride;
   a.U = U;
@@ -763,6 +766,8 @@ Run1Args run1_args(tfsm_plan* p, float2* U, char* ws) {
   a.coef = p->coef;
   a.coef_bstride = p->coef_bstride();
   a.coefc = p->cplx ? p->coefc : nullptr;
+  a.cpk = p->cpk;
+  a.cpk_bstride = p->Bc > 1 ? 2 * p->modes : 0;
   a.cons = p->term == TERM_CONS ? 1 : 0;
   a.src = p->src;
   a.src_bstride = p->src_bstride();
@@ -1562,7 +1567,7 @@ int64_t tfsm_plan_inverse_scratch_bytes(const tfsm_plan* plan, int32_t nbatch) {
 int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int32_t row_var, int32_t row_wg,
                          int32_t sub_batch) {
   if (!plan) return fail(TFSM_E_INVALID, "null plan");
-  if (!plan->fused_ok) return fail(TFSM_E_INVALID, "no fused kernels for this plan: it has no launch shape");
+  if (!plan->fused_ok || plan->l1) return fail(TFSM_E_INVALID, "no fused kernels for this plan: it has no launch shape");
   if (plan->D == 3 && (row_var < 0 || row_var > 1 || col_var < 0 || col_var > 1))
     return fail(TFSM_E_INVALID, "unsupported 3D tuning");
   if (plan->D == 3 && (col_var == 1 || row_var == 1) &&

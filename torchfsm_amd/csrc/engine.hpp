@@ -618,7 +618,8 @@ struct Run1Args {
   int B, N, H, P, kmax;
   float coef_t, scale;
   int scheme;
-  const float2* tw;
+  const float2* tw;           // stage twiddles of the default radix plan
+  const float2* tw_run;       // those of the stepper's plan (var1)
   const float* ax;            // [Bk][N] axis wavenumbers
   size_t ax_bstride;
   float2* U;
@@ -627,6 +628,8 @@ struct Run1Args {
   const float* coef;
   size_t coef_bstride;
   const float2* coefc = nullptr;  // complex-L plans: complex coefficient tables (same strides), else null
+  const float4* cpk = nullptr;    // packed coefficients (real L)
+  size_t cpk_bstride = 0;
   const float2* src;
   size_t src_bstride;
   int nsteps;
@@ -731,6 +734,10 @@ hipError_t launch_linear_steps_c(float2* U, const float2* E, size_t coef_bstride
 hipError_t launch_record(const float2* U, float2* traj, const int* rec_slot, int step, int B, size_t per_sample,
                          int T, hipStream_t st);
 hipError_t launch_run1d(const Run1Args& a, hipStream_t st);
+// radix-plan variant of the 1D stepper (k1_run) for a mesh of n points
+constexpr int var1(int n) {
+  return n == 32 || n == 64 || n == 128 || n == 256 ? 3 : (n == 1024 || n == 2048 || n == 4096 ? 1 : 0);
+}
 // KSConvection in 1D, one launch per stage: the raw product spectrum of stage spectrum S, then the
 // stage combine (with the batch-mean correction of the DC mode) into S, U, A1, A2
 hipError_t launch_k1_eval_ks(const Run1Args& a, const float2* S, float2* Nraw, hipStream_t st);

@@ -254,150 +254,198 @@ __global__ void k_record(const float2* __restrict__ U, float2* __restrict__ traj
 }
 
 // ---------------------------------------------------------------- 1D persistent stepper
-// V samples per workgroup (interleaved in LDS); every sample's state, stage spectrum and
-// auxiliary arrays stay owned by fixed threads for the whole run: thread j owns modes k = j + m*NT.
-// Convection (C = D = 1): N = coef_t * fft(u * u_x) [+ S], u from the dealiased stage spectrum;
-// ConservativeConvection: N = coef_t * (i a) fft(u * u) [+ S].
+// One launch runs every step of a call: NT = N / RMAX threads per sample, thread j owning the modes
+// k = j + m NT (k <= N/2) with their state U, stage arrays A1, A2 and (real L) packed coefficients in
+// registers for the whole run.  Convection (C = D = 1): N = coef_t * fft(u * u_x) [+ S], u from the
+// dealiased stage spectrum; ConservativeConvection: N = coef_t * (i a) fft(u * u) [+ S].
 // CPLX: complex-L plan (complex coefficient tables, stage_combine_c).
-// The state U, the stage arrays A1, A2 and (real plans) the per-mode coefficient table stay in LDS for
-// the whole run when they fit (LSTATE, LCOEF): the stage combine then waits on LDS instead of
-// on one memory round trip per mode, which at small N is most of an evaluation.  Each lane only
-// ever touches its own modes k = j + m NT of these copies, so they need no barriers of their own.
-template <int N, int V, bool CPLX>
-__global__ void __launch_bounds__(Fft<N>::NT* V) k1_run(Run1Args a) {
-  using F = Fft<N>;
-  constexpr int RMAX = F::RMAX, NT = F::NT, H = N / 2 + 1;
-  constexpr bool LSTATE = (size_t)V * H * 3 * sizeof(float2) <= 16384;
-  constexpr bool LCOEF = !CPLX && (size_t)V * H * NCOEF * sizeof(float) <= 20480;
-  __shared__ float2 s_tw[Fft<N>::tw_size()];
-  __shared__ float2 s_buf[LdsSize<N, V>::slots];
-  __shared__ float2 s_stage[V * H];
-  __shared__ float2 s_st[LSTATE ? 3 * V * H : 1];
-  __shared__ float s_cf[LCOEF ? V * NCOEF * H : 1];
-  constexpr bool LAX = (size_t)V * H * sizeof(float) <= 8192;  // wavenumbers k = 0..N/2 in LDS too
-  __shared__ float s_ax[LAX ? V * H : 1];
-  load_twiddles<N>(s_tw, a.tw);
-  const int vi = threadIdx.x % V, j = threadIdx.x / V;
-  const int smp = blockIdx.x * V + vi;
+//
+// Bound by one wavefront's serial chain: a few samples occupy a few CUs, so an evaluation takes as long
+// as its instructions and LDS exchanges in a row.  The radix plans (var1) therefore hold 4 or 8 values
+// per thread (up to 256 points 4, in one wavefront, without barriers; 512 and more 8, over two LDS
+// buffers with one barrier per exchange).  One SETDRK4 step, in us, before (16 values per
+// thread, state and coefficients in LDS or memory) and now: N = 128, B = 1 19.3 -> 5.2; 512, B = 8 12.1 ->
+// 8.0; 2048, B = 8 28.5 -> 13.3; 4096, B = 16 33.1 -> 17.1; 100, B = 1 30.0 -> 17.7; several waves per SIMD
+// gain as much (128, B = 4096 20.8 -> 7.5; 4096, B = 1024 133 -> 70).
+template <int N>
+struct Run1Shape {
+  static constexpr int VAR = var1(N);
+  using F = Fft<N, VAR>;
+  static constexpr int NT = F::NT, RMAX = F::RMAX;
+  static constexpr int G = NT >= 64 ? 1 : 64 / NT;  // samples per workgroup
+  static constexpr bool WS = RowSync<N, VAR>::WS;   // a sample lives inside one wavefront
+  static constexpr bool PP = NT > 64;               // two exchange buffers, workgroup barriers
+  static constexpr int HM = RMAX / 2 + 1;           // modes per thread (the last one: k = N/2, j = 0 only)
+};
+
+template <int N, int DIR>
+__device__ __forceinline__ void run1_fft(float2 (&v)[Run1Shape<N>::RMAX], float2* lds, const float2* tw, int j) {
+  using S = Run1Shape<N>;
+  if constexpr (S::PP) fft_wg_pp<N, DIR, 1, S::VAR>(v, lds, lds + LdsSize<N, 1>::slots, tw, j, 0);
+  else fft_wg<N, DIR, 1, S::VAR, S::WS>(v, lds, tw, j, 0);
+}
+
+// the combine of one compile-time stage over a thread's modes; cf: packed coefficient halves
+template <int N, bool CPLX, int ST>
+__device__ __forceinline__ void run1_combine(const Run1Args& a, const float2 (&nv)[Run1Shape<N>::HM],
+                                             float2 (&U)[Run1Shape<N>::HM], float2 (&A1)[Run1Shape<N>::HM],
+                                             float2 (&A2)[Run1Shape<N>::HM],
+                                             const float4 (&c0)[CPLX ? 1 : Run1Shape<N>::HM],
+                                             const float4 (&c1)[CPLX ? 1 : Run1Shape<N>::HM], const float2* cfc,
+                                             float2 (&s)[Run1Shape<N>::HM], int j) {
+  using S = Run1Shape<N>;
+#pragma unroll
+  for (int i = 0; i < S::HM; ++i) {
+    if constexpr (CPLX) {
+      const int k = j + i * S::NT;
+      s[i] = stage_combine_c(ST, nv[i], U, A1, A2, i, cfc, a.P, k <= N / 2 ? k : 0);
+    } else {
+      float2 w;
+      s[i] = stage_combine_v(ST, nv[i], U[i], A1[i], A2[i], stage_coef_half(ST) ? c1[i] : c0[i], c1[i].z, &w);
+      if constexpr (ST != ST_PRO) {
+        if (stage_target(ST) == 0) U[i] = w;
+        else if (stage_target(ST) == 1) A1[i] = w;
+        else A2[i] = w;
+      }
+    }
+  }
+}
+
+template <int N, bool CPLX>
+__global__ void __launch_bounds__((Run1Shape<N>::NT * Run1Shape<N>::G)) k1_run(Run1Args a) {
+  using S = Run1Shape<N>;
+  using F = typename S::F;
+  constexpr int RMAX = S::RMAX, NT = S::NT, HM = S::HM, SL = LdsSize<N, 1>::slots;
+  __shared__ float2 s_tw[F::tw_size()];
+  __shared__ float2 s_buf[S::G * (S::PP ? 2 : 1) * SL];
+  __shared__ float2 s_mir[S::G * N];  // mirror positions N - k of the packed spectrum
+  for (int i = threadIdx.x; i < F::tw_size(); i += NT * S::G) s_tw[i] = a.tw_run[i];
+  const int g = threadIdx.x / NT, j = threadIdx.x % NT;
+  const int smp = blockIdx.x * S::G + g;
   const bool valid = smp < a.B;
-  int nmax = 0;
-  for (int w = 0; w < V; ++w) {
-    const int sw = blockIdx.x * V + w;
+  const int sb = valid ? smp : 0;
+  int nmax = 0;  // steps of the workgroup: every thread takes part in every transform
+  for (int w = 0; w < S::G; ++w) {
+    const int sw = blockIdx.x * S::G + w;
     if (sw < a.B) {
       const int ns = a.nsteps_per ? a.nsteps_per[sw] : a.nsteps;
       nmax = ns > nmax ? ns : nmax;
     }
   }
   const int nst = valid ? (a.nsteps_per ? a.nsteps_per[smp] : a.nsteps) : 0;
-  const size_t so = (size_t)(valid ? smp : 0) * a.P;
-  float2* U = a.U + so;
-  float2* A1 = a.A1 + so;
-  float2* A2 = a.A2 + so;
-  const float* cf = a.coef + (size_t)(valid ? smp : 0) * a.coef_bstride;
-  const float2* cfc = CPLX ? a.coefc + (size_t)(valid ? smp : 0) * a.coef_bstride : nullptr;
-  const float* ax = a.ax + (size_t)(valid ? smp : 0) * a.ax_bstride;
-  const float2* src = a.src ? a.src + (size_t)(valid ? smp : 0) * a.src_bstride : nullptr;
-  float2* stg = s_stage + vi * H;
-  for (int k = j; k < H; k += NT) stg[k] = valid ? U[k] : make_float2(0.f, 0.f);
-  // working copies of U, A1, A2 (written back at the end: U after stepping, A1 after an
-  // evaluation-only call)
-  float2* Uw = U;
-  float2* A1w = A1;
-  float2* A2w = A2;
-  if constexpr (LSTATE) {
-    Uw = s_st + vi * H;
-    A1w = s_st + (V + vi) * H;
-    A2w = s_st + (2 * V + vi) * H;
-    for (int k = j; k < H; k += NT) Uw[k] = valid ? U[k] : make_float2(0.f, 0.f);
-  }
-  const float* axw = ax;
-  if constexpr (LAX) {
-    float* t = s_ax + (size_t)vi * H;
-    for (int k = j; k < H; k += NT) t[k] = ax[k];
-    axw = t;
-  }
-  const float* cfw = cf;
-  size_t cstride = a.P;
-  if constexpr (LCOEF) {
-    float* t = s_cf + (size_t)vi * NCOEF * H;
-    for (int sl = 0; sl < NCOEF; ++sl)
-      for (int k = j; k < H; k += NT) t[sl * H + k] = cf[(size_t)sl * a.P + k];
-    cfw = t;
-    cstride = H;
+  float2* lds = s_buf + g * (S::PP ? 2 : 1) * SL;
+  float2* mir = s_mir + g * N;
+  float2* Ug = a.U + (size_t)sb * a.P;
+  const float* ax = a.ax + (size_t)sb * a.ax_bstride;
+  const float2* cfc = CPLX ? a.coefc + (size_t)sb * a.coef_bstride : nullptr;
+  const float4* cpk = a.cpk + (size_t)sb * a.cpk_bstride;
+  const float2* src = a.src ? a.src + (size_t)sb * a.src_bstride : nullptr;
+  float2 U[HM], A1[HM], A2[HM], s[HM], sv[HM];
+  float4 c0[CPLX ? 1 : HM], c1[CPLX ? 1 : HM];
+  float axk[HM];
+#pragma unroll
+  for (int i = 0; i < HM; ++i) {
+    const int k = j + i * NT, kc = k <= N / 2 ? k : 0;  // the last slot belongs to k = N/2 (j = 0)
+    U[i] = Ug[kc];
+    if (!valid) U[i] = make_float2(0.f, 0.f);
+    A1[i] = A2[i] = make_float2(0.f, 0.f);
+    s[i] = U[i];
+    sv[i] = src ? src[kc] : make_float2(0.f, 0.f);
+    axk[i] = ax[kc];
+    if constexpr (!CPLX) {
+      c0[i] = cpk[cpk_index(kc, 0)];
+      c1[i] = cpk[cpk_index(kc, 1)];
+    }
   }
   __syncthreads();
   const int nev = a.eval_only ? 1 : scheme_evals(a.scheme);
   const int nloop = a.eval_only ? 1 : nmax;
+  const bool rec = a.rec_slot && valid && !a.eval_only;
+  auto record = [&](int sl) {
+    if (sl < 0 || sl >= a.T) return;
+    float2* t = a.traj + ((size_t)smp * a.T + sl) * a.P;
+#pragma unroll
+    for (int i = 0; i < HM; ++i)
+      if (j + i * NT <= N / 2) t[j + i * NT] = U[i];
+  };
+  int slot = rec ? a.rec_slot[0] : -1;
   for (int step = 0; step < nloop; ++step) {
     const bool active = valid && step < nst;
-    if (a.rec_slot && active) {
-      const int sl = a.rec_slot[step];
-      if (sl >= 0 && sl < a.T)
-        for (int k = j; k < H; k += NT) a.traj[((size_t)smp * a.T + sl) * a.P + k] = Uw[k];
+    if (rec && active) {
+      record(slot);
+      slot = a.rec_slot[step + 1];  // read a step ahead
     }
     for (int e = 0; e < nev; ++e) {
       const int stage = a.eval_only ? ST_EVAL : scheme_stage(a.scheme, e);
       float2 v[RMAX];
+      // Z = A + i B of the Hermitian spectra A = u^ and B = i a u^ (B = 0 for ConservativeConvection:
+      // u_x in the imaginary part would add its round-off to u): own positions k, and the mirrored
+      // conj(A) + i conj(B) through LDS to the owner of position N - k
 #pragma unroll
-      for (int m = 0; m < RMAX; ++m) {
-        const int pos = j + m * NT;
-        const bool cj = pos > N / 2;
-        const int k = cj ? N - pos : pos;
-        const bool edge = (k == 0) || (k == N / 2);
-        float2 val = make_float2(0.f, 0.f);
-        float axk = 0.f;
+      for (int i = 0; i < HM; ++i) {
+        const int k = j + i * NT;
+        float2 A = make_float2(0.f, 0.f);
+        float ak = 0.f;
         if (k <= a.kmax) {
-          val = stg[k];
-          val = make_float2(val.x * a.scale, val.y * a.scale);
-          axk = a.cons ? 0.f : axw[k];  // u alone: u_x in the imaginary part would add its round-off to u
+          A = make_float2(s[i].x * a.scale, s[i].y * a.scale);
+          ak = a.cons ? 0.f : axk[i];
         }
-        float2 A = val;
-        float2 Bv = make_float2(-axk * val.y, axk * val.x);  // i a_k u^
-        if (edge) {
+        float2 Bv = make_float2(-ak * A.y, ak * A.x);
+        if (k == 0 || k == N / 2) {
           A.y = 0.f;
           Bv.y = 0.f;
         }
-        v[m] = cj ? make_float2(A.x + Bv.y, Bv.x - A.y) : make_float2(A.x - Bv.y, A.y + Bv.x);
+        if (i < RMAX / 2) {
+          v[i] = make_float2(A.x - Bv.y, A.y + Bv.x);
+          if (k > 0) mir[N - k] = make_float2(A.x + Bv.y, Bv.x - A.y);
+        } else if (j == 0) {
+          mir[N / 2] = make_float2(A.x - Bv.y, A.y + Bv.x);
+        }
       }
-      fft_wg<N, +1, V>(v, s_buf, s_tw, j, vi);
+      lds_sync<S::WS>();
+#pragma unroll
+      for (int m = RMAX / 2; m < RMAX; ++m) v[m] = mir[j + m * NT];
+      run1_fft<N, +1>(v, lds, s_tw, j);
       // Convection u u_x, or ConservativeConvection's u u (its derivative follows the transform)
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) v[m] = make_float2(a.cons ? v[m].x * v[m].x : v[m].x * v[m].y, 0.f);
-      fft_wg<N, -1, V>(v, s_buf, s_tw, j, vi);
-      if (a.cons) {
+      run1_fft<N, -1>(v, lds, s_tw, j);
+      if (!(active || (a.eval_only && valid))) continue;  // no barrier below
+      float2 nv[HM];
 #pragma unroll
-        for (int m = 0; m < RMAX; ++m) {
-          const int pos = j + m * NT;
-          const float ap = pos <= N / 2 ? axw[pos] : 0.f;
-          v[m] = make_float2(-mulr(ap, v[m].y), mulr(ap, v[m].x));  // (i a) fft(u u)
-        }
+      for (int i = 0; i < HM; ++i) {
+        float2 f = v[i];
+        if (a.cons) f = make_float2(-mulr(axk[i], f.y), mulr(axk[i], f.x));  // (i a) fft(u u)
+        nv[i] = rscale(a.coef_t, f);
+        if (src) nv[i] = radd(nv[i], sv[i]);
       }
-#pragma unroll
-      for (int m = 0; m < RMAX; ++m) {
-        const int pos = j + m * NT;
-        if (pos <= N / 2) {
-          float2 sn = make_float2(0.f, 0.f);
-          if (active || (a.eval_only && valid)) {
-            float2 nv = nl_value(a.coef_t, v[m], src, pos);
-            if constexpr (CPLX) sn = stage_combine_c(stage, nv, Uw, A1w, A2w, pos, cfc, a.P, pos);
-            else sn = stage_combine(stage, nv, Uw, A1w, A2w, pos, cfw, cstride, pos, true);
-          }
-          stg[pos] = sn;
-        }
+      switch (stage) {
+#define TFSM_RUN1_STAGE(X) \
+  case X: run1_combine<N, CPLX, X>(a, nv, U, A1, A2, c0, c1, cfc, s, j); break;
+        TFSM_RUN1_STAGE(ST_R1_E0)
+        TFSM_RUN1_STAGE(ST_R2_E0)
+        TFSM_RUN1_STAGE(ST_R2_E1)
+        TFSM_RUN1_STAGE(ST_R3_E0)
+        TFSM_RUN1_STAGE(ST_R3_E1)
+        TFSM_RUN1_STAGE(ST_R3_E2)
+        TFSM_RUN1_STAGE(ST_R4_E0)
+        TFSM_RUN1_STAGE(ST_R4_E1)
+        TFSM_RUN1_STAGE(ST_R4_E2)
+        TFSM_RUN1_STAGE(ST_R4_E3)
+        TFSM_RUN1_STAGE(ST_EVAL)
+#undef TFSM_RUN1_STAGE
+        default: break;
       }
-      __syncthreads();
     }
   }
-  if (a.rec_slot && valid && !a.eval_only) {
-    const int sl = a.rec_slot[nst];
-    if (sl >= 0 && sl < a.T)
-      for (int k = j; k < H; k += NT) a.traj[((size_t)smp * a.T + sl) * a.P + k] = Uw[k];
-  }
-  if (LSTATE && valid) {
-    if (a.eval_only)
-      for (int k = j; k < H; k += NT) A1[k] = A1w[k];
-    else
-      for (int k = j; k < H; k += NT) U[k] = Uw[k];
+  if (rec) record(slot);
+  if (!valid) return;
+  float2* out = a.eval_only ? a.A1 + (size_t)smp * a.P : Ug;
+#pragma unroll
+  for (int i = 0; i < HM; ++i) {
+    // by component: a choice between the two arrays themselves would put both in scratch memory
+    const float2 n = A1[i], u = U[i];
+    if (j + i * NT <= N / 2) out[j + i * NT] = make_float2(a.eval_only ? n.x : u.x, a.eval_only ? n.y : u.y);
   }
 }
 
@@ -603,12 +651,12 @@ hipError_t launch_record(const float2* U, float2* traj, const int* rec_slot, int
 
 template <int N>
 static hipError_t launch_run1_t(const Run1Args& a, hipStream_t st) {
-  constexpr int NT = Fft<N>::NT;
-  constexpr int V = NT >= 64 ? 1 : 64 / NT;
+  using S = Run1Shape<N>;
+  const dim3 grid((a.B + S::G - 1) / S::G), block(S::NT * S::G);
   if (a.coefc)
-    hipLaunchKernelGGL((k1_run<N, V, true>), dim3((a.B + V - 1) / V), dim3(NT * V), 0, st, a);
+    hipLaunchKernelGGL((k1_run<N, true>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((k1_run<N, V, false>), dim3((a.B + V - 1) / V), dim3(NT * V), 0, st, a);
+    hipLaunchKernelGGL((k1_run<N, false>), grid, block, 0, st, a);
   return hipGetLastError();
 }
 
