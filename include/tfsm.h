@@ -122,7 +122,7 @@ int64_t tfsm_plan_inverse_scratch_bytes(const tfsm_plan* plan, int32_t nbatch);
 
 /* Launch shape of the fused 2D kernels (chosen per shape class by the autotuner): column tile
  * width (8 or 16 columns), radix-plan variant of the column and row transforms (0 or 1: variant 1
- * carries a transform with half as many threads), row-kernel workgroup size (64 or 256 threads),
+ * holds 4 values per thread at 64, 128 and 256 points, 16 at 512 and 8 at 1024), row-kernel workgroup size (64 or 256 threads),
  * and the sub-batch of samples stepped together (through all steps of a tfsm_step call on one
  * stream, in rounds of 16 steps on several; 0 = the whole batch; smaller sub-batches keep their
  * working set in the last-level cache).
@@ -132,8 +132,8 @@ int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int
 
 /* Current launch shape: out[6] = column tile, column variant, row variant, row workgroup,
  * sub-batch, streams.  A new plan starts from a default derived from its shape (2D: column tile
- * and radix variant per axis size and product term, 64-thread row groups for 64- and 128-point
- * rows, sub-batch sized to keep >= 512 column workgroups per launch, and sub-batches on two
+ * and radix variant per axis size and product term, 64-thread row groups where there are few
+ * rows of 64 to 256 points, sub-batch sized to keep >= 512 column workgroups per launch, and sub-batches on two
  * streams for 512^2 VorticityConvection (16 samples, B >= 32), Convection and
  * NSPressureConvection (16 samples from B = 32, 8 at B = 16..31) and 256^2 VorticityConvection
  * and Convection (16 samples, B >= 32; four streams from B = 64); 3D: radix-4

@@ -246,8 +246,6 @@ bool twiddle_table(int n, int var, std::vector<float2>& h) {
     }
   }
   switch (n) {
-    case 64: twiddle_table_t<64, 1>(h); return true;
-    case 128: twiddle_table_t<128, 1>(h); return true;
     case 256: twiddle_table_t<256, 1>(h); return true;
     case 512: twiddle_table_t<512, 1>(h); return true;
     case 1024: twiddle_table_t<1024, 1>(h); return true;
@@ -528,7 +526,7 @@ Row2Args row_args(tfsm_plan* p, char* ws, int b0, int nb) {
   r.PF = p->PF;
   r.kmax1 = p->kmax[1];
   r.NF = p->NF;
-  r.tw1 = p->tw[1][p->row_var];
+  r.tw1 = p->tw[1][plan2(p->n[1], p->row_var)];
   r.ay = p->kv[1];
   r.G = (const float2*)(ws + p->off_G);
   r.P = (float2*)(ws + p->off_P);
@@ -550,7 +548,7 @@ Col2Args col_args(tfsm_plan* p, float2* U, char* ws) {
   c.NF = p->NF;
   c.coef_t = p->coef_t;
   c.scale = (float)(1.0 / ((double)p->n[0] * p->n[1]));
-  c.tw0 = p->tw[0][p->col_var];
+  c.tw0 = p->tw[0][plan2(p->n[0], p->col_var)];
   c.ax = p->kv[0];
   c.ay = p->kv[1];
   c.P = (const float2*)(ws + p->off_P);
@@ -842,9 +840,9 @@ int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* tra
     // one workgroup per sample runs every step (small meshes: launch-bound otherwise)
     Col2Args ca = col_args(p, U, (char*)ws);
     Row2Args ra = row_args(p, (char*)ws, 0, p->B);
-    // k2_run runs the default radix plan (variant 0) on both axes, whatever the tiled kernels' tuning
-    ca.tw0 = p->tw[0][0];
-    ra.tw1 = p->tw[1][0];
+    // k2_run has a radix plan of its own, whatever the tiled kernels' tuning
+    ca.tw0 = p->tw[0][run2d_var(p->term, p->n[0])];
+    ra.tw1 = p->tw[1][run2d_var(p->term, p->n[0])];
     Run2Args r;
     r.b0 = 0;
     r.nb = p->B;
@@ -1460,18 +1458,26 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
   if (!rc && D == 2 && p->fused_ok) {
     const bool one_channel = term == TERM_VC || term == TERM_KS;
     const int n0 = p->n[0], n1 = p->n[1];
-    // measured per axis size (SETDRK4, B = 16..32): 512 keeps 16-column tiles; 256 runs 8-column
-    // tiles with the 8-values-per-thread plan (26 % faster than 16 columns of 16 values); 64 and
-    // 128 run 8-column tiles and one row per 64-thread row group (5-9 %)
-    p->col_var = n0 == 256 ? 1 : 0;
-    if (n0 == 64 || n0 == 128 || n0 == 256) p->V = 8;
+    // measured per axis size: 512 keeps 16-column tiles; 64, 128 and 256 run 8-column tiles and rows of 4
+    // values per thread.  Their launches are one round of workgroups, as long as one thread's chain of
+    // transforms, and shorter chains win at every batch (SETDRK4, us per step, against the plans of 8 and
+    // 16 values per thread that these replace: Burgers 128^2 B = 1 141 -> 62, B = 16 133 -> 70, B = 64 195
+    // -> 111; vorticity 64^2 B = 4 54 -> 42, 128^2 B = 16 97 -> 58, 256^2 B = 8 95 -> 80, B = 32 136 -> 122)
+    if (n0 == 64 || n0 == 128 || n0 == 256) {
+      p->V = 8;
+      p->col_var = 1;
+    }
     // 1024-point columns: 8 columns per tile (LDS), the 8-values-per-thread plan (the 16-value
     // plan holds 2 waves per SIMD and spills for NSPressureConvection and ConservativeConvection)
     if (n0 == 1024) {
       p->V = 8;
       p->col_var = 1;
     }
-    if (n1 == 64 || n1 == 128) p->row_wg = 64;
+    if (n1 == 64 || n1 == 128 || n1 == 256) {
+      p->row_var = 1;
+      // few rows: one-wavefront workgroups spread over more CUs (128^2 B = 1 63.9 -> 61.5; B = 16 the reverse)
+      if ((size_t)p->B * n0 <= 512) p->row_wg = 64;
+    }
     const size_t per_sample = 4 * (size_t)p->C * p->modes * sizeof(float2) +
                               (size_t)p->NF * p->n[0] * p->PF * sizeof(float2);
     const int tiles = (p->H + p->V - 1) / p->V;

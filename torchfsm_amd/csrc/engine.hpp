@@ -707,6 +707,9 @@ struct ConvArgs {
 };
 
 // ---------------------------------------------------------------- host launchers (defined in *.hip)
+// radix plan of the 2D kernels' variant `var` at n points: variant 1 is 4 values per thread at 64, 128
+// and 256 points (it beats 8 and 16 values there at every batch measured), 16 at 512, 8 at 1024
+constexpr int plan2(int n, int var) { return var == 1 && (n == 64 || n == 128 || n == 256) ? 3 : var; }
 hipError_t launch_col2d(int term, const Col2Args& a, int nb, int stage, int v, int var, hipStream_t st);
 hipError_t launch_row2d(int term, const Row2Args& a, int var, int wgt, hipStream_t st);
 bool col2d_supported(int n0, int v, int var);
@@ -714,6 +717,8 @@ bool col2d_supported(int n0, int v, int var);
 // VorticityConvection, field pitch pf at most that of the 2/3 rule
 hipError_t launch_run2d(int term, const Col2Args& ca, const Row2Args& ra, const Run2Args& r, hipStream_t st);
 bool run2d_supported(int term, int n0, int n1, int pf);
+// its radix-plan variant (both axes)
+constexpr int run2d_var(int term, int n) { return term == TERM_VC && n == 64 ? 0 : 3; }
 bool row2d_supported(int n1, int var, int wgt);
 hipError_t launch_rows_r2c(int n, const float* in, size_t in_ld, float2* out, size_t out_ld, int nrows, float scale,
                            const float2* tw, hipStream_t st);

@@ -210,8 +210,6 @@ template <> struct FftPlan<768, 0> { static constexpr int RMAX = 12; static cons
 template <> struct FftPlan<800, 0> { static constexpr int RMAX = 20; static constexpr int NST = 5; static constexpr int R[5] = {4, 4, 2, 5, 5}; };
 // VAR 1: twice the elements per thread (half the threads per transform), same radix sequence
 // where possible; lets a column tile of the same width run with half the workgroup size.
-template <> struct FftPlan<64, 1> { static constexpr int RMAX = 16; static constexpr int NST = 2; static constexpr int R[5] = {8, 8, 0, 0, 0}; };
-template <> struct FftPlan<128, 1> { static constexpr int RMAX = 16; static constexpr int NST = 3; static constexpr int R[5] = {8, 4, 4, 0, 0}; };
 template <> struct FftPlan<256, 1> { static constexpr int RMAX = 8; static constexpr int NST = 3; static constexpr int R[5] = {8, 8, 4, 0, 0}; };
 template <> struct FftPlan<512, 1> { static constexpr int RMAX = 16; static constexpr int NST = 3; static constexpr int R[5] = {8, 8, 8, 0, 0}; };
 // (1024: half the elements per thread of VAR 0, for 2D columns of 1024 points)

@@ -191,8 +191,8 @@ __device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, fl
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride : nullptr;
-    combine_column2<N0, VAR, 1>(a, stage, ((size_t)b * 2 + c) * plane, src, cpk, c5b, tb, cko, ky, colv, j, v[c],
-                                s[c], rs);
+    combine_column2<N0, VAR, (RMAX > 4 ? 1 : 4)>(a, stage, ((size_t)b * 2 + c) * plane, src, cpk, c5b, tb, cko, ky,
+                                                 colv, j, v[c], s[c], rs);
   }
 }
 
@@ -318,7 +318,7 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
         if (a.dc && ky == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
       }
       const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride : nullptr;
-      combine_column2<N0, VAR, (NC > 1 || RMAX >= 16) ? 1 : 4, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
+      combine_column2<N0, VAR, (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : 4, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
                                                                                   cko, kl, colv, j, v, s[c], rs,
                                                                                   &pre);
     }
@@ -694,10 +694,13 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_row(Row2Args a) 
 // 90-130 us for the tiled kernels, and 128^2 keeps them.)
 template <int N, int TERM>
 struct Run2Shape {
-  using F = Fft<N, 0>;
+  // 4 values per thread (SETDRK4 step, us: 32^2 vorticity 34 -> 27, Convection 51 -> 34, 64^2 Convection 64
+  // -> 60), 8 for the 64-point VorticityConvection (44 against 46)
+  static constexpr int VAR = run2d_var(TERM, N);
+  using F = Fft<N, VAR>;
   static constexpr int NT = F::NT;               // threads per transform (rows and columns)
   static constexpr int V = N;                    // one column tile holds all N/2 + 1 columns
-  static constexpr int THREADS = NT * V;         // 128 (N = 32), 512 (N = 64)
+  static constexpr int THREADS = NT * V;         // 256 (N = 32), 512 or 1024 (N = 64)
   static constexpr int ROWS = THREADS / NT;      // = N: every row in one pass
   static constexpr int PDR = F::PD < 16 ? F::PD : 16;
   static constexpr int SLR = N + N / PDR + 1;    // LDS slots of one row (padding of lds_slot<1, PD>)
@@ -718,7 +721,7 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
                                                       "Convection and VorticityConvection only");
   using S = Run2Shape<N, TERM>;
   constexpr int NT = S::NT, V = S::V;
-  __shared__ float2 s_tw[Fft<N, 0>::tw_size()];
+  __shared__ float2 s_tw[S::F::tw_size()];
   __shared__ float2 s_buf[S::SLOTS];
   __shared__ float2 s_G[S::G_SLOTS];
   __shared__ float2 s_P[S::P_SLOTS];
@@ -747,7 +750,7 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
   w.P = s_P;
   w.b0 = 0;
   // rows and columns share the plan: a square mesh with the same radix variant on both axes
-  load_twiddles<N, 0>(s_tw, ca.tw0);
+  load_twiddles<N, S::VAR>(s_tw, ca.tw0);
   for (int i = threadIdx.x; i < N; i += S::THREADS) s_ax[i] = ca.ax[i];
   __syncthreads();
   const int nev = scheme_evals(r.scheme);
@@ -771,10 +774,10 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
     if (k > 0) {
       __syncthreads();  // fields G of the previous column pass (and the state) complete
       if (e == 0 && r.rec_slot) record((k - 1) / nev);
-      row2_body<N, TERM, 0>(w, 0, g, true, s_buf + g * S::SLR, s_tw, jr);
+      row2_body<N, TERM, S::VAR>(w, 0, g, true, s_buf + g * S::SLR, s_tw, jr);
     }
     __syncthreads();  // products P complete; the LDS exchange buffer is reused
-    col2_tile<N, V, TERM, 0, -1, true>(c, k > 0 ? scheme_stage(r.scheme, e) : ST_PRO, 0, 0, s_buf, s_tw, s_ax, jc,
+    col2_tile<N, V, TERM, S::VAR, -1, true>(c, k > 0 ? scheme_stage(r.scheme, e) : ST_PRO, 0, 0, s_buf, s_tw, s_ax, jc,
                                        vi);
   }
   if (r.rec_slot) {
@@ -785,16 +788,17 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
 
 // ---------------------------------------------------------------- host launchers
 // Tuning knobs (chosen per shape class by the autotuner): column tile V in {8, 16}, radix-plan
-// variant of the column and row transforms (0: N/RMAX threads per transform; 1: half as many),
-// and the row-kernel workgroup size (64 or 256 threads).
-// Shapes whose column kernels are also compiled per SETDRK4 stage (and for the field pass of the
-// initial state): the 512-point VorticityConvection columns of the Navier-Stokes workloads with 8
-// values per thread.  One stage's kernel holds a quarter of the combine code of the run-time-stage
-// kernel (13-16 KB of code instead of 21 KB) and 87-128 VGPRs; with 16 values per thread the
-// stage kernels need 133-164 VGPRs (occupancy 3) and the run-time-stage kernel is kept.
+// variant of the column and row transforms (0: the default plan; 1: another number of values per
+// thread, plan2), and the row-kernel workgroup size (64 or 256 threads).
+// Shapes whose column kernels are also compiled per stage (and for the field pass of the initial
+// state): the 512-point VorticityConvection columns of the Navier-Stokes workloads with 8 values per
+// thread (13-16 KB of code instead of 21 KB, 87-128 VGPRs; with 16 values per thread the stage kernels
+// need 133-164 VGPRs, occupancy 3, and the run-time-stage kernel is kept), and the plans of 4 values
+// per thread, whose short launches spend much of their time in the run-time switch.
 template <int N0, int V, int TERM, int VAR>
 struct ColStageKernels {
-  static constexpr bool value = TERM == TERM_VC && N0 == 512 && VAR == 0;
+  static constexpr bool terms = TERM == TERM_VC || TERM == TERM_CONV || TERM == TERM_NSP;
+  static constexpr bool value = (TERM == TERM_VC && N0 == 512 && VAR == 0) || (terms && VAR == 3);
 };
 
 template <int N0, int V, int TERM, int VAR>
@@ -803,20 +807,29 @@ inline hipError_t launch_col_t(const Col2Args& a, int nb, int stage, hipStream_t
   Col2Args b = a;
   b.nb = nb;
   const dim3 grid(tiles * nb), block(Fft<N0, VAR>::NT * V);
-  // the stage kernels read SETDRK4's compact coefficient tables unconditionally
+#define TFSM_COL_STAGE(S) \
+  case S: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, S>), grid, block, 0, st, b, stage); return hipGetLastError();
   if constexpr (ColStageKernels<N0, V, TERM, VAR>::value) {
-    const bool tables = a.ck01 && a.c6t;
-    switch (tables ? stage : -1) {
-      case ST_PRO: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, ST_PRO>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E0: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, ST_R4_E0>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E1: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, ST_R4_E1>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E2: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, ST_R4_E2>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E3: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, ST_R4_E3>), grid, block, 0, st, b, stage); break;
-      default: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR>), grid, block, 0, st, b, stage);
+    if constexpr (VAR == 3) {
+      switch (stage) {
+        TFSM_COL_STAGE(ST_R2_E0)
+        TFSM_COL_STAGE(ST_R2_E1)
+        TFSM_COL_STAGE(ST_EVAL)
+        default: break;
+      }
     }
-  } else {
-    TFSM_LAUNCH((k2_col<N0, V, TERM, VAR>), grid, block, 0, st, b, stage);
+    // (SETDRK4's stage kernels read its compact coefficient tables unconditionally)
+    switch (a.ck01 && a.c6t ? stage : (stage == ST_PRO ? stage : -1)) {
+      TFSM_COL_STAGE(ST_PRO)
+      TFSM_COL_STAGE(ST_R4_E0)
+      TFSM_COL_STAGE(ST_R4_E1)
+      TFSM_COL_STAGE(ST_R4_E2)
+      TFSM_COL_STAGE(ST_R4_E3)
+      default: break;
+    }
   }
+#undef TFSM_COL_STAGE
+  TFSM_LAUNCH((k2_col<N0, V, TERM, VAR>), grid, block, 0, st, b, stage);
   return hipGetLastError();
 }
 
@@ -833,22 +846,22 @@ inline hipError_t launch_row_t(const Row2Args& a, hipStream_t st) {
 // size lists of the column (N0, tile V, radix variant) and row (N1, variant, workgroup size)
 // instantiations, split over the k_step2d_*.hip units to keep each compile short
 #define TFSM_COL_P2(X)                                                                                        \
-  X(16, 8, 0) X(16, 16, 0) X(32, 8, 0) X(32, 16, 0) X(64, 8, 0) X(64, 16, 0) X(64, 8, 1) X(64, 16, 1)          \
-  X(128, 8, 0) X(128, 16, 0) X(128, 8, 1) X(128, 16, 1) X(256, 8, 0) X(256, 16, 0) X(256, 8, 1) X(256, 16, 1) \
+  X(16, 8, 0) X(16, 16, 0) X(32, 8, 0) X(32, 16, 0) X(64, 8, 0) X(64, 16, 0) X(64, 8, 3) X(64, 16, 3)          \
+  X(128, 8, 0) X(128, 16, 0) X(128, 8, 3) X(128, 16, 3) X(256, 8, 0) X(256, 16, 0) X(256, 8, 3) X(256, 16, 3) \
   X(512, 8, 0) X(512, 16, 0) X(512, 8, 1) X(512, 16, 1) X(1024, 8, 0) X(1024, 8, 1)
 #define TFSM_COL_MX(X)                                                                                       \
   X(48, 8, 0) X(48, 16, 0) X(96, 8, 0) X(96, 16, 0) X(100, 8, 0) X(100, 16, 0) X(112, 8, 0) X(112, 16, 0)    \
   X(192, 8, 0) X(192, 16, 0) X(200, 8, 0) X(200, 16, 0)
 #define TFSM_ROW_P2(X)                                                                                        \
-  X(16, 0, 256) X(32, 0, 256) X(64, 0, 256) X(64, 1, 256) X(64, 0, 64) X(64, 1, 64) X(128, 0, 256)            \
-  X(128, 1, 256) X(128, 0, 64) X(128, 1, 64) X(256, 0, 256) X(256, 1, 256) X(256, 0, 64) X(256, 1, 64)        \
+  X(16, 0, 256) X(32, 0, 256) X(64, 0, 256) X(64, 3, 256) X(64, 0, 64) X(64, 3, 64) X(128, 0, 256)            \
+  X(128, 3, 256) X(128, 0, 64) X(128, 3, 64) X(256, 0, 256) X(256, 3, 256) X(256, 0, 64) X(256, 3, 64)        \
   X(512, 0, 256) X(512, 1, 256) X(512, 0, 64) X(512, 1, 64) X(1024, 0, 256) X(1024, 0, 64)
 #define TFSM_ROW_MX(X) X(48, 0, 256) X(96, 0, 256) X(100, 0, 256) X(112, 0, 256) X(192, 0, 256) X(200, 0, 256)
 
 #define TFSM_COL_CASE(N, VV, VR) \
-  if (a.N0 == N && v == VV && var == VR) return launch_col_t<N, VV, TERM, VR>(a, nb, stage, st);
+  if (a.N0 == N && v == VV && plan2(N, var) == VR) return launch_col_t<N, VV, TERM, VR>(a, nb, stage, st);
 #define TFSM_ROW_CASE(N, VR, W) \
-  if (a.N1 == N && var == VR && wgt == W) return launch_row_t<N, TERM, VR, W>(a, st);
+  if (a.N1 == N && plan2(N, var) == VR && wgt == W) return launch_row_t<N, TERM, VR, W>(a, st);
 
 template <int N, int TERM>
 inline hipError_t launch_run_t(const Col2Args& ca, const Row2Args& ra, const Run2Args& r, hipStream_t st) {
