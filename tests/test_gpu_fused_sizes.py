@@ -180,3 +180,80 @@ def test_1d_stepper_lengths_and_batches(dev, n, batch):
     plan.step(uh, 5)
     terms = [(-1e-4, "deriv", (0, 3)), (0.02, "lap", None), (-1, "conv", None)]
     assert _rel(plan.inverse(uh), refpath.integrate(terms, mi, u, dt, 5, scheme="SETDRK4")) <= TOL
+
+
+@pytest.mark.parametrize("kind", ["vc", "conv", "nsp", "ks", "ks_keep_mean"])
+@pytest.mark.parametrize("n0,n1,batch", [(30, 42, 3), (225, 301, 2), (67, 64, 5), (64, 67, 2), (17, 512, 2), (16, 18, 1), (128, 6, 2),
+                                         (9, 8, 4), (384, 50, 1), (143, 169, 1), (1024, 131, 1), (600, 601, 1), (5, 1031, 1)])
+def test_2d_run_time_lengths(dev, kind, n0, n1, batch):
+    """2D meshes where an axis has no fixed-size kernel (composite, prime and mixed with fixed-size axes):
+    every SETDRK4 stage with a source, per-sample step counts and a single evaluation, against the oracle."""
+    from oracle import refpath
+    from torchfsm_amd.engine import SpectralPlan
+    from torchfsm_amd.workloads import fourier_modes_field
+
+    c = 2 if kind in ("conv", "nsp") else 1
+    ks = kind.startswith("ks")
+    length = 20.0 if ks else 1.0
+    mi = [(0, length, n0), (0, length, n1)]
+    u = 0.5 * fourier_modes_field((n0, n1), 2, c, batch, seed=n0 + n1, kabs=2).to(dev)
+    g = torch.Generator(device=dev).manual_seed(n0)
+    u = u + 0.02 * torch.randn(u.shape, generator=g, device=dev)
+    src = torch.randn(1, 1, n0, n1, generator=g, device=dev)
+    dt = 0.01 if ks else 0.2 / max(n0, n1)
+    lin = [("lap", -1.0), ("biharm", -1.0)] if ks else [("lap", 0.01)]
+    coef = 1.0 if kind == "nsp" else -1.0
+    plan = SpectralPlan(mi, batch, c, nonlinear=kind, nonlinear_coef=coef, linear=lin, device=dev)
+    assert plan.general
+    plan.add_source(src, 0.3)
+    terms = [(v, k, None) for k, v in lin] + [(coef, kind, None), (0.3, "src", src)]
+    for scheme in ("SETDRK4", "SETDRK3"):
+        plan.set_scheme(scheme, dt)
+        uh = plan.forward(u)
+        plan.step(uh, 4)
+        ref = refpath.integrate(terms, mi, u, dt, 4, scheme=scheme)
+        assert _rel(plan.inverse(uh), ref) <= TOL
+    if not plan._plan or kind == "ks":
+        return
+    counts = torch.tensor([b % 3 for b in range(batch)], dtype=torch.int32, device=dev)
+    plan.set_scheme("SETDRK2", dt)
+    uh = plan.forward(u)
+    plan.step_varying(uh, counts, 2)
+    out = plan.inverse(uh)
+    for b in range(batch):
+        k = int(counts[b])
+        ref = u[b:b + 1] if k == 0 else refpath.integrate(terms, mi, u[b:b + 1], dt, k, scheme="SETDRK2")
+        assert _rel(out[b:b + 1], ref) <= TOL
+
+
+@pytest.mark.parametrize("n,batch", [(2, 1), (3, 2), (7, 3), (30, 2), (97, 1), (143, 5), (360, 2), (767, 1), (1000, 3), (1021, 2), (2039, 1),
+                                     (2187, 1), (4000, 2)])
+def test_1d_run_time_lengths(dev, n, batch):
+    """The persistent 1D stepper at run-time lengths: Convection and ConservativeConvection with a source,
+    per-sample coefficients, a recorded trajectory and a single evaluation, against the oracle."""
+    from oracle import refpath
+    from torchfsm_amd.engine import SpectralPlan
+
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.arange(n, device=dev) / n
+    amp = torch.rand(batch, 1, 1, generator=g, device=dev)
+    u = (amp * torch.sin(2 * math.pi * x) + 0.3 + 0.02 * torch.randn(batch, 1, n, generator=g, device=dev)).contiguous()
+    src = torch.randn(1, 1, n, generator=g, device=dev)
+    dt, mi = 0.1 / n, [(0, 1.0, n)]
+    nus = [0.02 + 0.01 * b for b in range(batch)]
+    for kind, scheme in (("conv", "SETDRK4"), ("cons", "SETDRK3")):
+        plan = SpectralPlan(mi, batch, 1, nonlinear=kind, nonlinear_coef=-1.0,
+                            linear=[("lap", nus if batch > 1 else nus[0])], device=dev)
+        assert plan.general
+        plan.add_source(src, 0.2)
+        plan.set_scheme(scheme, dt)
+        uh = plan.forward(u)
+        rec = torch.tensor([0, -1, 1, -1, 2], dtype=torch.int32, device=dev)
+        traj = torch.zeros((batch, 3) + tuple(plan.spec_shape[1:]), dtype=torch.complex64, device=dev)
+        plan.step(uh, 4, rec, traj)
+        for b in range(batch):
+            terms = [(nus[b], "lap", None), (-1, kind, None), (0.2, "src", src)]
+            for t, k in ((1, 2), (2, 4)):
+                ref = refpath.integrate(terms, mi, u[b:b + 1], dt, k, scheme=scheme)
+                assert _rel(plan.inverse(traj[b:b + 1, t].contiguous()), ref) <= TOL
+            assert _rel(plan.inverse(uh[b:b + 1].contiguous()), ref) <= TOL

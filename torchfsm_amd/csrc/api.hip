@@ -162,6 +162,9 @@ struct tfsm_plan {
   float2* gtmp = nullptr;  // four-step scratch of those axes
   float2* force = nullptr;  // NSPressureConvection's external force spectrum [forceB][forceC][modes]
   int forceB = 0, forceC = 0;
+  // general plans that step on the fused kernels of run-time lengths (k_genfused.hip): 2D (gf_row, gf_col: that
+  // axis takes the run-time kernel, the other one its fixed-size kernel) or the persistent 1D stepper
+  bool genf = false, gf_row = false, gf_col = false;
   size_t ws_fused = 0;     // workspace of the fused path (the unfused buffers follow it)
   size_t off_gS = 0, off_gF = 0, off_gR = 0, off_gQ = 0;
 
@@ -405,6 +408,15 @@ GenArgs gen_args(const tfsm_plan* p) {
 // unfused buffers after the fused workspace: S (stage spectrum), F (fields, later product spectra),
 // R (real fields), Q (real products)
 void gen_layout(tfsm_plan* p) {
+  if (p->genf) {
+    p->ws_bytes = p->ws_fused;
+    if (p->D == 2) {  // products and fields of the fused 2D layout
+      p->off_P = roundup(p->ws_fused, 256);
+      p->off_G = p->off_P + roundup(p->state_elems() * sizeof(float2), 256);
+      p->ws_bytes = p->off_G + roundup((size_t)p->B * p->NF * p->n[0] * p->PF * sizeof(float2), 256);
+    }
+    return;
+  }
   const GenArgs g = gen_args(p);
   const size_t sb = p->state_elems() * sizeof(float2);
   const size_t nfa = (size_t)(g.NF > g.NP ? g.NF : g.NP);
@@ -437,6 +449,35 @@ int build_gaxes(tfsm_plan* p) {
     if (t > tmp) tmp = t;
   }
   if (tmp) return dev_alloc(p, &p->gtmp, tmp, "general FFT scratch");
+  return TFSM_OK;
+}
+
+// Whether a general plan steps on the fused kernels of run-time lengths, and which axes take them (an axis
+// with fixed-size kernels keeps those: they hold the transform in registers)
+int plan_genfused(tfsm_plan* p) {
+  if (p->cplx || p->force) return TFSM_OK;
+  if (p->D == 1) {
+    p->genf = (p->term == TERM_CONV || p->term == TERM_CONS) && p->C == 1 && genfused_axis(p->gax[0]);
+    return TFSM_OK;
+  }
+  if (p->D != 2 || p->term == TERM_CONS) return TFSM_OK;
+  // fixed-size columns address whole pitch rows of the y wavenumber table (16 points at least); the paired
+  // 512-point vorticity rows need an even number of rows per sample
+  bool gen[2] = {!col2d_supported(p->n[0], 8, 0) || p->n[1] < 16,
+                 !row2d_supported(p->n[1], 0, 256) || (p->n[1] == 512 && p->n[0] % 2 != 0)};
+  for (int d = 0; d < 2; ++d) {
+    if (!gen[d]) continue;
+    if (p->gax[d].n != p->n[d]) {
+      hipError_t e = gaxis_build(p->gax[d], p->n[d], p->allocs);
+      if (e != hipSuccess) return hip_fail(e, "general FFT tables");
+    }
+    if (!genfused_axis(p->gax[d])) return TFSM_OK;
+  }
+  p->genf = true;
+  p->gf_col = gen[0];
+  p->gf_row = gen[1];
+  p->NF = p->term == TERM_KS ? 2 : 4;
+  p->PF = (int)roundup((size_t)p->kmax[1] + 1, 16);
   return TFSM_OK;
 }
 
@@ -580,6 +621,10 @@ Col2Args col_args(tfsm_plan* p, float2* U, char* ws) {
 int launch_row(tfsm_plan* p, char* ws, int b0, int nb, hipStream_t st, StepMask m = StepMask()) {
   Row2Args r = row_args(p, ws, b0, nb);
   r.mask = m;
+  if (p->gf_row) {
+    HIP_TRY(launch_g2row(p->term, r, p->gax[1], st), "row kernel launch");
+    return TFSM_OK;
+  }
   HIP_TRY(launch_row2d(p->term, r, p->row_var, p->row_wg, st), "row kernel launch");
   return TFSM_OK;
 }
@@ -588,6 +633,10 @@ int launch_col(tfsm_plan* p, float2* U, char* ws, int stage, int b0, int nb, hip
   Col2Args c = col_args(p, U, ws);
   c.b0 = b0;
   c.mask = m;
+  if (p->gf_col) {
+    HIP_TRY(launch_g2col(p->term, c, p->gax[0], nb, stage, st), "column kernel launch");
+    return TFSM_OK;
+  }
   HIP_TRY(launch_col2d(p->term, c, nb, stage, p->V, p->col_var, st), "column kernel launch");
   return TFSM_OK;
 }
@@ -778,6 +827,10 @@ Run1Args run1_args(tfsm_plan* p, float2* U, char* ws) {
   return a;
 }
 
+hipError_t run1d(tfsm_plan* p, const Run1Args& a, hipStream_t st) {
+  return p->genf ? launch_g1run(a, p->gax[0], st) : launch_run1d(a, st);
+}
+
 // act: optional per-sample step counts (device int32 [B], 2D / 3D): sample b advances by
 // min(act[b], nsteps) steps and is not touched after that
 int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* traj, int T, void* ws, hipStream_t st,
@@ -795,7 +848,7 @@ int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* tra
     return TFSM_OK;
   }
   if (!ws) return fail(TFSM_E_INVALID, "workspace pointer is null");
-  if (p->general) return gen_step(p, U, nsteps, rec_slot, traj, T, (char*)ws, st, act);
+  if (p->general && !p->genf) return gen_step(p, U, nsteps, rec_slot, traj, T, (char*)ws, st, act);
   if (p->D == 1 && p->term == TERM_KS) {
     // one launch per stage (the batch mean couples the samples): raw product -> mean -> combine
     Run1Args a = run1_args(p, U, (char*)ws);
@@ -833,7 +886,7 @@ int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* tra
     a.rec_slot = rec_slot;
     a.traj = (float2*)traj;
     a.T = T;
-    HIP_TRY(launch_run1d(a, st), "1D stepper launch");
+    HIP_TRY(run1d(p, a, st), "1D stepper launch");
     return TFSM_OK;
   }
   if (p->D == 2 && p->persistent && run2d_supported(p->term, p->n[0], p->n[1], p->PF) && !p->cplx) {
@@ -999,8 +1052,8 @@ int adj_jt(tfsm_plan* p, const float2* U, const float2* V, float2* W, char* wsa,
 
 // N(U) -> workspace A1
 int eval_nonlinear(tfsm_plan* p, float2* U, char* ws, hipStream_t st) {
-  if (p->general) return gen_stage(p, U, U, ws, ST_EVAL, StepMask(), st);
-  if (p->l1) {
+  if (p->general && !p->genf) return gen_stage(p, U, U, ws, ST_EVAL, StepMask(), st);
+  if (p->l1 && !p->general) {
     int rc = run_long1d(p, U, ws, ST_PRO, st);
     return rc ? rc : run_long1d(p, U, ws, ST_EVAL, st);
   }
@@ -1008,7 +1061,7 @@ int eval_nonlinear(tfsm_plan* p, float2* U, char* ws, hipStream_t st) {
     Run1Args r = run1_args(p, U, ws);
     r.eval_only = 1;
     r.nsteps = 1;
-    HIP_TRY(launch_run1d(r, st), "1D evaluation launch");
+    HIP_TRY(run1d(p, r, st), "1D evaluation launch");
     return TFSM_OK;
   }
   int rc = run_eval(p, U, ws, ST_PRO, 0, p->B, st);
@@ -1448,14 +1501,15 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     p->off_DC = p->ws_bytes;
     p->ws_bytes += 256;
     p->ws_fused = p->ws_bytes;
-    if (p->general) gen_layout(p);
+    if (p->general) rc = plan_genfused(p);
+    if (!rc && p->general) gen_layout(p);
   }
   // default launch shape (the autotuner may refine it): 2D columns of 512 points run the
   // half-thread radix plan for one-channel products (the two-channel ones keep a second column in
   // registers and run faster with 8 values per thread); temporal blocking uses the smallest
   // sub-batch (multiple of 8) that still gives >= 512 column workgroups (two per CU) while its
   // working set stays under 256 MB
-  if (!rc && D == 2 && p->fused_ok) {
+  if (!rc && D == 2 && (p->fused_ok || p->genf)) {
     const bool one_channel = term == TERM_VC || term == TERM_KS;
     const int n0 = p->n[0], n1 = p->n[1];
     // measured per axis size: 512 keeps 16-column tiles; 64, 128 and 256 run 8-column tiles and rows of 4
@@ -1483,13 +1537,13 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     const int tiles = (p->H + p->V - 1) / p->V;
     int sb = 8;
     while (sb < p->B && (size_t)tiles * sb < 512) sb += 8;
-    if (sb >= p->B || (size_t)sb * per_sample > ((size_t)256 << 20) || p->ks_mean) sb = 0;
+    if (sb >= p->B || (size_t)sb * per_sample > ((size_t)256 << 20) || p->ks_mean || p->genf) sb = 0;
     p->sub_batch = sb;
     // 512-point one-channel columns (VorticityConvection) with 32 or more samples: sub-batches of 16
     // on two streams, so one sub-batch's VALU-bound row pass overlaps the other's memory-bound
     // column pass (NS 512^2, B = 64: 0.630 ms/step against 0.662 for one stream and 32-sample
     // sub-batches, and 0.676 for the 16-values-per-thread columns it replaces)
-    if (n0 == 512 && term == TERM_VC && p->B >= 32) {
+    if (n0 == 512 && term == TERM_VC && p->B >= 32 && !p->genf) {
       p->sub_batch = 16;
       rc = tfsm_plan_set_streams(p, 2);
     }
@@ -1499,7 +1553,7 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     // 0.248); 256^2 VorticityConvection and Convection in 16-sample sub-batches, on two streams
     // from B = 32 (0.130 -> 0.119, 0.169 -> 0.157) and on four from B = 64 (0.259 -> 0.164, 0.337
     // -> 0.213)
-    const bool square = p->n[0] == p->n[1];
+    const bool square = p->n[0] == p->n[1] && !p->genf;
     if (!rc && square && n0 == 512 && (term == TERM_CONV || term == TERM_NSP) && p->B >= 16) {
       p->sub_batch = p->B >= 32 ? 16 : 8;
       rc = tfsm_plan_set_streams(p, 2);
@@ -1902,8 +1956,9 @@ int tfsm_plan_add_force(tfsm_plan* p, const float* force, int32_t force_batch, i
   // the forced core masks the integrator's stage tensors in place: only the unfused path does that
   p->fused_ok = false;
   p->persistent = false;
-  if (!p->general) {
+  if (!p->general || p->genf) {
     p->general = true;
+    p->genf = p->gf_row = p->gf_col = false;
     gen_layout(p);
   }
   return TFSM_OK;
@@ -1965,9 +2020,7 @@ int tfsm_apply(tfsm_plan* p, const void* uh, void* out, void* ws, void* stream) 
   float2* U = (float2*)uh;
   if (have_nl) {
     if (!ws) return fail(TFSM_E_INVALID, "workspace pointer is null");
-    if (p->general) {
-      if (int rc = gen_stage(p, U, U, (char*)ws, ST_EVAL, StepMask(), st)) return rc;
-    } else if (p->l1) {
+    if (p->general || p->l1) {
       if (int rc = eval_nonlinear(p, U, (char*)ws, st)) return rc;
     } else if (p->D == 1 && p->term == TERM_KS) {
       Run1Args a = run1_args(p, U, (char*)ws);

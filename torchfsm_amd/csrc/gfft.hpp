@@ -1,8 +1,9 @@
 // General-length batched FFTs for the axes the fixed-size kernels do not cover (mesh.py:481-491
-// transforms any length).  A length n that factors into 2, 3, 5 and 7 runs a Stockham FFT with
-// runtime radices (4, 2, 3, 5, 7) in one workgroup's LDS; any other n runs Bluestein's algorithm,
-// a circular convolution of length M = 2^k >= 2n - 1.  Transforms longer than GFFT_LDS_MAX points
-// split L = L1 * L2 into two LDS passes (four-step: L1-point FFTs, twiddles, L2-point FFTs).
+// transforms any length).  A length n that factors into 2, 3, 5, 7, 11 and 13 runs a Stockham FFT with
+// run-time radices 2..16 in one workgroup's LDS (gx_core.hpp); any other n runs Bluestein's algorithm, a
+// circular convolution of the cheapest such length M >= 2n - 1.  Transforms longer than GFFT_LDS_MAX points
+// split L = L1 * L2 into two LDS passes (four-step: L1-point FFTs, twiddles, L2-point FFTs; Bluestein's
+// M is then a power of two).
 //
 // A batch of lines is described by GLines: line (o, i) starts at element o * os + i * is and its
 // t-th element sits at + t * es.  Modes: C2C (complex n -> complex n), R2C (real n -> the n/2 + 1
@@ -19,17 +20,19 @@
 namespace tfsm {
 
 constexpr int GFFT_LDS_MAX = 4096;  // longest FFT held in one workgroup's LDS (2 x 32 KB ping-pong)
-constexpr int GFFT_MAX_RADICES = 16;
-constexpr int GFFT_THREADS = 256;
+constexpr int GFFT_MAX_RADICES = 8;
 
 enum GfftMode : int { GM_C2C = 0, GM_R2C = 1, GM_C2R = 2 };
 
-// radix sequence and twiddles exp(-2 pi i t / L), t < L, of one in-LDS FFT length
+// radix sequence and twiddles exp(-2 pi i t / L), t < L, of one in-LDS FFT length.  Stage s combines
+// ns[s] points (the product of the earlier radices) in nb[s] = L / r[s] butterflies; its twiddles are
+// w_L^(q k span[s]), span[s] = L / (ns[s] r[s]), and mg[s] = ceil(2^32 / ns[s]) divides by ns[s]
+// (exact below 2^16).
 struct GRadix {
   int L = 0;
   int nr = 0;
-  int r[GFFT_MAX_RADICES] = {};
-  int pow2 = 0;  // every radix is 2 or 4: stage indices by shifts and masks
+  int r[GFFT_MAX_RADICES] = {}, ns[GFFT_MAX_RADICES] = {}, nb[GFFT_MAX_RADICES] = {}, span[GFFT_MAX_RADICES] = {};
+  unsigned mg[GFFT_MAX_RADICES] = {};
   const float2* tw = nullptr;
 };
 
@@ -50,7 +53,7 @@ struct GLines {
   size_t os = 0, is = 0, es = 1;
 };
 
-// true when n factors into 2, 3, 5 and 7
+// true when n factors into 2, 3, 5, 7, 11 and 13
 bool gfft_smooth(int n);
 // build the tables of length n (n >= 1); device allocations are appended to `allocs`
 hipError_t gaxis_build(GAxis& a, int n, std::vector<void*>& allocs);
@@ -60,5 +63,14 @@ size_t gfft_tmp_elems(const GAxis& a, size_t lines);
 // tmp: gfft_tmp_elems(a, n_o * n_i) complex elements, or nullptr when that is 0
 hipError_t gfft_run(const GAxis& a, int mode, int dir, const void* in, const GLines& li, void* out, const GLines& lo,
                     float scale, float2* tmp, hipStream_t st);
+
+struct Col2Args;
+struct Row2Args;
+struct Run1Args;
+// fused kernels of run-time lengths (k_genfused.hip): whether an axis fits them, and their launches
+bool genfused_axis(const GAxis& ax);
+hipError_t launch_g2col(int term, const Col2Args& a, const GAxis& ax, int nb, int stage, hipStream_t st);
+hipError_t launch_g2row(int term, const Row2Args& a, const GAxis& ax, hipStream_t st);
+hipError_t launch_g1run(const Run1Args& a, const GAxis& ax, hipStream_t st);
 
 }  // namespace tfsm

@@ -1,15 +1,23 @@
-// General-length batched FFTs (declarations and conventions in gfft.hpp).
+// General-length batched FFTs (declarations and conventions in gfft.hpp, the in-LDS stages in gx_core.hpp).
 //
-// One workgroup of 256 threads transforms 256 / T lines, T threads per line (T = the power of two
-// nearest above L / 4, within 16..256).  A line is gathered from its strided layout into LDS (real
-// inputs promoted, Hermitian halves mirrored, Bluestein chirp applied), transformed by Stockham
-// autosort stages with runtime radices (a ping-pong pair of L-point buffers), and scattered back
-// with the output's own index map (first n/2 + 1 values for R2C, real parts for C2R).  Four-step
-// and Bluestein transforms chain these launches through a scratch buffer.
+// One workgroup transforms V lines that are consecutive in the batch's fastest index (V a power of two, up to
+// 16, so that two buffers of V lines fit LDS and the launch still fills the GPU).  The lines are gathered
+// from their strided layout into LDS (real inputs promoted, Hermitian halves mirrored, Bluestein chirp
+// applied), transformed, and scattered with the output's own index map (first n/2 + 1 values for R2C,
+// real parts for C2R).  Threads walk the lines interleaved where adjacent lines are adjacent in memory
+// (strided columns, four-step passes), one line after the other otherwise (rows), so that both coalesce; a
+// run of lines that V does not divide ends in a partly filled workgroup.  Four-step and long Bluestein
+// transforms chain these launches through a scratch buffer.
+//
+// Bound by latency and instruction issue, not bandwidth.  Forward transforms, us, before (radices 2..7, one
+// element's load at a time, 16 adjacent lines or one) and now: 65536 points, B = 16 57 -> 30; 225 x 301,
+// B = 16 65 -> 46; 1000^2, B = 4 89 -> 56; 120^3, B = 3 110 -> 82; 84 x 76 x 96, B = 3 65 -> 52.
 #include <cmath>
+#include <complex>
 #include <vector>
 
 #include "gfft.hpp"
+#include "gx_core.hpp"
 
 namespace tfsm {
 namespace {
@@ -35,11 +43,11 @@ struct GLaunch {
   int twdir;
   const float2* twt;     // its table exp(-2 pi i t / twn), t < twn (null: computed in float64)
   float scale;
-  int T;
-  // the workgroup's lines are consecutive s (n_s > 1) or i (n_s == 1) of one (o, i) / o, and
-  // adjacent lines are adjacent in memory on input (ilv_in) / output (ilv_out): the threads then
-  // walk those lines interleaved, so neighbouring threads touch neighbouring addresses
-  int ilv_in, ilv_out;
+  // set by launch_g: V = 1 << vl lines per workgroup, consecutive in the fastest index with more than one
+  // value (fd: 0 o, 1 i, 2 s); threads walk them interleaved on input / output where they are adjacent
+  int vl, fd, ilv_in, ilv_out;
+  unsigned mgL;          // ceil(2^32 / L)
+  int twlds;             // the stage twiddles are staged in LDS
 };
 
 __device__ __forceinline__ float2 gmul(float2 a, float2 b) {
@@ -51,287 +59,218 @@ __device__ __forceinline__ float2 gtw(const float2* tw, int t, int dir) {
   return dir < 0 ? w : make_float2(w.x, -w.y);
 }
 
-// in-register DFT of R values; w_R = exp(dir 2 pi i / R) read from the L-point table
-template <int R>
-__device__ __forceinline__ void gbfly(float2 (&v)[7], const float2* tw, int L, int dir) {
-  if constexpr (R == 2) {
-    const float2 a = v[0], b = v[1];
-    v[0] = make_float2(a.x + b.x, a.y + b.y);
-    v[1] = make_float2(a.x - b.x, a.y - b.y);
-  } else if constexpr (R == 4) {
-    const float2 t0 = make_float2(v[0].x + v[2].x, v[0].y + v[2].y);
-    const float2 t1 = make_float2(v[0].x - v[2].x, v[0].y - v[2].y);
-    const float2 t2 = make_float2(v[1].x + v[3].x, v[1].y + v[3].y);
-    const float2 d = make_float2(v[1].x - v[3].x, v[1].y - v[3].y);
-    const float2 t3 = dir < 0 ? make_float2(d.y, -d.x) : make_float2(-d.y, d.x);  // d * (-i) or d * i
-    v[0] = make_float2(t0.x + t2.x, t0.y + t2.y);
-    v[2] = make_float2(t0.x - t2.x, t0.y - t2.y);
-    v[1] = make_float2(t1.x + t3.x, t1.y + t3.y);
-    v[3] = make_float2(t1.x - t3.x, t1.y - t3.y);
-  } else {
-    float2 w[R];
-#pragma unroll
-    for (int m = 0; m < R; ++m) w[m] = gtw(tw, m * (L / R), dir);
-    float2 y[R];
-#pragma unroll
-    for (int m = 0; m < R; ++m) {
-      float2 acc = v[0];
-#pragma unroll
-      for (int q = 1; q < R; ++q) {
-        const float2 p = gmul(v[q], w[(q * m) % R]);
-        acc.x += p.x;
-        acc.y += p.y;
-      }
-      y[m] = acc;
-    }
-#pragma unroll
-    for (int m = 0; m < R; ++m) v[m] = y[m];
-  }
-}
-
-// one Stockham stage: Ns points already combined; butterfly b reads b + q L/R, twiddles by
-// w^(q (b mod Ns)) with w = exp(dir 2 pi i / (Ns R)), writes (b / Ns) Ns R + (b mod Ns) + q Ns
-template <int R>
-__device__ void gstage(const float2* src, float2* dst, const float2* tw, int L, int Ns, int nsl, int dir, int t,
-                       int T) {
-  const int nb = L / R, span = L / (Ns * R);
-  for (int b = t; b < nb; b += T) {
-    // nsl = log2(Ns) for power-of-two plans (no integer division), else -1
-    const int k = nsl >= 0 ? (b & (Ns - 1)) : b % Ns;
-    const int grp = nsl >= 0 ? (b >> nsl) : b / Ns;
-    float2 v[7];
-#pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = src[b + q * nb];
-    if (Ns > 1) {
-#pragma unroll
-      for (int q = 1; q < R; ++q) v[q] = gmul(v[q], gtw(tw, q * k * span, dir));
-    }
-    gbfly<R>(v, tw, L, dir);
-    const int d0 = grp * Ns * R + k;
-#pragma unroll
-    for (int q = 0; q < R; ++q) dst[d0 + q * Ns] = v[q];
-  }
-}
-
-// every stage of g; the result ends in *src (every thread of the workgroup takes part)
-__device__ void gfft_lds(const GRadix& g, int dir, float2*& src, float2*& dst, int t, int T) {
-  int Ns = 1, nsl = g.pow2 ? 0 : -1;
-  for (int s = 0; s < g.nr; ++s) {
-    const int R = g.r[s];
-    switch (R) {
-      case 4: gstage<4>(src, dst, g.tw, g.L, Ns, nsl, dir, t, T); break;
-      case 2: gstage<2>(src, dst, g.tw, g.L, Ns, nsl, dir, t, T); break;
-      case 3: gstage<3>(src, dst, g.tw, g.L, Ns, nsl, dir, t, T); break;
-      case 5: gstage<5>(src, dst, g.tw, g.L, Ns, nsl, dir, t, T); break;
-      default: gstage<7>(src, dst, g.tw, g.L, Ns, nsl, dir, t, T); break;
-    }
-    __syncthreads();
-    float2* x = src;
-    src = dst;
-    dst = x;
-    Ns *= R;
-    if (nsl >= 0) nsl += R == 4 ? 2 : 1;
-  }
-}
-
-__global__ void __launch_bounds__(GFFT_THREADS) k_gfft(GLaunch a) {
+__global__ void __launch_bounds__(512) k_gfft(GLaunch a) {
   extern __shared__ float2 g_lds[];
-  const int T = a.T, L = a.g.L;
-  const int lpw = GFFT_THREADS / T;
-  // T and lpw are powers of two
-  const int tsh = __ffs(T) - 1, lsh = __ffs(lpw) - 1;
-  const int sub = threadIdx.x >> tsh, t = threadIdx.x & (T - 1);
-  float2* src = g_lds + (size_t)sub * 2 * L;
-  float2* dst = src + L;
-  const long long nlines = a.n_o * a.n_i * a.n_s;
-  const long long line = (long long)blockIdx.x * lpw + sub;
-  const bool valid = line < nlines;
-  long long s = 0, i = 0, o = 0;
-  if (valid) {
-    s = line % a.n_s;
-    const long long r = line / a.n_s;
-    i = r % a.n_i;
-    o = r / a.n_i;
+  const int L = a.g.L, nth = blockDim.x, tid = threadIdx.x;
+  GxLines ln;
+  ln.vl = a.vl;
+  ln.V = 1 << a.vl;
+  const int slots = gx_slots(L, 1 << a.vl);
+  float2* cur = g_lds;
+  float2* alt = g_lds + slots;
+  const float2* tw = a.g.tw;
+  if (a.twlds) {
+    float2* t = g_lds + 2 * slots;
+    for (int i = tid; i < L; i += nth) t[i] = a.g.tw[i];
+    tw = t;
   }
-  const long long L0 = (long long)blockIdx.x * lpw;  // first line of the workgroup
-  long long s0 = 0, i0 = 0, o0 = 0;
-  if (a.ilv_in || a.ilv_out) {
-    s0 = L0 % a.n_s;
-    const long long r0 = L0 / a.n_s;
-    i0 = r0 % a.n_i;
-    o0 = r0 / a.n_i;
-  }
-  if (a.ilv_in) {
-    for (int e = threadIdx.x; e < lpw * L; e += GFFT_THREADS) {
-      const int ls = e & (lpw - 1), j = e >> lsh;
-      float2 v = make_float2(0.f, 0.f);
-      const long long sl = a.n_s > 1 ? s0 + ls : 0, il = a.n_s > 1 ? i0 : i0 + ls;
-      const long long q = (long long)j * a.qj + sl * a.qs;
-      if (L0 + ls < nlines && q < a.nload) {
-        const long long ibl = o0 * a.ios + il * a.iis;
-        if (a.in_mode == 1) {
-          v.x = ((const float*)a.in)[ibl + q * a.ies];
-        } else if (a.in_mode == 2) {
-          const float2* x = (const float2*)a.in;
-          if (q < a.hbins) {
-            v = x[ibl + q * a.ies];
-          } else {
-            const float2 m = x[ibl + (a.nfull - q) * a.ies];
-            v = make_float2(m.x, -m.y);
-          }
-          if (q == 0 || 2 * q == a.nfull) v.y = 0.f;
-        } else {
-          v = ((const float2*)a.in)[ibl + q * a.ies];
-        }
-        if (a.pre) v = gmul(v, a.pre[q]);
-      }
-      g_lds[(size_t)ls * 2 * L + j] = v;
-    }
-  }
-  const long long ib = o * a.ios + i * a.iis;
-  for (int j = t; j < L && !a.ilv_in; j += T) {
-    float2 v = make_float2(0.f, 0.f);
-    const long long q = (long long)j * a.qj + s * a.qs;
-    if (valid && q < a.nload) {
-      if (a.in_mode == 1) {
-        v.x = ((const float*)a.in)[ib + q * a.ies];
-      } else if (a.in_mode == 2) {
-        const float2* x = (const float2*)a.in;
-        if (q < a.hbins) {
-          v = x[ib + q * a.ies];
-        } else {
-          const float2 m = x[ib + (a.nfull - q) * a.ies];
-          v = make_float2(m.x, -m.y);
-        }
-        if (q == 0 || 2 * q == a.nfull) v.y = 0.f;
+  // the workgroup's first line, and how many of its V lines exist
+  const long long nf = a.fd == 0 ? a.n_o : (a.fd == 1 ? a.n_i : a.n_s);
+  const long long groups = (nf + ln.V - 1) >> a.vl;
+  const long long f0 = ((long long)blockIdx.x % groups) << a.vl, rest = (long long)blockIdx.x / groups;
+  const int nv = (int)(nf - f0 < ln.V ? nf - f0 : ln.V);
+  const long long o0 = a.fd == 0 ? f0 : (a.fd == 1 ? rest : rest / a.n_i);
+  const long long i0 = a.fd == 0 ? 0 : (a.fd == 1 ? f0 : rest % a.n_i);
+  const long long s0 = a.fd == 2 ? f0 : 0;
+  const long long ib0 = o0 * a.ios + i0 * a.iis, ob0 = o0 * a.oos + i0 * a.ois;
+  const long long dib = a.fd == 0 ? a.ios : (a.fd == 1 ? a.iis : 0), dob = a.fd == 0 ? a.oos : (a.fd == 1 ? a.ois : 0);
+  const int ds = a.fd == 2 ? 1 : 0;
+  const int total = L << a.vl;
+  const bool inv = a.dir > 0;
+  // loads in batches of GB per thread, issued before the first of them is used (one element at a time, a
+  // workgroup paid a memory latency per element of its longest thread)
+  constexpr int GB = 4;
+  for (int e0 = tid; e0 < total; e0 += GB * nth) {
+    float2 z[GB], c[GB];
+    int vv[GB], jj[GB];
+    bool ok[GB], cj[GB];
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      const int e = e0 + u * nth;
+      if (a.ilv_in) {
+        vv[u] = e & (ln.V - 1);
+        jj[u] = e >> a.vl;
       } else {
-        v = ((const float2*)a.in)[ib + q * a.ies];
+        vv[u] = (int)__umulhi((unsigned)e, a.mgL);
+        jj[u] = e - vv[u] * L;
       }
-      if (a.pre) v = gmul(v, a.pre[q]);
+      long long q = (long long)jj[u] * a.qj + (s0 + ds * vv[u]) * a.qs;
+      ok[u] = e < total && vv[u] < nv && q < a.nload;
+      if (!ok[u]) q = 0;
+      const long long ib = ib0 + (ok[u] ? vv[u] : 0) * dib;
+      cj[u] = a.in_mode == 2 && q >= a.hbins;
+      const long long o = ib + (cj[u] ? a.nfull - q : q) * a.ies;
+      if (a.in_mode == 1) z[u] = make_float2(((const float*)a.in)[o], 0.f);
+      else z[u] = ((const float2*)a.in)[o];
+      if (a.in_mode == 2 && (q == 0 || 2 * q == a.nfull)) z[u].y = 0.f;
+      c[u] = a.pre ? a.pre[q] : make_float2(1.f, 0.f);
     }
-    src[j] = v;
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      if (e0 + u * nth >= total) continue;
+      float2 x = cj[u] ? make_float2(z[u].x, -z[u].y) : z[u];
+      if (a.pre) x = gmul(x, c[u]);
+      if (!ok[u]) x = make_float2(0.f, 0.f);
+      cur[ln.slot(jj[u], vv[u])] = inv ? gx_swap(x) : x;
+    }
   }
   __syncthreads();
-  gfft_lds(a.g, a.dir, src, dst, t, T);
-  if (a.bmid) {
-    for (int k = t; k < L; k += T) src[k] = gmul(src[k], a.bmid[k]);
-    __syncthreads();
-    gfft_lds(a.g, +1, src, dst, t, T);
-  }
-  if (a.ilv_out) {
-    // every line ends in the same buffer of its pair: this thread's offset holds for all of them
-    const int fo = (int)(src - (g_lds + (size_t)sub * 2 * L));
-    for (int e = threadIdx.x; e < lpw * L; e += GFFT_THREADS) {
-      const int ls = e & (lpw - 1), k = e >> lsh;
-      if (L0 + ls >= nlines) continue;
-      const long long sl = a.n_s > 1 ? s0 + ls : 0, il = a.n_s > 1 ? i0 : i0 + ls;
-      const long long r = (long long)k * a.rk + sl * a.rs;
-      if (r >= a.nstore) continue;
-      float2 v = g_lds[(size_t)ls * 2 * L + fo + k];
-      if (a.twn) {
-        long long e2 = (long long)k * sl;  // k < L1, s < L2: below twn = L1 L2
-        if (e2 >= a.twn) e2 %= a.twn;
-        if (a.twt) {
-          v = gmul(v, gtw(a.twt, (int)e2, a.twdir));
-        } else {
-          double sn, cs;
-          sincos((double)a.twdir * 2.0 * M_PI * (double)e2 / (double)a.twn, &sn, &cs);
-          v = gmul(v, make_float2((float)cs, (float)sn));
-        }
-      }
-      if (a.post) v = gmul(v, a.post[r]);
-      v.x *= a.scale;
-      v.y *= a.scale;
-      const long long obl = o0 * a.oos + il * a.ois;
-      if (a.out_mode == 1)
-        ((float*)a.out)[obl + r * a.oes] = v.x;
-      else
-        ((float2*)a.out)[obl + r * a.oes] = v;
+  bool swapped = inv;
+#pragma unroll 1
+  for (int pass = 0;; ++pass) {
+    gx_fft(a.g, tw, cur, alt, ln, tid, nth);
+    if (!a.bmid || pass == 1) break;
+    for (int e = tid; e < total; e += nth) {
+      const int v = e & (ln.V - 1), k = e >> a.vl, sl = ln.slot(k, v);
+      const float2 z = cur[sl];
+      cur[sl] = gx_swap(gmul(swapped ? gx_swap(z) : z, a.bmid[k]));
     }
-    return;
+    swapped = true;
+    __syncthreads();
   }
-  if (!valid) return;
-  const long long ob = o * a.oos + i * a.ois;
-  for (int k = t; k < L; k += T) {
-    const long long r = (long long)k * a.rk + s * a.rs;
-    if (r >= a.nstore) continue;
-    float2 v = src[k];
+  for (int e = tid; e < total; e += nth) {
+    int v, k;
+    if (a.ilv_out) {
+      v = e & (ln.V - 1);
+      k = e >> a.vl;
+    } else {
+      v = (int)__umulhi((unsigned)e, a.mgL);
+      k = e - v * L;
+    }
+    const long long s = s0 + ds * v, r = (long long)k * a.rk + s * a.rs;
+    if (v >= nv || r >= a.nstore) continue;
+    float2 z = cur[ln.slot(k, v)];
+    if (swapped) z = gx_swap(z);
     if (a.twn) {
-      long long e = (long long)k * s;  // k < L1, s < L2: below twn = L1 L2
-      if (e >= a.twn) e %= a.twn;
+      long long t = (long long)k * s;  // k < L1, s < L2: below twn = L1 L2
+      if (t >= a.twn) t %= a.twn;
       if (a.twt) {
-        v = gmul(v, gtw(a.twt, (int)e, a.twdir));
+        z = gmul(z, gtw(a.twt, (int)t, a.twdir));
       } else {
         double sn, cs;
-        sincos((double)a.twdir * 2.0 * M_PI * (double)e / (double)a.twn, &sn, &cs);
-        v = gmul(v, make_float2((float)cs, (float)sn));
+        sincos((double)a.twdir * 2.0 * M_PI * (double)t / (double)a.twn, &sn, &cs);
+        z = gmul(z, make_float2((float)cs, (float)sn));
       }
     }
-    if (a.post) v = gmul(v, a.post[r]);
-    v.x *= a.scale;
-    v.y *= a.scale;
+    if (a.post) z = gmul(z, a.post[r]);
+    z.x *= a.scale;
+    z.y *= a.scale;
+    const long long ob = ob0 + v * dob;
     if (a.out_mode == 1)
-      ((float*)a.out)[ob + r * a.oes] = v.x;
+      ((float*)a.out)[ob + r * a.oes] = z.x;
     else
-      ((float2*)a.out)[ob + r * a.oes] = v;
+      ((float2*)a.out)[ob + r * a.oes] = z;
   }
 }
 
-int threads_per_line(int L) {
-  int t = 16;
-  while (t < GFFT_THREADS && t * 4 < L) t *= 2;
-  return t;
-}
+constexpr size_t GX_LDS_BYTES = 150 * 1024;  // of 160 KB
 
 hipError_t launch_g(GLaunch a, hipStream_t st) {
-  a.T = threads_per_line(a.g.L);
-  // lines adjacent in memory (strided transforms: columns, four-step passes): up to 16 lines per
-  // workgroup, walked interleaved, so that their loads and stores coalesce
-  const long long run = a.n_s > 1 ? a.n_s : a.n_i;
-  const long long din = a.n_s > 1 ? a.qs * a.ies : a.iis, dout = a.n_s > 1 ? a.rs * a.oes : a.ois;
-  a.ilv_in = a.ilv_out = 0;
-  if (din == 1 || dout == 1) {
-    int l = 1;
-    while (l < 16 && 2 * l * a.g.L <= GFFT_LDS_MAX && run % (2 * l) == 0) l *= 2;
-    if (l > 1) {
-      a.T = GFFT_THREADS / l;
-      a.ilv_in = din == 1;
-      a.ilv_out = dout == 1;
-    }
-  }
-  const long long lpw = GFFT_THREADS / a.T;
   const long long nlines = a.n_o * a.n_i * a.n_s;
   if (nlines <= 0) return hipSuccess;
-  const long long blocks = (nlines + lpw - 1) / lpw;
+  a.fd = a.n_s > 1 ? 2 : (a.n_i > 1 ? 1 : 0);
+  const long long nf = a.fd == 0 ? a.n_o : (a.fd == 1 ? a.n_i : a.n_s), outer = nlines / nf;
+  const long long din = a.fd == 2 ? a.qs * a.ies : (a.fd == 1 ? a.iis : a.ios);
+  const long long dout = a.fd == 2 ? a.rs * a.oes : (a.fd == 1 ? a.ois : a.oos);
+  const bool adj = din == 1 || dout == 1;
+  // lines per workgroup: about 4096 points, 16 lines at most; fewer while the launch has under two
+  // workgroups per CU (but 8 where adjacent lines share cache lines)
+  int vl = 0;
+  while (a.g.L > 1 && vl < 4 && ((long long)a.g.L << (vl + 1)) <= GFFT_LDS_MAX && (1 << vl) < nf) ++vl;
+  const int least = adj ? 3 : 0;
+  while (vl > least && outer * ((nf + (1 << vl) - 1) >> vl) < 512) --vl;
+  a.vl = vl;
+  a.ilv_in = vl && din == 1;
+  a.ilv_out = vl && dout == 1;
+  a.mgL = (unsigned)((0x100000000ULL + a.g.L - 1) / a.g.L);
+  const long long blocks = outer * ((nf + (1 << vl) - 1) >> vl);
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t lds = (size_t)lpw * 2 * a.g.L * sizeof(float2);
-  hipLaunchKernelGGL(k_gfft, dim3((unsigned)blocks), dim3(GFFT_THREADS), lds, st, a);
+  const size_t buf = (size_t)gx_slots(a.g.L, 1 << vl) * sizeof(float2);
+  a.twlds = 2 * buf + a.g.L * sizeof(float2) <= GX_LDS_BYTES ? 1 : 0;
+  const size_t lds = 2 * buf + (a.twlds ? a.g.L * sizeof(float2) : 0);
+  // one butterfly of about 8 values per thread
+  long long nth = ((((long long)a.g.L << vl) / 8 + 63) / 64) * 64;
+  nth = nth < 64 ? 64 : (nth > 512 ? 512 : nth);
+  hipLaunchKernelGGL(k_gfft, dim3((unsigned)blocks), dim3((unsigned)nth), lds, st, a);
   return hipGetLastError();
 }
 
-bool radices(int L, GRadix& g) {
-  g.L = L;
-  g.nr = 0;
-  g.pow2 = (L & (L - 1)) == 0 ? 1 : 0;
-  int n = L;
-  while (n % 4 == 0 && g.nr < GFFT_MAX_RADICES) {
-    g.r[g.nr++] = 4;
-    n /= 4;
+// The cheapest radix sequence by the time of one butterfly per thread, in cycles: a stage's barrier and LDS
+// latency, plus its LDS traffic, twiddles and index arithmetic (64 per value) and its arithmetic.  The
+// launches that matter are latency bound, so a few stages of radix 4 to 9 beat fewer of radix 15 and 16.
+constexpr int kRadices[] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 15, 16};
+constexpr int kStageCost[] = {670, 760, 820, 1020, 1110, 1350, 1270, 1550, 1720, 2100, 1850, 2500, 2560, 2300};
+void plan_radices(int n, int i, int cost, std::vector<int>& now, std::vector<int>& best, int& bestc) {
+  if (!best.empty() && cost >= bestc) return;
+  if (n == 1) {
+    best = now;
+    bestc = cost;
+    return;
   }
-  const int rs[4] = {2, 3, 5, 7};
-  for (int r : rs)
-    while (n % r == 0 && g.nr < GFFT_MAX_RADICES) {
-      g.r[g.nr++] = r;
-      n /= r;
+  for (int k = i; k >= 0; --k)
+    if (n % kRadices[k] == 0) {
+      now.push_back(kRadices[k]);
+      plan_radices(n / kRadices[k], k, cost + kStageCost[k], now, best, bestc);
+      now.pop_back();
     }
-  return n == 1;
 }
 
-// largest L1 <= GFFT_LDS_MAX dividing L with L / L1 <= GFFT_LDS_MAX (0: none)
+bool radices(int L, GRadix& g) {
+  g = GRadix();
+  g.L = L;
+  std::vector<int> now, best;
+  if (L > 1) {
+    int bestc = 0;
+    plan_radices(L, (int)(sizeof(kRadices) / sizeof(int)) - 1, 0, now, best, bestc);
+    if (best.empty() || (int)best.size() > GFFT_MAX_RADICES) return false;
+  }
+  int ns = 1;
+  for (int r : best) {
+    const int s = g.nr++;
+    g.r[s] = r;
+    g.ns[s] = ns;
+    g.nb[s] = L / r;
+    g.span[s] = L / (ns * r);
+    g.mg[s] = ns > 1 ? (unsigned)((0x100000000ULL + ns - 1) / ns) : 0;
+    ns *= r;
+  }
+  return true;
+}
+
+// L = L1 L2 with both at most GFFT_LDS_MAX, as square as possible (0: none).  Pass A's lines are strided by
+// L2 and gathered up to 16 adjacent ones at a time: a long L1 would leave LDS for one line only
+// (65536 points at 4096 * 16 and radices up to 7 57 us, at 256 * 256 30)
 int split_four(int L) {
-  for (int l1 = GFFT_LDS_MAX; l1 >= 2; --l1)
-    if (L % l1 == 0 && L / l1 <= GFFT_LDS_MAX) return l1;
+  for (int l1 = (int)std::ceil(std::sqrt((double)L)); l1 <= GFFT_LDS_MAX; ++l1)
+    if (L % l1 == 0) return l1;
   return 0;
+}
+
+// cheapest smooth circular length M >= 2n - 1 that one workgroup holds (0: none): points times LDS rounds
+int bluestein_length(int n) {
+  long long bestc = 0;
+  int best = 0;
+  for (int m = 2 * n - 1; m <= GFFT_LDS_MAX && m < 4 * n; ++m) {
+    if (best && (long long)m * 5 > bestc) break;  // no shorter plan than two stages
+    GRadix g;
+    if (!gfft_smooth(m) || !radices(m, g)) continue;
+    const long long c = (long long)m * (2 * g.nr + 1);
+    if (!best || c < bestc) {
+      best = m;
+      bestc = c;
+    }
+  }
+  return best;
 }
 
 hipError_t upload(const std::vector<float2>& h, const float2** out, std::vector<void*>& allocs) {
@@ -354,30 +293,27 @@ hipError_t build_radix(GRadix& g, int L, std::vector<void*>& allocs) {
   return upload(h, &g.tw, allocs);
 }
 
-// in-place radix-2 FFT in double (host), exponent sign -1
-void host_fft_pow2(std::vector<double>& re, std::vector<double>& im) {
-  const size_t n = re.size();
-  for (size_t i = 1, j = 0; i < n; ++i) {
-    size_t bit = n >> 1;
-    for (; j & bit; bit >>= 1) j ^= bit;
-    j ^= bit;
-    if (i < j) {
-      std::swap(re[i], re[j]);
-      std::swap(im[i], im[j]);
-    }
+// FFT in double (host), exponent sign -1, any smooth length, decimation in time by the smallest factor:
+// x[i * step], i < n, into out[0..n); w: the roots of unity of the whole length, n * wstep of them
+void host_fft(const std::complex<double>* x, size_t n, size_t step, std::complex<double>* out,
+              const std::vector<std::complex<double>>& w, size_t wstep) {
+  if (n == 1) {
+    out[0] = x[0];
+    return;
   }
-  for (size_t len = 2; len <= n; len <<= 1) {
-    const double ang = -2.0 * M_PI / (double)len;
-    for (size_t i = 0; i < n; i += len)
-      for (size_t k = 0; k < len / 2; ++k) {
-        const double wr = std::cos(ang * (double)k), wi = std::sin(ang * (double)k);
-        const size_t a = i + k, b = i + k + len / 2;
-        const double xr = re[b] * wr - im[b] * wi, xi = re[b] * wi + im[b] * wr;
-        re[b] = re[a] - xr;
-        im[b] = im[a] - xi;
-        re[a] += xr;
-        im[a] += xi;
-      }
+  size_t p = 2;
+  while (n % p) ++p;
+  const size_t m = n / p;
+  for (size_t q = 0; q < p; ++q) host_fft(x + q * step, m, step * p, out + q * m, w, wstep * p);
+  std::complex<double> t[16];
+  for (size_t k = 0; k < m; ++k) {
+    for (size_t q = 0; q < p; ++q) t[q] = out[q * m + k];
+    for (size_t h = 0; h < p; ++h) {
+      const size_t f = k + h * m;
+      std::complex<double> acc = t[0];
+      for (size_t q = 1; q < p; ++q) acc += w[(q * f % n) * wstep] * t[q];
+      out[f] = acc;
+    }
   }
 }
 
@@ -385,7 +321,7 @@ void host_fft_pow2(std::vector<double>& re, std::vector<double>& im) {
 
 bool gfft_smooth(int n) {
   if (n < 1) return false;
-  for (int r : {2, 3, 5, 7})
+  for (int r : {2, 3, 5, 7, 11, 13})
     while (n % r == 0) n /= r;
   return n == 1;
 }
@@ -397,8 +333,11 @@ hipError_t gaxis_build(GAxis& a, int n, std::vector<void*>& allocs) {
   if (gfft_smooth(n) && (n <= GFFT_LDS_MAX || split_four(n))) {
     a.L = n;
   } else {
-    long long m = 1;
-    while (m < 2LL * n - 1) m <<= 1;
+    long long m = bluestein_length(n);
+    if (!m) {
+      m = 1;
+      while (m < 2LL * n - 1) m <<= 1;
+    }
     if (m > (long long)GFFT_LDS_MAX * GFFT_LDS_MAX) return hipErrorInvalidValue;
     a.blu = true;
     a.L = (int)m;
@@ -426,26 +365,22 @@ hipError_t gaxis_build(GAxis& a, int n, std::vector<void*>& allocs) {
   // chirp c_d[t] = exp(-/+ i pi (t^2 mod 2n) / n); kernel b[m] = conj(c_d[|m|]) for |m| < n on the
   // circle of M points; bhat = FFT_M(b) / M
   const int M = a.L;
+  std::vector<std::complex<double>> c(n), b(M, 0.0), bf(M), w(M);
+  for (int t = 0; t < n; ++t) {
+    const long long q = ((long long)t * t) % (2LL * n);
+    c[t] = std::polar(1.0, -M_PI * (double)q / (double)n);
+    b[t] = std::conj(c[t]);
+    if (t > 0) b[M - t] = b[t];
+  }
+  for (int t = 0; t < M; ++t) w[t] = std::polar(1.0, -2.0 * M_PI * (double)t / (double)M);
+  host_fft(b.data(), M, 1, bf.data(), w, 1);
+  // the inverse direction's chirp and kernel are the conjugates, and as the kernel is even so is its spectrum
   for (int d = 0; d < 2; ++d) {
-    const double sg = d == 0 ? -1.0 : 1.0;
-    std::vector<float2> c(n);
-    std::vector<double> br(M, 0.0), bi(M, 0.0);
-    for (int t = 0; t < n; ++t) {
-      const long long q = ((long long)t * t) % (2LL * n);
-      const double ang = sg * M_PI * (double)q / (double)n;
-      const double cr = std::cos(ang), ci = std::sin(ang);
-      c[t] = make_float2((float)cr, (float)ci);
-      br[t] = cr;
-      bi[t] = -ci;
-      if (t > 0) {
-        br[M - t] = cr;
-        bi[M - t] = -ci;
-      }
-    }
-    host_fft_pow2(br, bi);
-    std::vector<float2> bh(M);
-    for (int k = 0; k < M; ++k) bh[k] = make_float2((float)(br[k] / M), (float)(bi[k] / M));
-    e = upload(c, &a.chirp[d], allocs);
+    const double sg = d == 0 ? 1.0 : -1.0;
+    std::vector<float2> ch(n), bh(M);
+    for (int t = 0; t < n; ++t) ch[t] = make_float2((float)c[t].real(), (float)(sg * c[t].imag()));
+    for (int k = 0; k < M; ++k) bh[k] = make_float2((float)(bf[k].real() / M), (float)(sg * bf[k].imag() / M));
+    e = upload(ch, &a.chirp[d], allocs);
     if (e == hipSuccess) e = upload(bh, &a.bhat[d], allocs);
     if (e != hipSuccess) return e;
   }
