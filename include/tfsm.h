@@ -217,6 +217,16 @@ int tfsm_forward(tfsm_plan* plan, const float* u, void* uh, int32_t nbatch, void
  * output path of OperatorLike.integrate, _base.py:751).  scratch >= tfsm_plan_inverse_scratch_bytes. */
 int tfsm_inverse(tfsm_plan* plan, const void* uh, float* u, int32_t nbatch, void* scratch, void* stream);
 
+/* 1 when tfsm_forward writes every element of its result, the padded columns (zeros) included; 0 when it
+ * leaves the padded columns as they are.  (No reference counterpart.) */
+int32_t tfsm_plan_forward_fills(const tfsm_plan* plan);
+
+/* u -> out = ifftn(E^nsteps fftn(u)).real for the plan's batch, real [B][C][N...] on both sides: a whole
+ * ETDRK0 integration (_etdrk.py:10-27 inside _base.py:676-751) without the state ever being returned.
+ * scratch: tfsm_plan_state_elems complex elements. */
+int tfsm_integrate_linear(tfsm_plan* plan, const float* u, float* out, int32_t nsteps, void* scratch,
+                          void* stream);
+
 /* Complex fields -> complex spectra (dir = -1, unnormalised) or back (dir = +1, scaled by
  * 1 / prod(N)) over the last D axes of contiguous [nbatch][C][N...] complex64 arrays; out may
  * equal in.  Replaces FourierMesh.fft / .ifft for complex input (mesh.py:481-491). */

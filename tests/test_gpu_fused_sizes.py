@@ -257,3 +257,48 @@ def test_1d_run_time_lengths(dev, n, batch):
                 ref = refpath.integrate(terms, mi, u[b:b + 1], dt, k, scheme=scheme)
                 assert _rel(plan.inverse(traj[b:b + 1, t].contiguous()), ref) <= TOL
             assert _rel(plan.inverse(uh[b:b + 1].contiguous()), ref) <= TOL
+
+
+@pytest.mark.parametrize("shape,batch,c", [((32,), 3, 1), ((100,), 1, 2), ((4096,), 2, 1), ((97,), 2, 1), ((16, 16), 2, 1), ((512, 48), 3, 2),
+                                           ((30, 42), 1, 1), ((64, 50), 2, 1), ((1024, 32), 1, 1), ((16, 32, 64), 2, 1), ((20, 16, 16), 1, 2)])
+def test_linear_integrate_from_field_to_field(dev, shape, batch, c):
+    """ETDRK0 from field to field (per-sample diffusion; a complex L with one channel) against the separate
+    transforms and steps of the same plan and against the oracle."""
+    from oracle import refpath
+    from torchfsm_amd.engine import SpectralPlan
+
+    g = torch.Generator(device=dev).manual_seed(sum(shape))
+    u = torch.randn(batch, c, *shape, generator=g, device=dev)
+    mi = [(0, 1.0, n) for n in shape]
+    nus = [1e-3 * (b + 1) for b in range(batch)]
+    lins = [[("lap", nus if batch > 1 else nus[0])]]
+    if c == 1:
+        # along the last axis: on another axis' Nyquist plane the half spectrum holds the Hermitian part
+        lins.append([(("deriv", len(shape) - 1, 1), -0.3), ("lap", 1e-3)])
+    for lin in lins:
+        plan = SpectralPlan(mi, batch, c, linear=lin, device=dev)
+        plan.set_scheme("ETDRK0", 0.1)
+        for steps in (0, 1, 3):
+            out = plan.integrate_linear(u, steps)
+            uh = plan.forward(u)
+            plan.step(uh, steps)
+            assert _rel(out, plan.inverse(uh)) <= 1e-6  # the same products, transforms of the same lengths
+            if steps == 0:
+                continue
+            for b in range(batch):
+                t = [(nus[b], "lap", None)] if len(lin) == 1 else [(-0.3, "deriv", (len(shape) - 1, 1)),
+                                                                              (1e-3, "lap", None)]
+                ref = refpath.integrate(t, mi, u[b:b + 1], 0.1, steps, scheme="ETDRK0")
+                assert _rel(out[b:b + 1], ref) <= TOL
+
+
+@pytest.mark.parametrize("shape", [(16,), (17,), (100,), (64, 48), (30, 34), (16, 16, 16), (6, 5, 4), (8, 8, 2)])
+def test_forward_leaves_zero_padding(dev, shape):
+    """The padded columns of a spectrum that forward() allocates are zero."""
+    from torchfsm_amd.engine import SpectralPlan
+
+    plan = SpectralPlan([(0, 1.0, n) for n in shape], 2, 1, device=dev)
+    junk = torch.full((2, 1) + shape[:-1] + (plan.pitch,), float("nan"), dtype=torch.complex64, device=dev)
+    del junk  # the allocator hands the same block out again
+    uh = plan.forward(torch.ones(2, 1, *shape, device=dev))
+    assert bool((uh[..., shape[-1] // 2 + 1:] == 0).all()) and bool(torch.isfinite(torch.view_as_real(uh)).all())

@@ -76,6 +76,8 @@ SIGNATURES = {
     "tfsm_plan_add_force": (ctypes.c_int, [VP, VP, I32, I32, ctypes.c_float, VP]),
     "tfsm_forward": (ctypes.c_int, [VP, VP, VP, I32, VP]),
     "tfsm_inverse": (ctypes.c_int, [VP, VP, VP, I32, VP, VP]),
+    "tfsm_plan_forward_fills": (I32, [VP]),
+    "tfsm_integrate_linear": (ctypes.c_int, [VP, VP, VP, I32, VP, VP]),
     "tfsm_c2c": (ctypes.c_int, [VP, VP, VP, I32, I32, VP]),
     "tfsm_half_to_full": (ctypes.c_int, [VP, VP, VP, I32, VP]),
     "tfsm_full_to_half": (ctypes.c_int, [VP, VP, VP, I32, VP]),

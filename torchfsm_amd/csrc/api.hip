@@ -1830,6 +1830,43 @@ int tfsm_inverse(tfsm_plan* p, const void* uh, float* u, int32_t nbatch, void* s
                            (hipStream_t)stream);
 }
 
+int32_t tfsm_plan_forward_fills(const tfsm_plan* p) { return p && fast_rows(p, p->D - 1) && p->P <= p->n[p->D - 1] ? 1 : 0; }
+
+int tfsm_integrate_linear(tfsm_plan* p, const float* u, float* out, int32_t nsteps, void* scratch, void* stream) {
+  if (!p || !u || !out || !scratch) return fail(TFSM_E_INVALID, "null argument");
+  if (p->scheme != ETDRK0) return fail(TFSM_E_STATE, "the exact linear stepper (ETDRK0) is not the plan's scheme");
+  if (nsteps < 0) return fail(TFSM_E_INVALID, "nsteps must be >= 0");
+  if (int rc = check_nbatch(p, p->B)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  float2* W = (float2*)scratch;
+  const int D = p->D, nl = p->n[D - 1];
+  const size_t blk = (size_t)p->B * p->C;
+  const float* E = p->coef + CS_E * p->modes;
+  const float2* Ec = p->cplx ? p->coefc + CS_E * p->modes : nullptr;
+  const float scale = (float)(1.0 / (double)plan_npts(p));
+  if (D == 1 && fast_rows(p, 0) && !p->per_len) {
+    HIP_TRY(launch_rows_linear(nl, u, out, (int)blk, scale, p->tw[0][0], E, Ec, p->coef_bstride(), p->C, nsteps, st),
+            "linear row launch");
+    return TFSM_OK;
+  }
+  if (D == 1 || !fast_cols(p, 0)) {  // the passes one by one
+    int rc = xf_forward_blocks(p, u, W, blk, st);
+    if (!rc) rc = step_impl(p, W, nsteps, nullptr, nullptr, 0, nullptr, st);
+    return rc ? rc : xf_inverse_blocks(p, W, W, out, blk, scale, st);
+  }
+  const size_t rows = blk * p->modes / p->P, plane = D == 3 ? (size_t)p->n[1] * p->P : (size_t)p->P;
+  HIP_TRY(xf_rows(p, GM_R2C, -1, u, (size_t)nl, W, (size_t)p->P, rows, 1.0f, st), "r2c launch");
+  if (D == 3)
+    HIP_TRY(xf_cols(p, 1, -1, W, W, blk * p->n[0], plane, (size_t)p->P, (size_t)p->H, st), "y fft launch");
+  HIP_TRY(launch_cols_linear(p->n[0], W, blk, p->modes, plane, D == 3 ? (int)plane : p->H, p->tw[0][0], E, Ec,
+                             p->coef_bstride(), p->C, nsteps, st),
+          "linear column launch");
+  if (D == 3)
+    HIP_TRY(xf_cols(p, 1, +1, W, W, blk * p->n[0], plane, (size_t)p->P, (size_t)p->H, st), "y ifft launch");
+  HIP_TRY(xf_rows(p, GM_C2R, +1, W, (size_t)p->P, out, (size_t)nl, rows, scale, st), "c2r launch");
+  return TFSM_OK;
+}
+
 int tfsm_c2c(tfsm_plan* p, const void* in, void* out, int32_t nbatch, int32_t dir, void* stream) {
   if (!p || !in || !out) return fail(TFSM_E_INVALID, "null argument");
   if (dir != -1 && dir != 1) return fail(TFSM_E_INVALID, "dir must be -1 or +1");

@@ -730,6 +730,12 @@ hipError_t launch_rows_c2c(int n, int dir, const float2* in, size_t in_ld, float
 hipError_t launch_cols_c2c(int n, int dir, const float2* in, float2* out, size_t nouter, size_t outer_stride,
                            size_t col_stride, int ninner, float scale, const float2* tw, hipStream_t st,
                            StepMask mask = StepMask(), int b0 = 0, size_t outer_per_sample = 1);
+// exact linear steps between the two directions of the last forward axis (2D / 3D columns; 1D: whole real rows)
+hipError_t launch_cols_linear(int n, float2* u, size_t nouter, size_t outer_stride, size_t col_stride, int ninner,
+                              const float2* tw, const float* E, const float2* Ec, size_t e_bstride, int C, int nsteps,
+                              hipStream_t st);
+hipError_t launch_rows_linear(int n, const float* in, float* out, int nrows, float scale, const float2* tw,
+                              const float* E, const float2* Ec, size_t e_bstride, int C, int nsteps, hipStream_t st);
 hipError_t launch_full_to_half(const float2* full, float2* half, const ConvArgs& a, hipStream_t st);
 hipError_t launch_half_to_full(const float2* half, float2* full, const ConvArgs& a, hipStream_t st);
 hipError_t launch_linear_steps(float2* U, const float* E, size_t coef_bstride, size_t modes, int C, size_t total,

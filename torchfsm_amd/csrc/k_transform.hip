@@ -6,7 +6,8 @@
 namespace tfsm {
 
 // ---------------------------------------------------------------- contiguous rows
-// real rows [nrows][in_ld] -> half spectrum rows [nrows][out_ld] (k = 0..N/2), times scale
+// real rows [nrows][in_ld] -> half spectrum rows [nrows][out_ld] (k = 0..N/2), times scale; the padded
+// columns up to the pitch out_ld become zero (as far as the row's N positions reach)
 template <int N, int ROWS>
 __global__ void __launch_bounds__(Fft<N>::NT* ROWS)
     k_rows_r2c(const float* __restrict__ in, size_t in_ld, float2* __restrict__ out, size_t out_ld, int nrows,
@@ -28,7 +29,8 @@ __global__ void __launch_bounds__(Fft<N>::NT* ROWS)
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
       const int pos = j + m * NT;
-      if (pos <= N / 2) out[(size_t)row * out_ld + pos] = make_float2(v[m].x * scale, v[m].y * scale);
+      if (pos < (int)out_ld)
+        out[(size_t)row * out_ld + pos] = pos <= N / 2 ? make_float2(v[m].x * scale, v[m].y * scale) : make_float2(0.f, 0.f);
     }
   }
 }
@@ -115,6 +117,87 @@ __global__ void __launch_bounds__(Fft<N>::NT* V)
 #pragma unroll
     for (int m = 0; m < RMAX; ++m)
       out[base + (size_t)(j + m * NT) * col_stride] = make_float2(v[m].x * scale, v[m].y * scale);
+  }
+}
+
+// U <- E^n U between the two directions of one axis, for the exact linear stepper (ETDRK0) of a call that
+// starts and ends in physical space: the last forward pass, the steps and the first inverse pass of a column
+// in one launch (heat equation 512^2, B = 16: forward 11.5, steps 13.3 and inverse 11.8 us as launches of their
+// own, 15.5 here; the whole call 61 -> 33 us).  The steps multiply one at a time, as k_linear_steps does.  EV: float (real L) or float2.
+__device__ __forceinline__ float2 lin_mul(float e, float2 u) { return rscale(e, u); }
+__device__ __forceinline__ float2 lin_mul(float2 e, float2 u) { return cmulr(e, u); }
+__device__ __forceinline__ float lin_conj(float e) { return e; }
+__device__ __forceinline__ float2 lin_conj(float2 e) { return make_float2(e.x, -e.y); }
+
+// strided columns (layout of k_cols_c2c), in place: block o = blockIdx.y belongs to sample (o0 + o) / C and its
+// element (p, i) is mode p * col_stride + i
+template <int N, int V, class EV>
+__global__ void __launch_bounds__(Fft<N>::NT* V)
+    k_cols_linear(float2* u, size_t outer_stride, size_t col_stride, int ninner, const float2* tw,
+                  const EV* __restrict__ E, size_t e_bstride, int C, unsigned o0, int nsteps) {
+  using F = Fft<N>;
+  constexpr int RMAX = F::RMAX, NT = F::NT;
+  __shared__ float2 s_tw[Fft<N>::tw_size()];
+  __shared__ float2 s_buf[LdsSize<N, V>::slots];
+  const int vi = threadIdx.x % V, j = threadIdx.x / V;
+  const int i = blockIdx.x * V + vi;
+  const bool iv = i < ninner;
+  float2* ub = u + (size_t)blockIdx.y * outer_stride + (iv ? i : 0);
+  const EV* Eb = E + (size_t)((o0 + blockIdx.y) / C) * e_bstride + (iv ? i : 0);
+  float2 v[RMAX];
+  EV e[RMAX];
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) v[m] = ub[(size_t)(j + m * NT) * col_stride];
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) e[m] = Eb[(size_t)(j + m * NT) * col_stride];
+  load_twiddles<N>(s_tw, tw);
+  __syncthreads();
+  fft_wg<N, -1, V>(v, s_buf, s_tw, j, vi);
+  for (int s = 0; s < nsteps; ++s)
+#pragma unroll
+    for (int m = 0; m < RMAX; ++m) v[m] = lin_mul(e[m], v[m]);
+  fft_wg<N, +1, V>(v, s_buf, s_tw, j, vi);
+  if (iv) {
+#pragma unroll
+    for (int m = 0; m < RMAX; ++m) ub[(size_t)(j + m * NT) * col_stride] = v[m];
+  }
+}
+
+// 1D: whole real rows, mode k of row r in row r / C of E; a mirrored position takes the conjugate factor
+template <int N, int ROWS, class EV>
+__global__ void __launch_bounds__(Fft<N>::NT* ROWS)
+    k_rows_linear(const float* __restrict__ in, float* __restrict__ out, int nrows, float scale, const float2* tw,
+                  const EV* __restrict__ E, size_t e_bstride, int C, int nsteps) {
+  using F = Fft<N>;
+  constexpr int RMAX = F::RMAX, NT = F::NT, SL = LdsSize<N, 1>::slots;
+  __shared__ float2 s_tw[Fft<N>::tw_size()];
+  __shared__ float2 s_buf[ROWS * SL];
+  const int g = threadIdx.x / NT, j = threadIdx.x % NT;
+  const int row = blockIdx.x * ROWS + g;
+  const bool rv = row < nrows;
+  const EV* Er = E + (size_t)((rv ? row : 0) / C) * e_bstride;
+  float2 v[RMAX];
+  EV e[RMAX];
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) {
+    const int pos = j + m * NT;
+    v[m] = make_float2(rv ? in[(size_t)row * N + pos] : 0.f, 0.f);
+    e[m] = pos > N / 2 ? lin_conj(Er[N - pos]) : Er[pos];
+  }
+  load_twiddles<N>(s_tw, tw);
+  __syncthreads();
+  fft_wg<N, -1, 1, 0, RowSync<N, 0>::WS>(v, s_buf + g * SL, s_tw, j, 0);
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) {
+    const int pos = j + m * NT;
+    for (int s = 0; s < nsteps; ++s) v[m] = lin_mul(e[m], v[m]);
+    if (pos == 0 || pos == N / 2) v[m].y = 0.f;
+  }
+  lds_sync<RowSync<N, 0>::WS>();
+  fft_wg<N, +1, 1, 0, RowSync<N, 0>::WS>(v, s_buf + g * SL, s_tw, j, 0);
+  if (rv) {
+#pragma unroll
+    for (int m = 0; m < RMAX; ++m) out[(size_t)row * N + j + m * NT] = v[m].x * scale;
   }
 }
 
@@ -609,6 +692,49 @@ hipError_t launch_cols_c2c(int n, int dir, const float2* in, float2* out, size_t
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
+  })
+}
+
+// the column passes around the exact linear steps (k_cols_linear); e_bstride in elements of E or Ec
+hipError_t launch_cols_linear(int n, float2* u, size_t nouter, size_t outer_stride, size_t col_stride, int ninner,
+                              const float2* tw, const float* E, const float2* Ec, size_t e_bstride, int C, int nsteps,
+                              hipStream_t st) {
+  if (nouter == 0 || ninner <= 0) return hipSuccess;
+  if (n > 512) return hipErrorInvalidValue;
+  TFSM_SWITCH_N(n, {
+    constexpr int V = (NN > 512) ? 1 : ((Fft<NN>::NT * 16 <= 1024) ? 16 : 8);
+    for (size_t o0 = 0; o0 < nouter; o0 += 65535) {
+      const size_t no = (nouter - o0) < 65535 ? (nouter - o0) : 65535;
+      const dim3 grid((ninner + V - 1) / V, (unsigned)no);
+      const dim3 block(Fft<NN>::NT * V);
+      float2* ub = u + o0 * outer_stride;
+      if (Ec)
+        hipLaunchKernelGGL((k_cols_linear<NN, V, float2>), grid, block, 0, st, ub, outer_stride, col_stride, ninner, tw,
+                           Ec, e_bstride, C, (unsigned)o0, nsteps);
+      else
+        hipLaunchKernelGGL((k_cols_linear<NN, V, float>), grid, block, 0, st, ub, outer_stride, col_stride, ninner, tw,
+                           E, e_bstride, C, (unsigned)o0, nsteps);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  })
+}
+
+hipError_t launch_rows_linear(int n, const float* in, float* out, int nrows, float scale, const float2* tw,
+                              const float* E, const float2* Ec, size_t e_bstride, int C, int nsteps, hipStream_t st) {
+  if (nrows <= 0) return hipSuccess;
+  TFSM_SWITCH_N(n, {
+    constexpr int R = rows_per_wg<NN>();
+    const dim3 grid((nrows + R - 1) / R);
+    const dim3 block(Fft<NN>::NT * R);
+    if (Ec)
+      hipLaunchKernelGGL((k_rows_linear<NN, R, float2>), grid, block, 0, st, in, out, nrows, scale, tw, Ec, e_bstride,
+                         C, nsteps);
+    else
+      hipLaunchKernelGGL((k_rows_linear<NN, R, float>), grid, block, 0, st, in, out, nrows, scale, tw, E, e_bstride, C,
+                         nsteps);
+    return hipGetLastError();
   })
 }
 

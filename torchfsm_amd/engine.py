@@ -126,6 +126,8 @@ class SpectralPlan:
         self.state_elems = int(lib.tfsm_plan_state_elems(self._plan))
         self.ws_bytes = int(lib.tfsm_plan_workspace_bytes(self._plan))
         self.spec_shape = (self.batch, self.channels) + self.n[:-1] + (self.pitch,)
+        # whether the forward transform writes the padded columns too (else they are cleared first)
+        self._forward_fills = bool(lib.tfsm_plan_forward_fills(self._plan))
         self._ws = None
         self.scheme = None
         self.dt = None
@@ -298,13 +300,18 @@ class SpectralPlan:
         return torch.zeros((nb, self.channels) + self.n[:-1] + (self.pitch,), dtype=torch.complex64,
                            device=self.device)
 
+    def _spectrum(self, nb: int) -> torch.Tensor:
+        """An uninitialised spectrum, for calls that write all of it."""
+        return torch.empty((nb, self.channels) + self.n[:-1] + (self.pitch,), dtype=torch.complex64, device=self.device)
+
     # ------------------------------------------------------------------ transforms
     def forward(self, u: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Real (nb, C, N...) float32 -> half spectrum (nb, C, ..., P)."""
         require_gpu_tensor(u, "forward input")
         u = u.to(torch.float32).contiguous()
         nb = self._check(u, (self.channels,) + self.n, torch.float32, "forward input")
-        out = self.empty_spectrum(nb) if out is None else out
+        if out is None:
+            out = self._spectrum(nb) if self._forward_fills else self.empty_spectrum(nb)
         self._check(out, self.spec_shape[1:], torch.complex64, "forward output", nb)
         with torch.cuda.device(self.device):
             check(lib.tfsm_forward(self._plan, _ptr(u), _ptr(out), int(nb), _stream(self.device)), "forward")
@@ -338,7 +345,7 @@ class SpectralPlan:
         require_gpu_tensor(full, "full spectrum")
         full = full.to(torch.complex64).contiguous()
         nb = self._check(full, (self.channels,) + self.n, torch.complex64, "full spectrum")
-        out = self.empty_spectrum(nb)
+        out = self._spectrum(nb)
         with torch.cuda.device(self.device):
             check(lib.tfsm_full_to_half(self._plan, _ptr(full), _ptr(out), int(nb), _stream(self.device)), "full_to_half")
         return out
@@ -389,6 +396,17 @@ class SpectralPlan:
             check(lib.tfsm_step(self._plan, _ptr(uh), int(nsteps), _ptr(rec_slot), _ptr(traj), T, _ptr(ws),
                                 _stream(self.device)), "step")
         return uh
+
+    def integrate_linear(self, u: torch.Tensor, nsteps: int) -> torch.Tensor:
+        """Real (B, C, N...) -> the real field after nsteps exact linear steps (tfsm_integrate_linear)."""
+        u = u.contiguous()
+        self._check(u, (self.channels,) + self.n, torch.float32, "u_0", self.batch)
+        out = torch.empty_like(u)
+        scratch = self._spectrum(self.batch)
+        with torch.cuda.device(self.device):
+            check(lib.tfsm_integrate_linear(self._plan, _ptr(u), _ptr(out), int(nsteps), _ptr(scratch),
+                                            _stream(self.device)), "integrate_linear")
+        return out
 
     def step_varying(self, uh: torch.Tensor, nsteps_per_sample: torch.Tensor, max_steps: int):
         """Advance sample b of uh by min(nsteps_per_sample[b], max_steps) steps (device int32 [B])."""

@@ -386,6 +386,10 @@ class OperatorLike(_MutableMixIn):
             return self._integrate_with_adjoint(u_0, u_0_fft, dt, step, trajectory_recorder, return_in_fourier)
         plan = self._prepare(x.shape[0], x.device, dt)
         try:
+            if (plan.scheme == "ETDRK0" and u_0_fft is None and trajectory_recorder is None and not progressive
+                    and not return_in_fourier and u_0.dtype == torch.float32):
+                # exact linear steps from field to field: the state is never needed
+                return plan.integrate_linear(u_0, max(step, 0))
             uh = self._to_half(plan, u_0, u_0_fft)
             if trajectory_recorder is None:
                 self._run_steps(plan, uh, step, progressive)
