@@ -137,7 +137,8 @@ int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int
  * streams for 512^2 VorticityConvection (16 samples, B >= 32), Convection and
  * NSPressureConvection (16 samples from B = 32, 8 at B = 16..31) and 256^2 VorticityConvection
  * and Convection (16 samples, B >= 32; four streams from B = 64); 3D: radix-4
- * z rows from 64 points, and for Convection and NSPressureConvection sub-batches of 2 on two
+ * z rows from 32 points, radix-4 columns where the longer of x and y has 32 points (64 for
+ * NSPressureConvection), and for Convection and NSPressureConvection sub-batches of 2 on two
  * streams at 128^3 with 4 or more samples and at 256^3 with 2 or more, on four streams at 64^3 with 8 or more).
  * (No reference counterpart: launch configuration.) */
 int tfsm_plan_get_tuning(const tfsm_plan* plan, int32_t* out);

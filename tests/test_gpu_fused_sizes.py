@@ -302,3 +302,31 @@ def test_forward_leaves_zero_padding(dev, shape):
     del junk  # the allocator hands the same block out again
     uh = plan.forward(torch.ones(2, 1, *shape, device=dev))
     assert bool((uh[..., shape[-1] // 2 + 1:] == 0).all()) and bool(torch.isfinite(torch.view_as_real(uh)).all())
+
+
+@pytest.mark.parametrize("kind", ["burgers", "nsp"])
+@pytest.mark.parametrize("shape,batch", [((32, 32, 32), 3), ((64, 64, 64), 2), ((64, 32, 16), 1), ((16, 64, 32), 2)])
+@pytest.mark.parametrize("scheme", ["SETDRK2", "SETDRK4"])
+def test_3d_small_mesh_defaults(dev, kind, shape, batch, scheme):
+    """The default plans of small 3D meshes, with content at every frequency and a source, against the
+    unfused path and the oracle."""
+    from oracle import refpath
+    from torchfsm_amd.engine import SpectralPlan
+
+    g = torch.Generator(device=dev).manual_seed(sum(shape))
+    u = 0.3 * torch.randn(batch, 3, *shape, generator=g, device=dev)
+    src = torch.randn(1, 3, *shape, generator=g, device=dev)
+    mi = [(0, 1.0, n) for n in shape]
+    name, coef = {"burgers": ("conv", -1.0), "nsp": ("nsp", 1.0)}[kind]
+    plan = SpectralPlan(mi, batch, 3, nonlinear=name, nonlinear_coef=coef, linear=[("lap", 0.01)], device=dev)
+    plan.add_source(src, 0.2)
+    plan.set_scheme(scheme, 1e-3)
+    uh = plan.forward(u)
+    plan.step(uh, 3)
+    out = plan.inverse(uh)
+    plan.set_general(True)
+    uh = plan.forward(u)
+    plan.step(uh, 3)
+    terms = [(0.01, "lap", None), (coef, name, None), (0.2, "src", src)]
+    ref = refpath.integrate(terms, mi, u, 1e-3, 3, scheme=scheme)
+    assert _rel(out, plan.inverse(uh)) <= TOL and _rel(out, ref) <= TOL

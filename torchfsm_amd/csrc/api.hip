@@ -1566,7 +1566,15 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
   // small square meshes step with the persistent per-sample kernel (one launch per call)
   if (!rc && D == 2 && p->fused_ok && run2d_supported(term, p->n[0], p->n[1], p->PF) && !p->cplx)
     p->persistent = true;
-  if (!rc && D == 3) p->row_var = (p->n[2] >= 64 && is_pow2(p->n[2])) ? 1 : 0;  // radix-4 z rows (fewer registers)
+  // 3D plans of 4 values per thread: z rows from 32 points; the columns of meshes up to 32 points along x and y,
+  // and up to 64 for NSPressureConvection (with its stage kernels), whose launches are as long as one thread's
+  // chain of transforms (SETDRK4, us per step: NSP 64^3 B = 2 224 -> 180, B = 16 947 -> 778, 32^3 B = 4 197 ->
+  // 130; Burgers 32^3 B = 4 194 -> 140; at 64^3 Burgers, and at 128 points, no gain)
+  if (!rc && D == 3 && is_pow2(p->n[0]) && is_pow2(p->n[1]) && is_pow2(p->n[2])) {
+    const int nxy = p->n[0] > p->n[1] ? p->n[0] : p->n[1];
+    p->row_var = p->n[2] >= 32 ? 1 : 0;
+    p->col_var = nxy == 32 || (nxy == 64 && term == TERM_NSP) ? 1 : 0;
+  }
   // 3D Convection and NSPressureConvection at 128^3 with 4 or more samples: sub-batches of 2 on two
   // streams, so one sub-batch's VALU-bound z-row pass overlaps the other's memory-bound column
   // passes (Burgers, B = 8: ETDRK2 1.52 -> 1.34 ms/step, SETDRK4 3.04 -> 2.71; NavierStokes SETDRK4,

@@ -475,19 +475,24 @@ __device__ __forceinline__ void nsp_project(float2 (&cv)[C], const float (&av)[C
 #pragma unroll
   for (int i = 1; i < C; ++i) lap = addr(lap, -mulr(av[i], av[i]));
   const float il = (lap == 0.f) ? 1.0f : __fdiv_rn(1.0f, lap);
-  float2 sum[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-  bool have[2] = {false, false};
+  // the sums over the Nyquist and the other axes, chosen by value (an array indexed by the flag would put
+  // both in scratch memory)
+  float2 s0 = make_float2(0.f, 0.f), s1 = s0;
+  bool h0 = false, h1 = false;
 #pragma unroll
   for (int i = 0; i < C; ++i) {
     const float2 t = make_float2(-mulr(av[i], cv[i].y), mulr(av[i], cv[i].x));
-    const int q = ny[i] ? 1 : 0;
-    sum[q] = have[q] ? radd(sum[q], t) : t;
-    have[q] = true;
+    const float2 n0 = h0 ? radd(s0, t) : t, n1 = h1 ? radd(s1, t) : t;
+    const bool q = ny[i];
+    s0 = make_float2(q ? s0.x : n0.x, q ? s0.y : n0.y);
+    s1 = make_float2(q ? n1.x : s1.x, q ? n1.y : s1.y);
+    h0 = h0 || !q;
+    h1 = h1 || q;
   }
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    const int q = ny[c] ? 1 : 0;
-    const float2 p = make_float2(mulr(il, sum[q].x), mulr(il, sum[q].y));
+    const float sx = ny[c] ? s1.x : s0.x, sy = ny[c] ? s1.y : s0.y;
+    const float2 p = make_float2(mulr(il, sx), mulr(il, sy));
     cv[c] = rsub(make_float2(-mulr(av[c], p.y), mulr(av[c], p.x)), cv[c]);
   }
 }

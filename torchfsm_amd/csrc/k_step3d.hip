@@ -412,12 +412,37 @@ __global__ void __launch_bounds__((Fft<N2, VAR>::NT * ROWS)) k3_row(Row3Args a) 
     default: return hipErrorInvalidValue;              \
   }
 
-// Convection column kernels also compiled per ETDRK2 / SETDRK2 and SETDRK4 stage (and for the
-// field pass of the initial state): the 64-, 128- and 256-point x columns with the default radix plan
-template <int NN, int VR>
+// Column kernels also compiled per ETDRK2 / SETDRK2 and SETDRK4 stage (and for the field pass of the
+// initial state): Convection at 64, 128 and 256 points with the default radix plan, and
+// NSPressureConvection at 32 and 64 points with the plan of 4 values per thread, its default there
+// (NSP 64^3 B = 2 SETDRK4: 224 us per step with 8 values and the run-time stage, 196 with 4, 180 with both)
+template <int NN, int VR, int TERM>
 struct Col3StageKernels {
-  static constexpr bool value = (NN == 64 || NN == 128 || NN == 256) && VR == var3(NN);
+  static constexpr bool value = (TERM == TERM_CONV && (NN == 64 || NN == 128 || NN == 256) && VR == var3(NN)) ||
+                                (TERM == TERM_NSP && (NN == 32 || NN == 64) && VR == 3);
 };
+
+template <int NN, int VR, int TERM>
+static hipError_t launch_col3d_term(const Col3Args& b, dim3 grid, dim3 block, int stage, hipStream_t st) {
+  constexpr int V = 16;
+#define TFSM_COL3_STAGE(S) \
+  case S: TFSM_LAUNCH((k3_col<NN, V, VR, TERM, S>), grid, block, 0, st, b, stage); return hipGetLastError();
+  if constexpr (Col3StageKernels<NN, VR, TERM>::value) {
+    switch (stage) {
+      TFSM_COL3_STAGE(ST_PRO)
+      TFSM_COL3_STAGE(ST_R2_E0)
+      TFSM_COL3_STAGE(ST_R2_E1)
+      TFSM_COL3_STAGE(ST_R4_E0)
+      TFSM_COL3_STAGE(ST_R4_E1)
+      TFSM_COL3_STAGE(ST_R4_E2)
+      TFSM_COL3_STAGE(ST_R4_E3)
+      default: break;
+    }
+  }
+#undef TFSM_COL3_STAGE
+  TFSM_LAUNCH((k3_col<NN, V, VR, TERM>), grid, block, 0, st, b, stage);
+  return hipGetLastError();
+}
 
 template <int NN, int VR>
 static hipError_t launch_col3d_t(const Col3Args& a, int nb, int stage, hipStream_t st) {
@@ -426,26 +451,10 @@ static hipError_t launch_col3d_t(const Col3Args& a, int nb, int stage, hipStream
   const int slots = (ntiles + 7) / 8;
   Col3Args b = a;
   b.nb = nb;
-  if (a.term == TERM_NSP)
-    TFSM_LAUNCH((k3_col<NN, V, VR, TERM_NSP>), dim3(slots * 8 * nb), dim3(Fft<NN, VR>::NT * V), 0, st, b, stage);
-  else if (a.term == TERM_KS)
-    TFSM_LAUNCH((k3_col<NN, V, VR, TERM_KS>), dim3(slots * 8 * nb), dim3(Fft<NN, VR>::NT * V), 0, st, b, stage);
-  else if constexpr (Col3StageKernels<NN, VR>::value) {
-    const dim3 grid(slots * 8 * nb), block(Fft<NN, VR>::NT * V);
-    switch (stage) {
-      case ST_PRO: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_PRO>), grid, block, 0, st, b, stage); break;
-      case ST_R2_E0: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R2_E0>), grid, block, 0, st, b, stage); break;
-      case ST_R2_E1: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R2_E1>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E0: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R4_E0>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E1: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R4_E1>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E2: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R4_E2>), grid, block, 0, st, b, stage); break;
-      case ST_R4_E3: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV, ST_R4_E3>), grid, block, 0, st, b, stage); break;
-      default: TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV>), grid, block, 0, st, b, stage);
-    }
-  } else
-    TFSM_LAUNCH((k3_col<NN, V, VR, TERM_CONV>), dim3(slots * 8 * nb), dim3(Fft<NN, VR>::NT * V), 0, st, b,
-                       stage);
-  return hipGetLastError();
+  const dim3 grid(slots * 8 * nb), block(Fft<NN, VR>::NT * V);
+  if (a.term == TERM_NSP) return launch_col3d_term<NN, VR, TERM_NSP>(b, grid, block, stage, st);
+  if (a.term == TERM_KS) return launch_col3d_term<NN, VR, TERM_KS>(b, grid, block, stage, st);
+  return launch_col3d_term<NN, VR, TERM_CONV>(b, grid, block, stage, st);
 }
 
 template <int NN, int VR>
