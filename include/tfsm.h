@@ -133,13 +133,12 @@ int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int
 /* Current launch shape: out[6] = column tile, column variant, row variant, row workgroup,
  * sub-batch, streams.  A new plan starts from a default derived from its shape (2D: column tile
  * and radix variant per axis size and product term, 64-thread row groups where there are few
- * rows of 64 to 256 points, sub-batch sized to keep >= 512 column workgroups per launch, and sub-batches on two
- * streams for 512^2 VorticityConvection (16 samples, B >= 32), Convection and
- * NSPressureConvection (16 samples from B = 32, 8 at B = 16..31) and 256^2 VorticityConvection
- * and Convection (16 samples, B >= 32; four streams from B = 64); 3D: radix-4
- * z rows from 32 points, radix-4 columns where the longer of x and y has 32 points (64 for
- * NSPressureConvection), and for Convection and NSPressureConvection sub-batches of 2 on two
- * streams at 128^3 with 4 or more samples and at 256^3 with 2 or more, on four streams at 64^3 with 8 or more).
+ * rows of 64 to 256 points, and from 2^21 points per batch sub-batches of about that many points on
+ * two streams, with other lines for 256^2, 512- and 1024-point columns; 3D: radix-4 z rows from 32
+ * points, radix-4 columns where the longer of x and y has 32 points (64 for NSPressureConvection),
+ * and for Convection and NSPressureConvection sub-batches on two streams: one sample each for meshes of
+ * 800k points or more (2 at 128^3 with 4 or more samples), halves of the batch for meshes of 100k
+ * points or more with 800k points per batch, and pairs on four streams at 64^3 with 8 or more samples).
  * (No reference counterpart: launch configuration.) */
 int tfsm_plan_get_tuning(const tfsm_plan* plan, int32_t* out);
 

@@ -330,3 +330,38 @@ def test_3d_small_mesh_defaults(dev, kind, shape, batch, scheme):
     terms = [(0.01, "lap", None), (coef, name, None), (0.2, "src", src)]
     ref = refpath.integrate(terms, mi, u, 1e-3, 3, scheme=scheme)
     assert _rel(out, plan.inverse(uh)) <= TOL and _rel(out, ref) <= TOL
+
+
+@pytest.mark.parametrize("term,shape,B,sb,ns", [("vc", (128, 128), 129, 65, 2), ("conv", (200, 200), 53, 27, 2),
+                                                ("nsp", (256, 256), 33, 17, 2), ("nsp", (512, 512), 9, 5, 2),
+                                                ("conv", (48, 48, 48), 9, 5, 2), ("nsp", (96, 96, 96), 3, 1, 2)])
+def test_default_sub_batches_equal_whole_batch(dev, term, shape, B, sb, ns):
+    """The default sub-batches on two streams, with a shorter last one, against one launch over the whole
+    batch: the same kernels, so equal bit for bit; the last sample against a plan of one sample (other
+    launch shapes at most) within the float32 bar."""
+    from torchfsm_amd.engine import SpectralPlan
+
+    D = len(shape)
+    C = 1 if term == "vc" else D
+    g = torch.Generator(device=dev).manual_seed(B)
+    u = 0.3 * torch.randn(B, C, *shape, generator=g, device=dev)
+
+    def plan_of(batch):
+        p = SpectralPlan([(0, 1.0, n) for n in shape], batch, C, nonlinear=term, nonlinear_coef=-1.0,
+                         linear=[("lap", 0.01)], device=dev)
+        p.set_scheme("SETDRK4", 1e-3)
+        return p
+
+    plan = plan_of(B)
+    assert plan.tuning[4] == sb and plan.streams == ns and not plan.general
+    uh = plan.forward(u)
+    plan.step(uh, 3)
+    plan.set_tuning(*plan.tuning[:4], 0)
+    plan.set_streams(1)
+    uw = plan.forward(u)
+    plan.step(uw, 3)
+    assert torch.equal(uh, uw)
+    one = plan_of(1)
+    u1 = one.forward(u[B - 1:].contiguous())
+    one.step(u1, 3)
+    assert _rel(plan.inverse(uh)[B - 1:], one.inverse(u1)) <= TOL

@@ -1504,13 +1504,8 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     if (p->general) rc = plan_genfused(p);
     if (!rc && p->general) gen_layout(p);
   }
-  // default launch shape (the autotuner may refine it): 2D columns of 512 points run the
-  // half-thread radix plan for one-channel products (the two-channel ones keep a second column in
-  // registers and run faster with 8 values per thread); temporal blocking uses the smallest
-  // sub-batch (multiple of 8) that still gives >= 512 column workgroups (two per CU) while its
-  // working set stays under 256 MB
+  // default launch shape (the autotuner may refine it)
   if (!rc && D == 2 && (p->fused_ok || p->genf)) {
-    const bool one_channel = term == TERM_VC || term == TERM_KS;
     const int n0 = p->n[0], n1 = p->n[1];
     // measured per axis size: 512 keeps 16-column tiles; 64, 128 and 256 run 8-column tiles and rows of 4
     // values per thread.  Their launches are one round of workgroups, as long as one thread's chain of
@@ -1532,35 +1527,40 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
       // few rows: one-wavefront workgroups spread over more CUs (128^2 B = 1 63.9 -> 61.5; B = 16 the reverse)
       if ((size_t)p->B * n0 <= 512) p->row_wg = 64;
     }
-    const size_t per_sample = 4 * (size_t)p->C * p->modes * sizeof(float2) +
-                              (size_t)p->NF * p->n[0] * p->PF * sizeof(float2);
-    const int tiles = (p->H + p->V - 1) / p->V;
-    int sb = 8;
-    while (sb < p->B && (size_t)tiles * sb < 512) sb += 8;
-    if (sb >= p->B || (size_t)sb * per_sample > ((size_t)256 << 20) || p->ks_mean || p->genf) sb = 0;
-    p->sub_batch = sb;
-    // 512-point one-channel columns (VorticityConvection) with 32 or more samples: sub-batches of 16
-    // on two streams, so one sub-batch's VALU-bound row pass overlaps the other's memory-bound
-    // column pass (NS 512^2, B = 64: 0.630 ms/step against 0.662 for one stream and 32-sample
-    // sub-batches, and 0.676 for the 16-values-per-thread columns it replaces)
-    if (n0 == 512 && term == TERM_VC && p->B >= 32 && !p->genf) {
-      p->sub_batch = 16;
-      rc = tfsm_plan_set_streams(p, 2);
+    // Sub-batches of about 2M points on two streams, from 2M points per batch: the tail of one sub-batch's
+    // launch overlaps the other's next pass and its arrays stay in the cache.  On one stream they only
+    // shorten the launches (SETDRK4, us per step, one stream / whole batch / two streams: vorticity 128^2
+    // B = 256 382 / 184 / 157, 100^2 B = 256 401 / 229 / 228; Burgers 128^2 B = 256 378 / 263 / 221;
+    // NavierStokes 256^2 B = 64 338 / 286 / 255).  Other lines where sweeps drew them:
+    const bool pair = term == TERM_CONV || term == TERM_NSP;
+    const size_t pts = (size_t)p->B * n0 * n1, sub_pts = (size_t)1 << 21;
+    int sub = 0, ns = 2;
+    if (pts >= sub_pts) {
+      const int parts = pts / sub_pts > 2 ? (int)(pts / sub_pts) : 2;
+      sub = (p->B + parts - 1) / parts;
     }
-    // the same overlap for the other square shape classes where sweeps showed it (SETDRK4, 200
-    // steps): 512^2 Convection and NSPressureConvection on two streams, sub-batches of 16 from
-    // B = 32 (0.606 -> 0.544 and 0.734 -> 0.682 ms/step), of 8 at B = 16..31 (Convection 0.285 ->
-    // 0.248); 256^2 VorticityConvection and Convection in 16-sample sub-batches, on two streams
-    // from B = 32 (0.130 -> 0.119, 0.169 -> 0.157) and on four from B = 64 (0.259 -> 0.164, 0.337
-    // -> 0.213)
-    const bool square = p->n[0] == p->n[1] && !p->genf;
-    if (!rc && square && n0 == 512 && (term == TERM_CONV || term == TERM_NSP) && p->B >= 16) {
-      p->sub_batch = p->B >= 32 ? 16 : 8;
-      rc = tfsm_plan_set_streams(p, 2);
+    // 512-point one-channel columns: 16 samples (512^2 B = 64: 603 us, against 651 for 32 and 666 for 32 on one
+    // stream; B = 16 as a whole 178, in halves 186); two-channel ones: 16 from B = 32
+    if (n0 == 512 && !pair) sub = p->B >= 32 ? 16 : 0;
+    if (n0 == 512 && pair && p->B >= 32) sub = 16;
+    // 1024-point columns: two-channel products by 4 from B = 8 (Burgers ETDRK2 342 -> 313 us; one channel, or
+    // fewer samples, no gain)
+    if (n0 == 1024) sub = pair && p->B >= 8 ? 4 : 0;
+    // 256^2 up to 95 samples: 16 samples on two streams, on four from B = 48 (Burgers B = 48: 233 -> 180 us)
+    if (n0 == 256 && n1 == 256 && term != TERM_NSP && p->B >= 32 && p->B < 96) {
+      sub = 16;
+      ns = p->B >= 48 ? 4 : 2;
     }
-    if (!rc && square && n0 == 256 && (term == TERM_VC || term == TERM_CONV) && p->B >= 32) {
-      p->sub_batch = 16;
-      rc = tfsm_plan_set_streams(p, p->B >= 64 ? 4 : 2);
+    if (sub > 0 && sub < p->B && !p->ks_mean && !p->genf) {
+      p->sub_batch = sub;
+      rc = tfsm_plan_set_streams(p, ns);
+    }
+    // 512-point two-channel columns: 8 columns per tile where a launch has few tiles (Burgers B = 16 in
+    // sub-batches of 8, 4 values more per thread: 272 -> 236 us; NavierStokes, every batch: B = 4 138 -> 128,
+    // B = 32 596 -> 578)
+    if (n0 == 512 && (term == TERM_NSP || (term == TERM_CONV && p->B >= 16 && p->B < 32))) {
+      p->V = 8;
+      p->col_var = term == TERM_CONV ? 1 : 0;
     }
   }
   // small square meshes step with the persistent per-sample kernel (one launch per call)
@@ -1575,27 +1575,27 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     p->row_var = p->n[2] >= 32 ? 1 : 0;
     p->col_var = nxy == 32 || (nxy == 64 && term == TERM_NSP) ? 1 : 0;
   }
-  // 3D Convection and NSPressureConvection at 128^3 with 4 or more samples: sub-batches of 2 on two
-  // streams, so one sub-batch's VALU-bound z-row pass overlaps the other's memory-bound column
-  // passes (Burgers, B = 8: ETDRK2 1.52 -> 1.34 ms/step, SETDRK4 3.04 -> 2.71; NavierStokes SETDRK4,
-  // B = 4: 1.74 -> 1.66)
+  // 3D Convection and NSPressureConvection: sub-batches on several streams, so that one's VALU-bound z-row pass
+  // overlaps another's memory-bound column passes and their launches' tails (whole batch -> sub-batches, us
+  // per step).  Meshes of 800k points or more: one sample each on two streams (96^3 B = 4 NavierStokes 1248
+  // -> 1052, 100^3 B = 2 1304 -> 935, 128^3 B = 2 Burgers ETDRK2 363 -> 331), pairs at 128^3 from B = 4.
+  // Smaller ones, down to 100k points, from 800k points per batch: two halves (48^3 B = 8 NavierStokes 410 ->
+  // 296, 64^3 B = 4 247 -> 239; 32^3 loses at every batch), pairs on four streams at 64^3 from B = 8.
   const bool conv3 = D == 3 && p->fused_ok && (term == TERM_CONV || term == TERM_NSP);
-  if (!rc && conv3 && p->n[0] == 128 && p->n[1] == 128 && p->n[2] == 128 && p->B >= 4) {
-    p->sub_batch = 2;
-    rc = tfsm_plan_set_streams(p, 2);
-  }
-  // 256^3 with 2 or more samples: one sample per sub-batch on two streams, for the same overlap
-  // (Burgers ETDRK2, B = 2: 3.20 -> 3.10 ms/step)
-  if (!rc && conv3 && p->n[0] == 256 && p->n[1] == 256 && p->n[2] == 256 && p->B >= 2) {
-    p->sub_batch = 1;
-    rc = tfsm_plan_set_streams(p, 2);
-  }
-  // 64^3 with 8 or more samples: sub-batches of 2 on four streams (a 2-sample pass is too short to
-  // fill the GPU alone; four in flight do): Burgers SETDRK4, B = 8: 0.41 -> 0.37 ms/step, B = 16:
-  // 0.93 -> 0.78; NavierStokes SETDRK4, B = 16: 1.09 -> 0.91
-  if (!rc && conv3 && p->n[0] == 64 && p->n[1] == 64 && p->n[2] == 64 && p->B >= 8) {
-    p->sub_batch = 2;
-    rc = tfsm_plan_set_streams(p, 4);
+  if (!rc && conv3 && p->B >= 2) {
+    const size_t npts = (size_t)p->n[0] * p->n[1] * p->n[2], pts = npts * p->B;
+    int sub = 0, ns = 2;
+    if (npts >= 800000) sub = 1;
+    else if (npts >= 100000 && pts >= 800000) sub = (p->B + 1) / 2;
+    if (p->n[0] == 128 && p->n[1] == 128 && p->n[2] == 128 && p->B >= 4) sub = 2;
+    if (p->n[0] == 64 && p->n[1] == 64 && p->n[2] == 64 && p->B >= 8) {
+      sub = 2;
+      ns = 4;
+    }
+    if (sub > 0) {
+      p->sub_batch = sub;
+      rc = tfsm_plan_set_streams(p, ns);
+    }
   }
   if (rc) {
     tfsm_plan_destroy(p);

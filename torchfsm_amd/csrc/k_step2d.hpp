@@ -138,23 +138,21 @@ struct LdsFill {
 };
 
 // Velocity-form Navier-Stokes (NSPressureConvection): both channels' convection spectra are
-// transformed first, projected mode by mode (nsp_project), then combined channel by channel.
+// transformed first, projected mode by mode (nsp_project), then channel ch is combined.
 template <int N0, int V, int VAR, bool PP = false>
-__device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, float2 (&s)[2][Fft<N0, VAR>::RMAX],
+__device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, float2 (&s)[1][Fft<N0, VAR>::RMAX],
                                                 float2* s_buf, const float2* s_tw, int b, int ky, bool colv, int j,
-                                                int vi) {
+                                                int vi, int ch) {
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
   const size_t plane = (size_t)N0 * a.P1;
   const float2 z = make_float2(0.f, 0.f);
   if (stage == ST_PRO) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int m = 0; m < RMAX; ++m) {
-        const float2 t = a.U[((size_t)b * 2 + c) * plane + (size_t)(j + m * NT) * a.P1 + ky];
-        s[c][m] = colv ? t : z;
-      }
+    for (int m = 0; m < RMAX; ++m) {
+      const float2 t = a.U[((size_t)b * 2 + ch) * plane + (size_t)(j + m * NT) * a.P1 + ky];
+      s[0][m] = colv ? t : z;
+    }
     return;
   }
   // per-column values the projection and the combine need, loaded before the transforms
@@ -180,33 +178,33 @@ __device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, fl
     const bool nyx = 2 * x == N0, own = (x == 0 || nyx) && (zy || nyy);
     const bool ny[2] = {nyx && !own, nyy && !own};
     nsp_project<2>(cv, av, ny);
-    v[0][m] = cv[0];
-    v[1][m] = cv[1];
+    v[0][m] = ch ? cv[1] : cv[0];
   }
   const float4* cpk = a.cpk + (size_t)b * a.cpk_bstride;
   const size_t tb = (size_t)b * (a.cpk_bstride / 2);
   const float* c5b = a.c5t + tb;
   // cpk_index(ci, half) = 2 ci + cko: every mode of this lane has ci & 15 == ky & 15
   const int cko = (stage_coef_half(stage) << 4) - (ky & 15);
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride : nullptr;
-    combine_column2<N0, VAR, (RMAX > 4 ? 1 : 4)>(a, stage, ((size_t)b * 2 + c) * plane, src, cpk, c5b, tb, cko, ky,
-                                                 colv, j, v[c], s[c], rs);
-  }
+  const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)ch * a.src_cstride : nullptr;
+  combine_column2<N0, VAR, (RMAX > 4 ? 1 : 4)>(a, stage, ((size_t)b * 2 + ch) * plane, src, cpk, c5b, tb, cko, ky,
+                                               colv, j, v[0], s[0], rs);
 }
 
 // Stage combine, fields and inverse x-transforms of column tile `tile` of sample b: the body of
 // k2_col (and of the column pass of k2_run).  ST >= 0: the stage is a compile-time constant.
 // FILL: the caller has issued the LDS twiddle and wavenumber loads (fill) and this function writes
 // them to LDS, with a barrier, right before its first LDS use; otherwise they are in LDS already.
-template <int N0, int V, int TERM, int VAR, int ST, bool CLAMP = false, bool FILL = false, bool PP = false>
+// CH: only channel ch (products whose channels meet in the row kernel alone: Convection).
+template <int N0, int V, int TERM, int VAR, int ST, bool CLAMP = false, bool FILL = false, bool PP = false,
+          bool CH = false>
 __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile, int b, float2* s_buf,
                                           float2* s_tw, float* s_ax, int j, int vi,
-                                          const LdsFill<N0, VAR, Fft<N0, VAR>::NT * V>* fill = nullptr) {
+                                          const LdsFill<N0, VAR, Fft<N0, VAR>::NT * V>* fill = nullptr, int ch = 0) {
+  static_assert(CH ? (TERM == TERM_CONV || TERM == TERM_NSP) : TERM != TERM_NSP, "channel by channel");
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
-  constexpr int NC = Term2<TERM>::NC, NF = Term2<TERM>::NF;
+  constexpr int NCT = Term2<TERM>::NC, NFT = Term2<TERM>::NF;            // channels and fields of the product
+  constexpr int NC = CH ? 1 : NCT, NF = CH ? NFT / NCT : NFT;            // those of this call
   const int ky = tile * V + vi;
   const bool colv = ky < a.H1;
   // the column the lane's loads address: its own, or (CLAMP, tiles wider than the pitch P1) the last
@@ -234,12 +232,12 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
   float2 s[NC][RMAX];
   if constexpr (TERM == TERM_NSP) {
     fill_lds();
-    col_nsp_combine<N0, V, VAR, PP>(a, stage, s, s_buf, s_tw, b, ky, colv, j, vi);
+    col_nsp_combine<N0, V, VAR, PP>(a, stage, s, s_buf, s_tw, b, ky, colv, j, vi, ch);
   } else {
   if constexpr (TERM == TERM_CONS) fill_lds();
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const size_t base = ((size_t)b * NC + c) * plane;
+    const size_t base = ((size_t)b * NCT + (CH ? ch : c)) * plane;
     if (stage == ST_PRO) {
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) {
@@ -317,7 +315,7 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
         // remove_mean: fft(p - mean(p)) differs from fft(p) only at k = 0, by the batch mean of the DC
         if (a.dc && ky == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
       }
-      const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride : nullptr;
+      const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)(CH ? ch : c) * a.src_cstride : nullptr;
       combine_column2<N0, VAR, (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : 4, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
                                                                                   cko, kl, colv, j, v, s[c], rs,
                                                                                   &pre);
@@ -361,7 +359,7 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
     }
     col_fft<N0, +1, V, VAR, PP>(v, s_buf, s_tw, j, vi);
     if (ky <= a.kmax1) {  // kept columns only: the row kernel reads no other
-      float2* g = a.G + (((size_t)b * NF + f) * N0) * a.PF + ky;
+      float2* g = a.G + (((size_t)b * NFT + (CH ? ch * NF : 0) + f) * N0) * a.PF + ky;
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.PF] = v[m];
     }
@@ -369,6 +367,18 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
 }
 
 
+
+// Channels of a product taken by different workgroups of the column kernel: those of Convection, whose
+// combine and fields need one channel only, and of NSPressureConvection, where each of the two
+// transforms and projects both channels' products and combines its own (8 transforms instead of 6,
+// but 4 one after the other).  A launch was one or two rounds of workgroups, as long as one thread's
+// six transforms, with both channels' values in its registers (SETDRK4, us per step: Burgers 128^2
+// B = 16 70 -> 55, 512^2 B = 1 146 -> 97, 1024^2 B = 4 455 -> 357; NavierStokes 200^2 B = 16 266 -> 197,
+// 512^2 B = 4 192 -> 128, 1024^2 B = 8 898 -> 739 with its sub-batches)
+template <int TERM>
+struct ColChannels {
+  static constexpr int value = TERM == TERM_CONV || TERM == TERM_NSP ? Term2<TERM>::NC : 1;
+};
 
 // ST >= 0: the stage is a compile-time constant (only that stage's combine is compiled, which keeps
 // the code a launch executes small); ST = -1: the stage comes at run time.
@@ -393,19 +403,23 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_col(Col2Args a, int
   // (A tile-major order, each XCD taking an eighth of the tiles for all samples so that every
   // coefficient tile is fetched by one or two XCDs only, made the 512-point columns 35 % slower: at
   // any moment every CU then reads the same band of columns, at one stride across the rows.)
+  // Convection and NSPressureConvection: a workgroup takes one channel (ColChannels), and "sample" is a (sample, channel) pair.
   const int ntiles = (a.H1 + V - 1) / V;
+  constexpr int CW = ColChannels<TERM>::value;
+  const int np = a.nb * CW;
   int tile, bl;
-  if ((a.nb & 7) == 0) {
-    const int x = blockIdx.x & 7, sidx = blockIdx.x >> 3, g = a.nb >> 3;
+  if ((np & 7) == 0) {
+    const int x = blockIdx.x & 7, sidx = blockIdx.x >> 3, g = np >> 3;
     tile = sidx / g;
     bl = x * g + sidx % g;
   } else {
     tile = blockIdx.x % ntiles;
     bl = blockIdx.x / ntiles;
   }
-  const int b = a.b0 + bl;
+  const int b = a.b0 + bl / CW;
   if (a.mask.skip(b)) return;  // uniform per workgroup: this sample's steps are done
-  col2_tile<N0, V, TERM, VAR, ST, false, true, PP>(a, stage, tile, b, s_buf, s_tw, s_ax, j, vi, &fill);
+  col2_tile<N0, V, TERM, VAR, ST, false, true, PP, (CW > 1)>(a, stage, tile, b, s_buf, s_tw, s_ax, j, vi, &fill,
+                                                             bl % CW);
 }
 
 // Row x of sample b (rv false: idle row that only takes part in the transforms' synchronisation):
@@ -806,7 +820,7 @@ inline hipError_t launch_col_t(const Col2Args& a, int nb, int stage, hipStream_t
   const int tiles = (a.H1 + V - 1) / V;
   Col2Args b = a;
   b.nb = nb;
-  const dim3 grid(tiles * nb), block(Fft<N0, VAR>::NT * V);
+  const dim3 grid(tiles * nb * ColChannels<TERM>::value), block(Fft<N0, VAR>::NT * V);
 #define TFSM_COL_STAGE(S) \
   case S: TFSM_LAUNCH((k2_col<N0, V, TERM, VAR, S>), grid, block, 0, st, b, stage); return hipGetLastError();
   if constexpr (ColStageKernels<N0, V, TERM, VAR>::value) {

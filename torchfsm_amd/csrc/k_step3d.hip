@@ -74,6 +74,21 @@ __device__ __forceinline__ void col3_fields(const Col3Args& a, const float2 (&s)
   }
 }
 
+// Channels NC of a product and the workgroups that share them in the x column kernel.  The combine and
+// the fields of a channel need that channel only, so each takes one; for NSPressureConvection each of
+// them transforms and projects all three products (15 transforms instead of 9, but 5 one after the
+// other and a third of the values live), except on 256-point axes, whose launches fill the chip
+// anyway (256^3 SETDRK4 3.29 ms per step against 3.83).  As one workgroup per tile a launch was as
+// long as all three channels' chains (us per step, with the y-inverse pass's split: Burgers ETDRK2
+// 32^3 B = 4 71 -> 50, 64^3 B = 2 95 -> 74, 256^3 1614 -> 1451; NavierStokes SETDRK4 32^3 B = 1 118 -> 89,
+// 128^3 470 -> 399; a loop over a run-time range of channels instead of one keeps three channels'
+// addresses: 172 VGPRs against 90, slower everywhere)
+template <int TERM, int N0>
+struct Col3Channels {
+  static constexpr int NC = TERM == TERM_KS ? 1 : 3;
+  static constexpr int groups = TERM == TERM_NSP && N0 >= 256 ? 1 : NC;
+};
+
 // ST >= 0: the stage is a compile-time constant (only that stage's combine is compiled, which
 // lowers the register count: 128-point Convection columns 193 -> 133 / 148 VGPRs for ETDRK2's
 // evaluations, three waves per SIMD instead of two); ST = -1: the stage comes at run time.
@@ -90,15 +105,16 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k3_col(Col3Args a, int
   for (int i = threadIdx.x; i < N0; i += NT * V) s_ax[i] = a.ax[i];
   __syncthreads();
   const int vi = threadIdx.x % V, j = threadIdx.x / V;
-  // tiles (ky, kz-tile) go round-robin to the XCDs (block v on XCD v % 8); the nb samples of one
-  // tile run back to back on the same XCD, so each coefficient tile is fetched once per launch
+  // tiles (ky, kz-tile) go round-robin to the XCDs (block v on XCD v % 8); the nb samples' workgroups of
+  // one tile run back to back on the same XCD, so each coefficient tile is fetched once per launch
+  constexpr int NC3 = Col3Channels<TERM, N0>::NC, NW = Col3Channels<TERM, N0>::groups;
   const int nzt = a.P2 / V;
   const int ntiles = a.N1 * nzt;
   const int x8 = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int tile = x8 + 8 * (slot / a.nb);
-  const int bl = slot % a.nb;
+  const int tile = x8 + 8 * (slot / (a.nb * NW));
+  const int bl = slot % (a.nb * NW);
   if (tile >= ntiles) return;
-  const int b = a.b0 + bl;
+  const int b = a.b0 + bl / NW, c0 = bl % NW;  // first (NW = NC3: only) channel
   if (a.mask.skip(b)) return;
   const int ky = tile / nzt;
   const int kz = (tile % nzt) * V + vi;
@@ -110,97 +126,71 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k3_col(Col3Args a, int
   const size_t tb = (size_t)b * (a.cpk_bstride / 2);  // per-mode tables (c5t, ck01, c6t) of this sample
   // cpk_index(coff + xo, half) = 2 (coff + xo) + cko: (coff + xo) & 15 == kz & 15
   const int cko = (stage_coef_half(stage) << 4) - (kz & 15);
-  constexpr int NC3 = TERM == TERM_KS ? 1 : 3;  // channels
-  // combine batch (modes whose operands are loaded together): fewer than in 2D, the NSP kernel keeps
-  // all three channels' values live
+  // combine batch (modes whose operands are loaded together): fewer than in 2D
   constexpr int CBM = RMAX >= 16 ? 1 : (RMAX >= 8 ? 2 : 4);
   const int kyc = ky_compress(ky, a.N1, a.kmax1);
   const bool kept = kyc >= 0 && (tile % nzt) * V <= a.kmax2;  // uniform: the tile has kept columns
-  if constexpr (TERM == TERM_NSP) {
-    float2 s[3][RMAX];
-    if (stage == ST_PRO) {
+  auto combine = [&](int c, const float2 (&v)[RMAX], float2 (&s)[RMAX]) {
+    const size_t base = ((size_t)b * NC3 + c) * plane + coff;
+    const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride + coff : nullptr;
+    combine_column<RMAX, NT, CBM, (ST >= 0)>(stage, a.U + base, a.A1 + base, a.A2 + base, src, cpk + (2 * coff + cko),
+                                  a.c5t + tb, (unsigned)coff, a.coef_t, (unsigned)inner, j, colv, v, s,
+                                  a.ck01 ? a.ck01 + tb : nullptr, a.c6t ? a.c6t + tb : nullptr);
+  };
+  auto load = [&](const float2* X, int c, float2 (&v)[RMAX]) {
+    const size_t base = ((size_t)b * NC3 + c) * plane + coff;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const size_t base = ((size_t)b * 3 + c) * plane + coff;
+    for (int m = 0; m < RMAX; ++m) {
+      const float2 t = X[base + (size_t)(j + m * NT) * inner];
+      v[m] = colv ? t : make_float2(0.f, 0.f);
+    }
+  };
+  float2 s[NC3 / NW][RMAX];
+  if (stage == ST_PRO) {
 #pragma unroll
-        for (int m = 0; m < RMAX; ++m) {
-          const float2 t = a.U[base + (size_t)(j + m * NT) * inner];
-          s[c][m] = colv ? t : make_float2(0.f, 0.f);
-        }
-      }
-    } else {
-      // velocity-form Navier-Stokes: the three convection spectra first, projected mode by mode
-      float2 v3[3][RMAX];
+    for (int k = 0; k < NC3 / NW; ++k) load(a.U, c0 + k, s[k]);
+  } else if constexpr (TERM == TERM_NSP) {
+    // velocity-form Navier-Stokes: the three convection spectra first, projected mode by mode
+    float2 v3[3][RMAX];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const size_t base = ((size_t)b * 3 + c) * plane + coff;
+    for (int c = 0; c < 3; ++c) {
+      load(a.P, c, v3[c]);
+      fft_wg<N0, -1, V, VAR>(v3[c], s_buf, s_tw, j, vi);
+    }
+    const float ayv = a.ay[ky], azv = colv ? a.az[kz] : 0.f;
+    // Nyquist-plane parity of nsp_project (every fused 3D size is even)
+    const bool nyy = 2 * ky == a.N1, nyz = 2 * kz == a.N2, oyz = (ky == 0 || nyy) && (kz == 0 || nyz);
 #pragma unroll
-        for (int m = 0; m < RMAX; ++m) {
-          const float2 t = a.P[base + (size_t)(j + m * NT) * inner];
-          v3[c][m] = colv ? t : make_float2(0.f, 0.f);
-        }
-        fft_wg<N0, -1, V, VAR>(v3[c], s_buf, s_tw, j, vi);
-      }
-      const float ayv = a.ay[ky], azv = colv ? a.az[kz] : 0.f;
-      // Nyquist-plane parity of nsp_project (every fused 3D size is even)
-      const bool nyy = 2 * ky == a.N1, nyz = 2 * kz == a.N2, oyz = (ky == 0 || nyy) && (kz == 0 || nyz);
-#pragma unroll
-      for (int m = 0; m < RMAX; ++m) {
-        float2 cv[3] = {v3[0][m], v3[1][m], v3[2][m]};
-        const int x = j + m * NT;
-        const float av[3] = {a.ax[x], ayv, azv};
-        const bool nyx = 2 * x == N0, own = (x == 0 || nyx) && oyz;
-        const bool ny[3] = {nyx && !own, nyy && !own, nyz && !own};
-        nsp_project<3>(cv, av, ny);
+    for (int m = 0; m < RMAX; ++m) {
+      float2 cv[3] = {v3[0][m], v3[1][m], v3[2][m]};
+      const int x = j + m * NT;
+      const float av[3] = {a.ax[x], ayv, azv};
+      const bool nyx = 2 * x == N0, own = (x == 0 || nyx) && oyz;
+      const bool ny[3] = {nyx && !own, nyy && !own, nyz && !own};
+      nsp_project<3>(cv, av, ny);
+      if constexpr (NW == 3) {
+        v3[0][m] = c0 == 0 ? cv[0] : (c0 == 1 ? cv[1] : cv[2]);
+      } else {
 #pragma unroll
         for (int c = 0; c < 3; ++c) v3[c][m] = cv[c];
       }
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const size_t base = ((size_t)b * 3 + c) * plane + coff;
-        const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride + coff : nullptr;
-        combine_column<RMAX, NT, CBM, (ST >= 0)>(stage, a.U + base, a.A1 + base, a.A2 + base, src, cpk + (2 * coff + cko),
-                                      a.c5t + tb, (unsigned)coff, a.coef_t, (unsigned)inner, j, colv, v3[c], s[c],
-                                      a.ck01 ? a.ck01 + tb : nullptr, a.c6t ? a.c6t + tb : nullptr);
-      }
     }
-    if (!kept) return;
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-      col3_fields<N0, V, VAR>(a, s[c], 2 * c, b, 3, kyc, kz, colv, s_buf, s_tw, s_ax, j, vi);
+    for (int k = 0; k < NC3 / NW; ++k) combine(c0 + k, v3[k], s[k]);
   } else {
-    // one channel at a time: its spectrum, combine and two fields (u^_c, a_x u^_c), so that only
-    // that channel's values are live (the fields of channel c need nothing of the others)
-#pragma unroll
-    for (int c = 0; c < NC3; ++c) {
-      const size_t base = ((size_t)b * NC3 + c) * plane + coff;
-      float2 s[RMAX];
-      if (stage == ST_PRO) {
-#pragma unroll
-        for (int m = 0; m < RMAX; ++m) {
-          const float2 t = a.U[base + (size_t)(j + m * NT) * inner];
-          s[m] = colv ? t : make_float2(0.f, 0.f);
-        }
-      } else {
-        float2 v[RMAX];
-#pragma unroll
-        for (int m = 0; m < RMAX; ++m) {
-          const float2 t = a.P[base + (size_t)(j + m * NT) * inner];
-          v[m] = colv ? t : make_float2(0.f, 0.f);
-        }
-        fft_wg<N0, -1, V, VAR>(v, s_buf, s_tw, j, vi);
-        if constexpr (TERM == TERM_KS) {
-          // remove_mean: fft(p - mean(p)) differs from fft(p) only at k = 0, by the batch mean of the DC
-          if (a.dc && ky == 0 && kz == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
-        }
-        const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)c * a.src_cstride + coff : nullptr;
-        combine_column<RMAX, NT, CBM, (ST >= 0)>(stage, a.U + base, a.A1 + base, a.A2 + base, src, cpk + (2 * coff + cko),
-                                      a.c5t + tb, (unsigned)coff, a.coef_t, (unsigned)inner, j, colv, v, s,
-                                      a.ck01 ? a.ck01 + tb : nullptr, a.c6t ? a.c6t + tb : nullptr);
-      }
-      if (kept) col3_fields<N0, V, VAR>(a, s, 2 * c, b, NC3, kyc, kz, colv, s_buf, s_tw, s_ax, j, vi);
+    float2 v[RMAX];
+    load(a.P, c0, v);
+    fft_wg<N0, -1, V, VAR>(v, s_buf, s_tw, j, vi);
+    if constexpr (TERM == TERM_KS) {
+      // remove_mean: fft(p - mean(p)) differs from fft(p) only at k = 0, by the batch mean of the DC
+      if (a.dc && ky == 0 && kz == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
     }
+    combine(c0, v, s[0]);
   }
+  if (!kept) return;
+#pragma unroll
+  for (int k = 0; k < NC3 / NW; ++k)
+    col3_fields<N0, V, VAR>(a, s[k], 2 * (c0 + k), b, NC3, kyc, kz, colv, s_buf, s_tw, s_ax, j, vi);
 }
 
 // ---------------------------------------------------------------- y columns (inverse, 6 -> 9 fields)
@@ -216,40 +206,40 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * V)) k3_yinv(Yinv3Args a) {
   const int nzt = a.PF2 / V;
   const int kz = (blockIdx.x % nzt) * V + vi;
   const int x = (blockIdx.x / nzt) % a.N0;
-  const int b = a.b0 + blockIdx.x / (nzt * a.N0);
+  // one channel of one sample per workgroup (a loop over the channels was 6 transforms longer: the pass of
+  // NavierStokes 64^3 B = 2 is part of 180 -> 168 us per SETDRK4 step)
+  const int bc = blockIdx.x / (nzt * a.N0);
+  const int b = a.b0 + bc / NCH, c = bc % NCH;
   if (a.mask.skip(b)) return;
   const bool kv = kz <= a.kmax2;
-#pragma unroll 1
-  for (int c = 0; c < NCH; ++c) {
-    const float2* g0 = a.G1 + ((((size_t)b * 2 * NCH + 2 * c) * a.N0 + x) * a.K1) * a.PF2 + kz;
-    const float2* g1 = a.G1 + ((((size_t)b * 2 * NCH + 2 * c + 1) * a.N0 + x) * a.K1) * a.PF2 + kz;
-    float2 f0[RMAX], f1[RMAX];
+  const float2* g0 = a.G1 + ((((size_t)b * 2 * NCH + 2 * c) * a.N0 + x) * a.K1) * a.PF2 + kz;
+  const float2* g1 = a.G1 + ((((size_t)b * 2 * NCH + 2 * c + 1) * a.N0 + x) * a.K1) * a.PF2 + kz;
+  float2 f0[RMAX], f1[RMAX];
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) {
+    const int ky = j + m * NT;
+    const int kc = ky_compress(ky, N1, a.kmax1);
+    const bool ld = kv && kc >= 0;
+    f0[m] = ld ? g0[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
+    f1[m] = ld ? g1[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    float2 v[RMAX];
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
-      const int ky = j + m * NT;
-      const int kc = ky_compress(ky, N1, a.kmax1);
-      const bool ld = kv && kc >= 0;
-      f0[m] = ld ? g0[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
-      f1[m] = ld ? g1[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
+      if (k == 0) v[m] = f0[m];
+      else if (k == 2) v[m] = f1[m];
+      else {
+        const float ay = a.ay[j + m * NT];
+        v[m] = make_float2(mulr(ay, f0[m].x), mulr(ay, f0[m].y));
+      }
     }
+    fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+    if (kz < a.PF2) {
+      float2* g = a.G2 + ((((size_t)b * 3 * NCH + 3 * c + k) * a.N0 + x) * N1) * a.PF2 + kz;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float2 v[RMAX];
-#pragma unroll
-      for (int m = 0; m < RMAX; ++m) {
-        if (k == 0) v[m] = f0[m];
-        else if (k == 2) v[m] = f1[m];
-        else {
-          const float ay = a.ay[j + m * NT];
-          v[m] = make_float2(mulr(ay, f0[m].x), mulr(ay, f0[m].y));
-        }
-      }
-      fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
-      if (kz < a.PF2) {
-        float2* g = a.G2 + ((((size_t)b * 3 * NCH + 3 * c + k) * a.N0 + x) * N1) * a.PF2 + kz;
-#pragma unroll
-        for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.PF2] = v[m];
-      }
+      for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.PF2] = v[m];
     }
   }
 }
@@ -451,20 +441,21 @@ static hipError_t launch_col3d_t(const Col3Args& a, int nb, int stage, hipStream
   const int slots = (ntiles + 7) / 8;
   Col3Args b = a;
   b.nb = nb;
-  const dim3 grid(slots * 8 * nb), block(Fft<NN, VR>::NT * V);
-  if (a.term == TERM_NSP) return launch_col3d_term<NN, VR, TERM_NSP>(b, grid, block, stage, st);
-  if (a.term == TERM_KS) return launch_col3d_term<NN, VR, TERM_KS>(b, grid, block, stage, st);
-  return launch_col3d_term<NN, VR, TERM_CONV>(b, grid, block, stage, st);
+  const dim3 block(Fft<NN, VR>::NT * V);
+  auto grid = [&](int groups) { return dim3(slots * 8 * nb * groups); };
+  if (a.term == TERM_NSP) return launch_col3d_term<NN, VR, TERM_NSP>(b, grid(Col3Channels<TERM_NSP, NN>::groups), block, stage, st);
+  if (a.term == TERM_KS) return launch_col3d_term<NN, VR, TERM_KS>(b, grid(Col3Channels<TERM_KS, NN>::groups), block, stage, st);
+  return launch_col3d_term<NN, VR, TERM_CONV>(b, grid(Col3Channels<TERM_CONV, NN>::groups), block, stage, st);
 }
 
 template <int NN, int VR>
 static hipError_t launch_yinv3d_t(const Yinv3Args& a, hipStream_t st) {
   constexpr int V = 16;
-  const int nzt = a.PF2 / V;
+  const dim3 grid(a.PF2 / V * a.N0 * a.nb * a.nc), block(Fft<NN, VR>::NT * V);
   if (a.nc == 1)
-    TFSM_LAUNCH((k3_yinv<NN, V, VR, 1>), dim3(nzt * a.N0 * a.nb), dim3(Fft<NN, VR>::NT * V), 0, st, a);
+    TFSM_LAUNCH((k3_yinv<NN, V, VR, 1>), grid, block, 0, st, a);
   else
-    TFSM_LAUNCH((k3_yinv<NN, V, VR, 3>), dim3(nzt * a.N0 * a.nb), dim3(Fft<NN, VR>::NT * V), 0, st, a);
+    TFSM_LAUNCH((k3_yinv<NN, V, VR, 3>), grid, block, 0, st, a);
   return hipGetLastError();
 }
 
