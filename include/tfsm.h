@@ -335,8 +335,8 @@ int tfsm_launch_pass(tfsm_plan* plan, void* uh, void* ws, int32_t pass_id, int32
 int tfsm_launch_pass_timed(tfsm_plan* p, void* uh, void* ws, int32_t pass_id, int32_t stage, int32_t sub,
                            void* ev_start, void* ev_stop, void* stream);
 
-/* Bytes of the adjoint workspace tfsm_adjoint_step needs (stage arrays, transposed-Jacobian
- * fields and products). */
+/* Bytes of the adjoint workspace tfsm_adjoint_step needs with the plan's current scheme and path (stage
+ * arrays, transposed-Jacobian fields and products; less on the fused 2D kernels). */
 int64_t tfsm_plan_adjoint_workspace_bytes(const tfsm_plan* plan);
 
 /* Prepare the adjoint of the plan's current scheme (ETDRK1/2, SETDRK1/2; Convection in 1D/2D):

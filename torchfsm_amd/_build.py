@@ -16,7 +16,7 @@ OBJDIR = os.path.join(CSRC, "_build")
 LIB = os.path.join(HERE, "libtfsm.so")
 SOURCES = ["api.hip", "k_coefs.hip", "k_transform.hip", "k_step2d.hip", "k_step2d_vc.hip", "k_step2d_conv.hip",
            "k_step2d_nsp.hip", "k_step2d_ks.hip", "k_step2d_cons.hip",
-           "k_step2d_mixed.hip", "k_step3d.hip", "k_adjoint.hip",
+           "k_step2d_mixed.hip", "k_step3d.hip", "k_adjoint.hip", "k_adjoint2d.hip",
            "k_maps.hip", "k_gfft.hip", "k_long1d.hip", "k_genfused.hip", "k_general.hip"]
 ARCH = "gfx950"
 # packed FP32 instructions are disabled for all device code

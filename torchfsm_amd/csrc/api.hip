@@ -993,39 +993,70 @@ AdjArgs adj_args(tfsm_plan* p) {
 }
 
 struct AdjLayout {
-  size_t Aa, N0s, T1, Jv, Ab, Nb, Na, Ac, Nc, Cb, Bb, Abar, gpart, F, Fs, X, Q, total;
+  size_t Aa, N0s, T1, Jv, Ab, Nb, Na, Ac, Nc, Cb, Bb, Abar, part, F, Fs, X, Q;
+  size_t Ga, Gb, Gc, Qs, GP;  // fused 2D path
+  size_t total;
 };
 
 // fields and products of the transposed Jacobian (k_adj_fields / k_adj_products)
 int adj_nfa(const tfsm_plan* p) { return p->term == TERM_VC ? 5 : 2 * p->C + p->C * p->D; }
 int adj_nq(const tfsm_plan* p) { return p->term == TERM_VC ? 4 : p->C + p->C * p->D; }
 
+// 2D plans of the fused kernels whose axes k_adjoint2d.hip covers
+bool adj_fused(const tfsm_plan* p) {
+  return p->D == 2 && p->fused_ok && !p->general && adj2d_size(p->n[0]) && adj2d_size(p->n[1]) && !p->force &&
+         (p->term == TERM_VC ? p->C == 1 : p->term == TERM_CONV && p->C == 2);
+}
+
+// workgroups per sample of the coefficient gradient: 512 modes each, up to 256
+int adj_grad_blocks(const tfsm_plan* p) {
+  const size_t n = ((size_t)p->C * p->modes + 511) / 512;
+  return n > 256 ? 256 : (int)n;
+}
+
 AdjLayout adj_layout(const tfsm_plan* p) {
   const int nfa = adj_nfa(p), nq = adj_nq(p);
   size_t npts = 1;
   for (int d = 0; d < p->D; ++d) npts *= p->n[d];
   const size_t S = roundup(p->state_elems() * sizeof(float2), 256);
-  AdjLayout l;
-  size_t o = 0;
-  l.Aa = o; o += S;
-  l.N0s = o; o += S;
-  l.T1 = o; o += S;
-  l.Jv = o; o += S;
-  l.Ab = o; o += S;
-  l.Nb = o; o += S;
-  // SETDRK4 only: Na, c, Nc and the stage adjoints
   const bool four = p->scheme == SETDRK4;
-  l.Na = o; o += four ? S : 0;
-  l.Ac = o; o += four ? S : 0;
-  l.Nc = o; o += four ? S : 0;
-  l.Cb = o; o += four ? S : 0;
-  l.Bb = o; o += four ? S : 0;
-  l.Abar = o; o += four ? S : 0;
-  l.gpart = o; o += roundup(p->state_elems() * sizeof(float), 256);
-  l.F = o; o += roundup((size_t)p->B * nfa * p->modes * sizeof(float2), 256);
-  l.Fs = o; o += roundup((size_t)p->B * (nfa > nq ? nfa : nq) * p->modes * sizeof(float2), 256);
-  l.X = o; o += roundup((size_t)p->B * nfa * npts * sizeof(float), 256);
-  l.Q = o; o += roundup((size_t)p->B * nq * npts * sizeof(float), 256);
+  AdjLayout l = {};
+  size_t o = 0;
+  auto take = [&](size_t& at, size_t bytes) { at = o; o += roundup(bytes, 256); };
+  take(l.part, (size_t)p->B * adj_grad_blocks(p) * sizeof(double));
+  take(l.Na, S);
+  take(l.Ab, S);
+  if (four) {
+    take(l.Nb, S);
+    take(l.Nc, S);
+    take(l.Cb, S);
+    take(l.Bb, S);
+  }
+  if (adj_fused(p)) {
+    const size_t fields = (size_t)p->B * 4 * p->n[0] * p->PF * sizeof(float2);
+    take(l.Ga, fields);
+    if (four) {
+      take(l.Gb, fields);
+      take(l.Gc, fields);
+    }
+    take(l.Qs, fields);
+    take(l.GP, S);
+    l.total = o;
+    return l;
+  }
+  take(l.Aa, S);
+  take(l.N0s, S);
+  take(l.T1, S);
+  take(l.Jv, S);
+  if (!four) take(l.Nb, S);
+  if (four) {
+    take(l.Ac, S);
+    take(l.Abar, S);
+  }
+  take(l.F, (size_t)p->B * nfa * p->modes * sizeof(float2));
+  take(l.Fs, (size_t)p->B * (nfa > nq ? nfa : nq) * p->modes * sizeof(float2));
+  take(l.X, (size_t)p->B * nfa * npts * sizeof(float));
+  take(l.Q, (size_t)p->B * nq * npts * sizeof(float));
   l.total = o;
   return l;
 }
@@ -1090,7 +1121,7 @@ void lin_term(AdjLinArgs& a, const float2* X, int slot, float s) {
   ++a.nt;
 }
 
-AdjGradArgs grad_args(tfsm_plan* p, const float2* Xbar, float* gpart, int accumulate) {
+AdjGradArgs grad_args(tfsm_plan* p, char* wsa, double* grad) {
   AdjGradArgs g;
   g.B = p->B;
   g.C = p->C;
@@ -1098,28 +1129,210 @@ AdjGradArgs grad_args(tfsm_plan* p, const float2* Xbar, float* gpart, int accumu
   g.H = p->H;
   g.nlast = p->n[p->D - 1];
   g.modes = p->modes;
+  g.coef = p->coef;
+  g.coef_bstride = p->coef_bstride();
   g.dcoef = p->dcoef;
   g.dcoef_bstride = p->Bc > 1 ? (size_t)ADJ_NDCOEF * p->modes : 0;
   g.sym = p->sym;
-  g.Xbar = Xbar;
   g.nt = 0;
-  g.gpart = gpart;
-  g.accumulate = accumulate;
+  g.nblk = adj_grad_blocks(p);
+  g.part = (double*)(wsa + adj_layout(p).part);
+  g.out = grad;
   return g;
 }
 
-void grad_term(AdjGradArgs& g, const float2* Y, int dslot, float s) {
+// one term s dc c <X, Y>
+void grad_term(AdjGradArgs& g, const float2* X, const float2* Y, int dslot, float s, int cslot = -1) {
+  g.X[g.nt] = X;
   g.Y[g.nt] = Y;
   g.dslot[g.nt] = dslot;
-  g.s[g.nt] = s;
-  ++g.nt;
+  g.cslot[g.nt] = cslot;
+  g.s[g.nt++] = s;
+}
+
+enum { D_E = 0, D_C1 = 1, D_C2 = 2 };                                                // slots of 1- and 2-stage schemes
+enum { D4_E = 0, D4_E2 = 1, D4_C1 = 2, D4_C4 = 3, D4_C5 = 4, D4_C6 = 5 };  // of SETDRK4
+
+// SETDRK4's coefficient gradient; a = E2 u + c1 N0 enters as its two terms
+int adj_grad4(tfsm_plan* p, const float2* U, const float2* Ubn, const float2* N0, const float2* Na, const float2* Nb,
+              const float2* Nc, const float2* Cb, const float2* Bb, const float2* Ab, char* wsa, double* grad,
+              hipStream_t st) {
+  AdjGradArgs g = grad_args(p, wsa, grad);
+  grad_term(g, Ubn, U, D4_E, 1.f);
+  grad_term(g, Ubn, N0, D4_C4, 1.f);
+  grad_term(g, Ubn, Na, D4_C5, 2.f);
+  grad_term(g, Ubn, Nb, D4_C5, 2.f);
+  grad_term(g, Ubn, Nc, D4_C6, 1.f);
+  grad_term(g, Cb, U, D4_E2, 1.f, CS_E2);
+  grad_term(g, Cb, N0, D4_E2, 1.f, CS_C1);
+  grad_term(g, Cb, Nb, D4_C1, 2.f);
+  grad_term(g, Cb, N0, D4_C1, -1.f);
+  grad_term(g, Bb, U, D4_E2, 1.f);
+  grad_term(g, Bb, Na, D4_C1, 1.f);
+  grad_term(g, Ab, U, D4_E2, 1.f);
+  grad_term(g, Ab, N0, D4_C1, 1.f);
+  HIP_TRY(launch_adj_grad(g, st), "adjoint gradient launch");
+  return TFSM_OK;
+}
+
+// One adjoint step on the fused kernels (k_adjoint2d.hip).  The step's own stages run on k2_row and k2_col
+// into one field array each; on the way back, every stage is a row launch (products, and with `grad` that
+// state's own product) and a column launch that ends in the next stage's adjoint fields.
+int adj_step_fused(tfsm_plan* p, float2* U, const float2* Ubn, float2* Ubo, double* grad, char* W, char* A,
+                   hipStream_t st) {
+  const AdjLayout l = adj_layout(p);
+  const bool want = grad && p->adj_term >= 0;
+  float2* Pr = (float2*)(W + p->off_P);
+  float2* A1 = (float2*)(W + p->off_A1);  // N0
+  float2* Gu = (float2*)(W + p->off_G);
+  float2 *Ga = (float2*)(A + l.Ga), *Gb = (float2*)(A + l.Gb), *Gc = (float2*)(A + l.Gc);
+  float2 *Na = (float2*)(A + l.Na), *Nb = (float2*)(A + l.Nb), *Nc = (float2*)(A + l.Nc);
+  float2 *Ab = (float2*)(A + l.Ab), *Bb = (float2*)(A + l.Bb), *Cb = (float2*)(A + l.Cb);
+  Adj2RowArgs r;
+  r.B = p->B;
+  r.N0 = p->n[0];
+  r.N1 = p->n[1];
+  r.P1 = p->P;
+  r.PF = p->PF;
+  r.kmax1 = p->kmax[1];
+  r.tw1 = p->tw[1][adj2d_var(p->n[1])];
+  r.ay = p->kv[1];
+  r.GP = (float2*)(A + l.GP);
+  r.Q = (float2*)(A + l.Qs);
+  Adj2ColArgs base;
+  base.B = p->B;
+  base.N0 = p->n[0];
+  base.H1 = p->H;
+  base.P1 = p->P;
+  base.PF = p->PF;
+  base.kmax0 = p->kmax[0];
+  base.kmax1 = p->kmax[1];
+  base.coef_t = p->coef_t;
+  base.scale = (float)(1.0 / ((double)p->n[0] * p->n[1]));
+  base.tw0 = p->tw[0][adj2d_var(p->n[0])];
+  base.ax = p->kv[0];
+  base.ay = p->kv[1];
+  base.coef = p->coef;
+  base.coef_bstride = p->coef_bstride();
+  base.P = Pr;
+  base.src = p->src;
+  base.src_bstride = p->src_bstride();
+  base.src_cstride = p->src_cstride();
+  base.Q = nullptr;
+  base.N = base.Y = base.GP = nullptr;
+  base.nt = base.nv = 0;
+  base.yslot = CS_C1;
+  base.ys = 0.f;
+  auto x_term = [](Adj2ColArgs& c, const float2* X, int slot, float s) {
+    c.X[c.nt] = X;
+    c.slot[c.nt] = slot;
+    c.s[c.nt++] = s;
+  };
+  auto v_term = [](Adj2ColArgs& c, const float2* X, int slot, float s) {
+    c.V[c.nv] = X;
+    c.vslot[c.nv] = slot;
+    c.vs[c.nv++] = s;
+  };
+  // fields of stage `stage`'s result into G (the last array the stage reads is the product in ws)
+  auto stage = [&](int sc, float2* G) -> int {
+    Col2Args c = col_args(p, U, W);
+    c.G = G;
+    HIP_TRY(launch_col2d(p->term, c, p->B, sc, p->V, p->col_var, st), "column kernel launch");
+    return TFSM_OK;
+  };
+  auto rows = [&](float2* G) -> int {
+    Row2Args q = row_args(p, W, 0, p->B);
+    q.G = G;
+    HIP_TRY(launch_row2d(p->term, q, p->row_var, p->row_wg, st), "row kernel launch");
+    return TFSM_OK;
+  };
+  auto in = [&](int slot) -> int {  // c u'bar -> GP
+    Adj2ColArgs c = base;
+    v_term(c, Ubn, slot, 1.f);
+    c.GP = (float2*)(A + l.GP);
+    HIP_TRY(launch_adj2d_col(p->term, c, st), "adjoint column launch");
+    return TFSM_OK;
+  };
+  // products of the fields G with the adjoint fields, then the column pass c; N(state) -> N with `want`
+  auto back = [&](Adj2ColArgs& c, const float2* G, float2* N) -> int {
+    r.G = G;
+    r.P = want && N ? Pr : nullptr;
+    HIP_TRY(launch_adj2d_row(p->term, r, st), "adjoint row launch");
+    c.Q = r.Q;
+    c.N = want ? N : nullptr;
+    HIP_TRY(launch_adj2d_col(p->term, c, st), "adjoint column launch");
+    return TFSM_OK;
+  };
+  int rc = stage(ST_PRO, Gu);
+  if (rc) return rc;
+  if (p->scheme == SETDRK4) {
+    if ((rc = rows(Gu)) || (rc = stage(ST_R4_E0, Ga)) || (rc = rows(Ga)) || (rc = stage(ST_R4_E1, Gb)) ||
+        (rc = rows(Gb)) || (rc = stage(ST_R4_E2, Gc)) || (rc = in(CS_C6)))
+      return rc;
+    Adj2ColArgs c = base;  // cbar = J(c)^T c6 u'bar;  Nb bar = 2 c1 cbar + 2 c5 u'bar
+    c.Y = Cb;
+    c.ys = 2.f;
+    v_term(c, Ubn, CS_C5, 2.f);
+    c.GP = (float2*)(A + l.GP);
+    if ((rc = back(c, Gc, Nc))) return rc;
+    c = base;  // bbar = J(b)^T Nb bar;  Na bar = c1 bbar + 2 c5 u'bar
+    c.Y = Bb;
+    c.ys = 1.f;
+    v_term(c, Ubn, CS_C5, 2.f);
+    c.GP = (float2*)(A + l.GP);
+    if ((rc = back(c, Gb, Nb))) return rc;
+    c = base;  // abar = E2 cbar + J(a)^T Na bar;  N0 bar = c1 abar - c1 cbar + c4 u'bar
+    x_term(c, Cb, CS_E2, 1.f);
+    c.Y = Ab;
+    c.ys = 1.f;
+    v_term(c, Cb, CS_C1, -1.f);
+    v_term(c, Ubn, CS_C4, 1.f);
+    c.GP = (float2*)(A + l.GP);
+    if ((rc = back(c, Ga, Na))) return rc;
+    c = base;  // ubar = E u'bar + E2 bbar + E2 abar + J(u)^T N0 bar
+    x_term(c, Ubn, CS_E, 1.f);
+    x_term(c, Bb, CS_E2, 1.f);
+    x_term(c, Ab, CS_E2, 1.f);
+    c.Y = Ubo;
+    if ((rc = back(c, Gu, nullptr))) return rc;
+    return want ? adj_grad4(p, U, Ubn, A1, Na, Nb, Nc, Cb, Bb, Ab, A, grad, st) : TFSM_OK;
+  }
+  const bool two = p->scheme == ETDRK2 || p->scheme == SETDRK2;
+  AdjGradArgs g = grad_args(p, A, grad);
+  if (two) {
+    if ((rc = rows(Gu)) || (rc = stage(scheme_stage(p->scheme, 0), Ga)) || (rc = in(CS_C2))) return rc;
+    Adj2ColArgs c = base;  // abar = u'bar + J(a)^T c2 u'bar;  N0 bar = c1 abar - c2 u'bar
+    x_term(c, Ubn, -1, 1.f);
+    c.Y = Ab;
+    c.ys = 1.f;
+    v_term(c, Ubn, CS_C2, -1.f);
+    c.GP = (float2*)(A + l.GP);
+    if ((rc = back(c, Ga, Na))) return rc;
+    c = base;  // ubar = E abar + J(u)^T N0 bar
+    x_term(c, Ab, CS_E, 1.f);
+    c.Y = Ubo;
+    if ((rc = back(c, Gu, nullptr))) return rc;
+    grad_term(g, Ubn, Na, D_C2, 1.f);
+    grad_term(g, Ubn, A1, D_C2, -1.f);
+    grad_term(g, Ab, U, D_E, 1.f);
+    grad_term(g, Ab, A1, D_C1, 1.f);
+  } else {
+    if ((rc = in(CS_C1))) return rc;
+    Adj2ColArgs c = base;  // ubar = E u'bar + J(u)^T c1 u'bar
+    x_term(c, Ubn, CS_E, 1.f);
+    c.Y = Ubo;
+    if ((rc = back(c, Gu, Na))) return rc;  // (Na: N0 here)
+    grad_term(g, Ubn, U, D_E, 1.f);
+    grad_term(g, Ubn, Na, D_C1, 1.f);
+  }
+  if (want) HIP_TRY(launch_adj_grad(g, st), "adjoint gradient launch");
+  return TFSM_OK;
 }
 
 // One adjoint SETDRK4 step (see k_adjoint.hip): recompute N0, a, Na, b, Nb, c (and Nc for the
 // coefficient gradient) from u, then the transposed stages from c back to u.
 int adjoint_step4(tfsm_plan* p, float2* U, const float2* Ubn, float2* Ubo, double* grad, char* W, char* A,
                   hipStream_t st) {
-  enum { D_E = 0, D_E2 = 1, D_C1 = 2, D_C4 = 3, D_C5 = 4, D_C6 = 5 };
   const AdjLayout l = adj_layout(p);
   float2* A1 = (float2*)(W + p->off_A1);
   float2* N0 = (float2*)(A + l.N0s);
@@ -1134,7 +1347,7 @@ int adjoint_step4(tfsm_plan* p, float2* U, const float2* Ubn, float2* Ubo, doubl
   float2* Cb = (float2*)(A + l.Cb);
   float2* Bb = (float2*)(A + l.Bb);
   float2* Ab = (float2*)(A + l.Abar);
-  float* gp = (grad && p->adj_term >= 0) ? (float*)(A + l.gpart) : nullptr;
+  const bool want = grad && p->adj_term >= 0;
   const size_t sbytes = p->state_elems() * sizeof(float2);
   auto nonlin = [&](float2* X, float2* out) -> int {
     int rc = eval_nonlinear(p, X, W, st);
@@ -1161,7 +1374,7 @@ int adjoint_step4(tfsm_plan* p, float2* U, const float2* Ubn, float2* Ubo, doubl
   lin_term(a, Nb, CS_C1, 2.f);
   lin_term(a, N0, CS_C1, -1.f);
   if ((rc = comb(a))) return rc;
-  if (gp && (rc = nonlin(Sc, Nc))) return rc;
+  if (want && (rc = nonlin(Sc, Nc))) return rc;
   // backward
   a = lin_args(p, T);  // Nc bar = c6 u'bar
   lin_term(a, Ubn, CS_C6, 1.f);
@@ -1189,29 +1402,7 @@ int adjoint_step4(tfsm_plan* p, float2* U, const float2* Ubn, float2* Ubo, doubl
   lin_term(a, Ab, CS_E2, 1.f);
   lin_term(a, Jv, -1, 1.f);
   if ((rc = comb(a))) return rc;
-  if (!gp) return TFSM_OK;
-  AdjGradArgs g = grad_args(p, Ubn, gp, 0);
-  grad_term(g, U, D_E, 1.f);
-  grad_term(g, N0, D_C4, 1.f);
-  grad_term(g, Na, D_C5, 2.f);
-  grad_term(g, Nb, D_C5, 2.f);
-  grad_term(g, Nc, D_C6, 1.f);
-  HIP_TRY(launch_adj_gacc(g, st), "adjoint gradient launch");
-  g = grad_args(p, Cb, gp, 1);
-  grad_term(g, Sa, D_E2, 1.f);
-  grad_term(g, Nb, D_C1, 2.f);
-  grad_term(g, N0, D_C1, -1.f);
-  HIP_TRY(launch_adj_gacc(g, st), "adjoint gradient launch");
-  g = grad_args(p, Bb, gp, 1);
-  grad_term(g, U, D_E2, 1.f);
-  grad_term(g, Na, D_C1, 1.f);
-  HIP_TRY(launch_adj_gacc(g, st), "adjoint gradient launch");
-  g = grad_args(p, Ab, gp, 1);
-  grad_term(g, U, D_E2, 1.f);
-  grad_term(g, N0, D_C1, 1.f);
-  HIP_TRY(launch_adj_gacc(g, st), "adjoint gradient launch");
-  HIP_TRY(launch_adj_reduce(gp, (size_t)p->C * p->modes, p->B, grad, st), "adjoint reduce launch");
-  return TFSM_OK;
+  return want ? adj_grad4(p, U, Ubn, N0, Na, Nb, Nc, Cb, Bb, Ab, A, grad, st) : TFSM_OK;
 }
 
 AdjStageArgs stage_args(tfsm_plan* p, int op) {
@@ -1222,16 +1413,11 @@ AdjStageArgs stage_args(tfsm_plan* p, int op) {
   s.C = p->C;
   s.P = p->P;
   s.H = p->H;
-  s.nlast = p->n[p->D - 1];
   s.modes = p->modes;
   s.coef = p->coef;
   s.coef_bstride = p->coef_bstride();
-  s.dcoef = p->dcoef;
-  s.dcoef_bstride = p->Bc > 1 ? (size_t)ADJ_NDCOEF * p->modes : 0;
-  s.sym = p->sym;
-  s.X0 = s.X1 = s.X2 = s.X3 = nullptr;
+  s.X0 = s.X1 = nullptr;
   s.Y0 = s.Y1 = nullptr;
-  s.gpart = nullptr;
   return s;
 }
 
@@ -2278,9 +2464,11 @@ int tfsm_adjoint_step(tfsm_plan* p, void* u, const void* ubar_next, void* ubar, 
   float2* Jv = (float2*)(A + l.Jv);
   float2* Ab = (float2*)(A + l.Ab);
   float2* Nb = (float2*)(A + l.Nb);
-  float* gp = (grad && p->adj_term >= 0) ? (float*)(A + l.gpart) : nullptr;
+  const bool want = grad && p->adj_term >= 0;
   const size_t sbytes = p->state_elems() * sizeof(float2);
+  if (adj_fused(p)) return adj_step_fused(p, U, Ubn, Ubo, grad, W, A, st);
   if (p->scheme == SETDRK4) return adjoint_step4(p, U, Ubn, Ubo, grad, W, A, st);
+  AdjGradArgs g = grad_args(p, A, grad);
   int rc = eval_nonlinear(p, U, W, st);
   if (rc) return rc;
   HIP_TRY(hipMemcpyAsync(N0s, A1, sbytes, hipMemcpyDeviceToDevice, st), "adjoint copy");
@@ -2302,16 +2490,15 @@ int tfsm_adjoint_step(tfsm_plan* p, void* u, const void* ubar_next, void* ubar, 
     s = stage_args(p, ADJ_MID);
     s.X0 = Ubn;
     s.X1 = Jv;
-    s.X2 = A1;
-    s.X3 = N0s;
     s.Y0 = Ab;
     s.Y1 = Nb;
-    s.gpart = gp;
     HIP_TRY(launch_adj_stage(s, st), "adjoint stage launch");
     rc = adj_jt(p, U, Nb, Jv, A, st);
     if (rc) return rc;
     s = stage_args(p, ADJ_POST);
     s.X0 = Ab;
+    grad_term(g, Ubn, A1, D_C2, 1.f);
+    grad_term(g, Ubn, N0s, D_C2, -1.f);
   } else {
     s.X0 = Ubn;
     s.Y0 = T1;
@@ -2322,12 +2509,11 @@ int tfsm_adjoint_step(tfsm_plan* p, void* u, const void* ubar_next, void* ubar, 
     s.X0 = Ubn;
   }
   s.X1 = Jv;
-  s.X2 = U;
-  s.X3 = N0s;
   s.Y0 = Ubo;
-  s.gpart = gp;
   HIP_TRY(launch_adj_stage(s, st), "adjoint stage launch");
-  if (gp) HIP_TRY(launch_adj_reduce(gp, (size_t)p->C * p->modes, p->B, grad, st), "adjoint reduce launch");
+  grad_term(g, s.X0, U, D_E, 1.f);
+  grad_term(g, s.X0, N0s, D_C1, 1.f);
+  if (want) HIP_TRY(launch_adj_grad(g, st), "adjoint gradient launch");
   return TFSM_OK;
 }
 

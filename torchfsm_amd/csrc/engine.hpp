@@ -793,20 +793,14 @@ struct AdjArgs {
 enum AdjOp : int { ADJ_STAGE_A = 0, ADJ_PRE = 1, ADJ_MID = 2, ADJ_POST = 3 };
 struct AdjStageArgs {
   int op, two_stage;
-  int B, C, P, H, nlast;
+  int B, C, P, H;
   size_t modes;
   const float* coef;        // [Bc][NCOEF][modes]
   size_t coef_bstride;
-  const float* dcoef;       // [Bc][3][modes]: dE/dL, dc1/dL, dc2/dL
-  size_t dcoef_bstride;
-  const float* sym;         // dL/dtheta [modes]
   const float2* X0;
   const float2* X1;
-  const float2* X2;
-  const float2* X3;
   float2* Y0;
   float2* Y1;
-  float* gpart;             // [B][C][modes] per-mode gradient terms, or null
 };
 constexpr int ADJ_NDCOEF = 6;  // coefficient-derivative slots: 2-stage dE, dc1, dc2; SETDRK4 dE, dE2, dc1, dc4, dc5, dc6
 constexpr int ADJ_MAXT = 5;
@@ -821,29 +815,75 @@ struct AdjLinArgs {
   float s[ADJ_MAXT];
   float2* Y;
 };
+// Coefficient gradient of one step: sum over modes and terms of w S s dc c <X, Y>, per sample; dc a derivative
+// table (dslot), c a coefficient table (cslot, or 1).
+constexpr int ADJ_MAXGT = 13;  // SETDRK4's: 5 + 4 + 2 + 2 terms
 struct AdjGradArgs {
   int B, C, P, H, nlast;
   size_t modes;
+  const float* coef;        // [Bc][NCOEF][modes]
+  size_t coef_bstride;
   const float* dcoef;       // [Bc][ADJ_NDCOEF][modes]
   size_t dcoef_bstride;
   const float* sym;         // dL/dtheta [modes]
-  const float2* Xbar;
-  int nt;
-  const float2* Y[ADJ_MAXT];
-  int dslot[ADJ_MAXT];
-  float s[ADJ_MAXT];
-  float* gpart;
-  int accumulate;
+  int nt;                   // 2, 4 or 13
+  const float2* X[ADJ_MAXGT];
+  const float2* Y[ADJ_MAXGT];
+  int dslot[ADJ_MAXGT], cslot[ADJ_MAXGT];
+  float s[ADJ_MAXGT];
+  int nblk;                 // workgroups per sample
+  double* part;             // [B][nblk]
+  double* out;              // [B], added to
 };
+// fused 2D adjoint (k_adjoint2d.hip)
+struct Adj2RowArgs {
+  int B, N0, N1, P1, PF, kmax1;
+  const float2* tw1;
+  const float* ay;
+  const float2* G;          // fields of the stage's state [B][4][N0][PF]
+  const float2* GP;         // x-inverse of the stage adjoint [B][C][N0][P1]
+  float2* Q;                // row transforms of the products [B][4][N0][PF]
+  float2* P;                // row transforms of the state's own product [B][C][N0][P1], or null
+};
+constexpr int ADJ2_MAXT = 3;
+struct Adj2ColArgs {
+  int B, N0, H1, P1, PF, kmax0, kmax1;
+  float coef_t, scale;
+  const float2* tw0;
+  const float* ax;
+  const float* ay;
+  const float* coef;        // [Bc][NCOEF][N0 P1]
+  size_t coef_bstride;
+  const float2* Q;          // null: no W and no Y
+  const float2* P;          // rows of the state's own product, read when N is set
+  float2* N;                // N(u), or null
+  const float2* src;
+  size_t src_bstride, src_cstride;
+  int nt;                   // Y = W + sum s c X  (slot < 0: c = 1)
+  const float2* X[ADJ2_MAXT];
+  int slot[ADJ2_MAXT];
+  float s[ADJ2_MAXT];
+  float2* Y;
+  int yslot;                // v = ys c_yslot Y + sum vs c V
+  float ys;
+  int nv;
+  const float2* V[ADJ2_MAXT];
+  int vslot[ADJ2_MAXT];
+  float vs[ADJ2_MAXT];
+  float2* GP;               // x-inverse of v, or null
+};
+bool adj2d_size(int n);
+int adj2d_var(int n);
+hipError_t launch_adj2d_row(int term, const Adj2RowArgs& a, hipStream_t st);
+hipError_t launch_adj2d_col(int term, const Adj2ColArgs& a, hipStream_t st);
 hipError_t launch_adj_fields(const AdjArgs& a, const float2* U, const float2* V, float2* F, hipStream_t st);
 hipError_t launch_adj_dcoefs4(const float* L, size_t modes, int Bc, double dt, int M, double r, float* dcoef,
                               hipStream_t st);
 hipError_t launch_adj_lincomb(const AdjLinArgs& a, hipStream_t st);
-hipError_t launch_adj_gacc(const AdjGradArgs& a, hipStream_t st);
+hipError_t launch_adj_grad(const AdjGradArgs& a, hipStream_t st);
 hipError_t launch_adj_products(const AdjArgs& a, const float* X, float* Q, hipStream_t st);
 hipError_t launch_adj_combine(const AdjArgs& a, const float2* R, float2* W, hipStream_t st);
 hipError_t launch_adj_stage(const AdjStageArgs& a, hipStream_t st);
-hipError_t launch_adj_reduce(const float* gpart, size_t per, int B, double* out, hipStream_t st);
 hipError_t launch_adj_dcoefs(const float* L, size_t modes, int Bc, double dt, float* dcoef, hipStream_t st);
 hipError_t launch_adj_sym(const AdjArgs& a, int kind, float* S, hipStream_t st);
 

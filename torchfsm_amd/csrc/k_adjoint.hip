@@ -207,11 +207,8 @@ __global__ void k_adj_stage(AdjStageArgs a) {
   const size_t total = (size_t)a.B * a.C * a.modes;
   for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
     const size_t mode = e % a.modes;
-    const size_t bc = e / a.modes;
-    const size_t b = bc / a.C;
-    const int k = (int)(mode % a.P);
-    const bool valid = k < a.H;
-    const float w = !valid ? 0.f : ((k == 0 || 2 * k == a.nlast) ? 1.f : 2.f);
+    const size_t b = e / a.modes / a.C;
+    const bool valid = (int)(mode % a.P) < a.H;
     const float* cf = a.coef + b * a.coef_bstride + mode;
     const float E = cf[CS_E * a.modes];
     const float c1 = cf[CS_C1 * a.modes];
@@ -225,50 +222,65 @@ __global__ void k_adj_stage(AdjStageArgs a) {
       case ADJ_PRE:  // t = c u'bar (c = c2 for 2-stage, c1 for 1-stage)
         a.Y0[e] = cscale(a.two_stage ? c2 : c1, x0);
         break;
-      case ADJ_MID: {  // abar = u'bar + J1; N0bar = c1 abar - c2 u'bar; g = <u'bar, dc2 (Na - N0)>
+      case ADJ_MID: {  // abar = u'bar + J1; N0bar = c1 abar - c2 u'bar
         const float2 ab = valid ? cadd(x0, a.X1[e]) : z;
         a.Y0[e] = ab;
         a.Y1[e] = valid ? csub(cscale(c1, ab), cscale(c2, x0)) : z;
-        float g = 0.f;
-        if (valid && a.gpart) {
-          const float* dc = a.dcoef + b * a.dcoef_bstride + mode;
-          const float s = a.sym[mode];
-          g = w * rdot(x0, cscale(dc[2 * a.modes] * s, csub(a.X2[e], a.X3[e])));
-        }
-        if (a.gpart) a.gpart[e] = g;
         break;
       }
-      case ADJ_POST: {  // ubar = E abar + J0; g += <abar, dE u + dc1 N0>
+      case ADJ_POST:  // ubar = E abar + J0
         a.Y0[e] = valid ? cadd(cscale(E, x0), a.X1[e]) : z;
-        if (a.gpart) {
-          float g = 0.f;
-          if (valid) {
-            const float* dc = a.dcoef + b * a.dcoef_bstride + mode;
-            const float s = a.sym[mode];
-            const float2 d = cadd(cscale(dc[0] * s, a.X2[e]), cscale(dc[a.modes] * s, a.X3[e]));
-            g = w * rdot(x0, d);
-          }
-          a.gpart[e] = a.two_stage ? a.gpart[e] + g : g;
-        }
         break;
-      }
     }
   }
 }
 
-// per-sample sum of gpart [B][per] in a fixed order (float64), added to out[b]
-__global__ void k_adj_reduce(const float* __restrict__ gpart, size_t per, double* __restrict__ out) {
-  __shared__ double s[256];
-  const size_t b = blockIdx.x;
+// Coefficient gradient (AdjGradArgs) in float64 from the float32 states, in a fixed order: a.nblk workgroups
+// per sample, whose partial sums k_adj_gsum adds up.  The terms are unrolled, so that their loads are in
+// flight together.  (One workgroup per sample that summed per-mode terms stored by the stage kernels took
+// 20.8 us at 128^2, C = 2, B = 16; this and
+// k_adj_gsum 5.6 + 2.5, with a run-time loop over the terms 15.1 + 3.8.)
+template <int NT>
+__global__ void __launch_bounds__(256) k_adj_grad(AdjGradArgs a) {
+  __shared__ double s_acc[4];
+  const int b = blockIdx.x / a.nblk, blk = blockIdx.x % a.nblk;
+  const unsigned modes = (unsigned)a.modes, per = a.C * modes;
+  const float* dc = a.dcoef + (size_t)b * a.dcoef_bstride;
+  const float* cf = a.coef + (size_t)b * a.coef_bstride;
   double acc = 0.0;
-  for (size_t i = threadIdx.x; i < per; i += blockDim.x) acc += (double)gpart[b * per + i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
+  for (unsigned i = blk * 256 + threadIdx.x; i < per; i += a.nblk * 256) {
+    const unsigned mode = a.C == 1 ? i : i % modes;
+    const int k = (int)(mode % (unsigned)a.P);
+    if (k >= a.H) continue;
+    const size_t e = (size_t)b * per + i;
+    float2 x[NT], y[NT];
+    float d[NT], c[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      x[t] = a.X[t][e];
+      y[t] = a.Y[t][e];
+      d[t] = dc[(size_t)a.dslot[t] * modes + mode];
+      c[t] = cf[(size_t)(a.cslot[t] >= 0 ? a.cslot[t] : 0) * modes + mode];
+    }
+    double g = 0.0;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const double f = (double)(a.s[t] * d[t]) * (a.cslot[t] >= 0 ? (double)c[t] : 1.0);
+      g += f * ((double)x[t].x * y[t].x + (double)x[t].y * y[t].y);
+    }
+    acc += g * (double)(((k == 0 || 2 * k == a.nlast) ? 1.f : 2.f) * a.sym[mode]);
   }
-  if (threadIdx.x == 0) out[b] += s[0];
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
+  if ((threadIdx.x & 63) == 0) s_acc[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) a.part[blockIdx.x] = s_acc[0] + s_acc[1] + s_acc[2] + s_acc[3];
+}
+
+__global__ void __launch_bounds__(64) k_adj_gsum(const double* __restrict__ part, int nblk, double* __restrict__ out) {
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < nblk; i += 64) acc += part[(size_t)blockIdx.x * nblk + i];
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
+  if (threadIdx.x == 0) out[blockIdx.x] += acc;
 }
 
 // d(E, c1, c2)/dL of the exact phi functions in float64: E = e^z, c1 = dt phi1(z), c2 = dt phi2(z),
@@ -405,29 +417,6 @@ __global__ void k_adj_lincomb(AdjLinArgs a) {
   }
 }
 
-// gpart (+)= w S <Xbar, sum_k s_k dc_k Y_k> per mode (w: half-spectrum weight, S = dL/dtheta)
-__global__ void k_adj_gacc(AdjGradArgs a) {
-  const size_t total = (size_t)a.B * a.C * a.modes;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-    const size_t mode = e % a.modes;
-    const size_t b = e / (a.C * a.modes);
-    const int k = (int)(mode % a.P);
-    float g = 0.f;
-    if (k < a.H) {
-      const float w = (k == 0 || 2 * k == a.nlast) ? 1.f : 2.f;
-      const float* dc = a.dcoef + b * a.dcoef_bstride + mode;
-      float2 d = make_float2(0.f, 0.f);
-      for (int t = 0; t < a.nt; ++t) {
-        const float c = a.s[t] * dc[(size_t)a.dslot[t] * a.modes];
-        const float2 y = a.Y[t][e];
-        d = make_float2(d.x + c * y.x, d.y + c * y.y);
-      }
-      g = w * a.sym[mode] * rdot(a.Xbar[e], d);
-    }
-    a.gpart[e] = a.accumulate ? a.gpart[e] + g : g;
-  }
-}
-
 static unsigned grid_of(size_t n) {
   size_t g = (n + 255) / 256;
   return (unsigned)(g > 65536 ? 65536 : (g < 1 ? 1 : g));
@@ -449,10 +438,6 @@ hipError_t launch_adj_stage(const AdjStageArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(k_adj_stage, dim3(grid_of((size_t)a.B * a.C * a.modes)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
-hipError_t launch_adj_reduce(const float* gpart, size_t per, int B, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_reduce, dim3(B), dim3(256), 0, st, gpart, per, out);
-  return hipGetLastError();
-}
 hipError_t launch_adj_dcoefs(const float* L, size_t modes, int Bc, double dt, float* dcoef, hipStream_t st) {
   hipLaunchKernelGGL(k_adj_dcoefs, dim3(grid_of(modes * Bc)), dim3(256), 0, st, L, modes, Bc, dt, dcoef);
   return hipGetLastError();
@@ -466,8 +451,15 @@ hipError_t launch_adj_lincomb(const AdjLinArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(k_adj_lincomb, dim3(grid_of((size_t)a.B * a.C * a.modes)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
-hipError_t launch_adj_gacc(const AdjGradArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_gacc, dim3(grid_of((size_t)a.B * a.C * a.modes)), dim3(256), 0, st, a);
+hipError_t launch_adj_grad(const AdjGradArgs& a, hipStream_t st) {
+  const dim3 grid(a.B * a.nblk), block(256);
+  if (a.nt == 2) hipLaunchKernelGGL(k_adj_grad<2>, grid, block, 0, st, a);        // 1-stage schemes
+  else if (a.nt == 4) hipLaunchKernelGGL(k_adj_grad<4>, grid, block, 0, st, a);   // 2-stage schemes
+  else if (a.nt == ADJ_MAXGT) hipLaunchKernelGGL(k_adj_grad<ADJ_MAXGT>, grid, block, 0, st, a);  // SETDRK4
+  else return hipErrorInvalidValue;
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_adj_gsum, dim3(a.B), dim3(64), 0, st, (const double*)a.part, a.nblk, a.out);
   return hipGetLastError();
 }
 hipError_t launch_adj_sym(const AdjArgs& a, int kind, float* S, hipStream_t st) {
