@@ -365,3 +365,26 @@ def test_default_sub_batches_equal_whole_batch(dev, term, shape, B, sb, ns):
     u1 = one.forward(u[B - 1:].contiguous())
     one.step(u1, 3)
     assert _rel(plan.inverse(uh)[B - 1:], one.inverse(u1)) <= TOL
+
+
+@pytest.mark.parametrize("n", [32, 64])
+@pytest.mark.parametrize("term,C", [("vc", 1), ("conv", 2)])
+@pytest.mark.parametrize("rate", [0.5, 2 / 3, 0.9])
+def test_persistent_2d_stepper_bands(dev, n, term, C, rate):
+    """The persistent 2D stepper with the 2/3 rule's band, a narrower and a wider one, against the tiled kernels
+    (the same arithmetic up to fused multiply-adds)."""
+    from torchfsm_amd.engine import SpectralPlan
+
+    plan = SpectralPlan([(0, 1.0, n)] * 2, 3, C, nonlinear=term, nonlinear_coef=-1.0, linear=[("lap", 0.01)],
+                        dealias_rate=rate, device=dev)
+    plan.set_scheme("SETDRK4", 1e-3)
+    g = torch.Generator(device=dev).manual_seed(n)
+    u = 0.3 * torch.randn(3, C, n, n, generator=g, device=dev)
+    assert plan.persistent
+    res = []
+    for on in (True, False):
+        plan.set_persistent(on)
+        uh = plan.forward(u)
+        plan.step(uh, 4)
+        res.append(plan.inverse(uh))
+    assert _rel(res[0], res[1]) <= 1e-6

@@ -894,8 +894,8 @@ int step_impl(tfsm_plan* p, void* uh, int nsteps, const int* rec_slot, void* tra
     Col2Args ca = col_args(p, U, (char*)ws);
     Row2Args ra = row_args(p, (char*)ws, 0, p->B);
     // k2_run has a radix plan of its own, whatever the tiled kernels' tuning
-    ca.tw0 = p->tw[0][run2d_var(p->term, p->n[0])];
-    ra.tw1 = p->tw[1][run2d_var(p->term, p->n[0])];
+    ca.tw0 = p->tw[0][RUN2D_VAR];
+    ra.tw1 = p->tw[1][RUN2D_VAR];
     Run2Args r;
     r.b0 = 0;
     r.nb = p->B;

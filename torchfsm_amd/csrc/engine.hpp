@@ -722,8 +722,8 @@ bool col2d_supported(int n0, int v, int var);
 // VorticityConvection, field pitch pf at most that of the 2/3 rule
 hipError_t launch_run2d(int term, const Col2Args& ca, const Row2Args& ra, const Run2Args& r, hipStream_t st);
 bool run2d_supported(int term, int n0, int n1, int pf);
-// its radix-plan variant (both axes)
-constexpr int run2d_var(int term, int n) { return term == TERM_VC && n == 64 ? 0 : 3; }
+// its radix-plan variant (both axes): 4 values per thread
+constexpr int RUN2D_VAR = 3;
 bool row2d_supported(int n1, int var, int wgt);
 hipError_t launch_rows_r2c(int n, const float* in, size_t in_ld, float2* out, size_t out_ld, int nrows, float scale,
                            const float2* tw, hipStream_t st);

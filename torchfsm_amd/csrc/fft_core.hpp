@@ -347,6 +347,66 @@ __device__ __forceinline__ void fft_wg(float2 (&v)[(Fft<N, VAR>::RMAX)], float2*
   if constexpr (F::NST > 4) fft_stage<N, 4, DIR, V, VAR, WS>(v, lds, tw, j, vi);
 }
 
+// K transforms at once, stage by stage, each with its own LDS region (ls slots apart): one exchange's latency
+// and synchronisation serve all K.  Same arithmetic as fft_wg.
+template <int K, int N, int S, int DIR, int V, int VAR, bool WS>
+__device__ __forceinline__ void fft_stage_k(float2 (&v)[K][(Fft<N, VAR>::RMAX)], float2* lds, int ls, const float2* tw,
+                                            int j, int vi) {
+  using F = Fft<N, VAR>;
+  constexpr int RMAX = F::RMAX;
+  constexpr int NT = F::NT;
+  constexpr int R = F::radix(S);
+  constexpr int NS = F::ns_before(S);
+  constexpr int Q = RMAX / R;
+  constexpr bool LAST = (S == F::NST - 1);
+  constexpr int TWO = F::tw_offset(S);
+  if constexpr (S > 0) {
+#pragma unroll
+    for (int l = 0; l < K; ++l)
+#pragma unroll
+      for (int m = 0; m < RMAX; ++m) v[l][m] = lds[l * ls + lds_slot<V, F::PD>(j + m * NT, vi)];
+    lds_sync<WS>();
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int jb = j + q * NT;
+    float2 w[R];
+    if constexpr (NS > 1) {
+#pragma unroll
+      for (int r = 1; r < R; ++r) w[r] = tw[TWO + r * NS + jb % NS];
+    }
+    const int idxd = (jb / NS) * NS * R + (jb % NS);
+#pragma unroll
+    for (int l = 0; l < K; ++l) {
+      float2 x[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) x[r] = v[l][q + r * Q];
+      if constexpr (NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) x[r] = (DIR < 0) ? cmul(x[r], w[r]) : cmulc(x[r], w[r]);
+      }
+      dft<R, DIR>(x);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if constexpr (LAST) v[l][q + r * Q] = x[r];
+        else lds[l * ls + lds_slot<V, F::PD>(idxd + r * NS, vi)] = x[r];
+      }
+    }
+  }
+  if constexpr (!LAST) lds_sync<WS>();
+}
+
+template <int K, int N, int DIR, int V, int VAR = 0, bool WS = false>
+__device__ __forceinline__ void fft_wg_k(float2 (&v)[K][(Fft<N, VAR>::RMAX)], float2* lds, int ls, const float2* tw,
+                                         int j, int vi) {
+  using F = Fft<N, VAR>;
+  fft_stage_k<K, N, 0, DIR, V, VAR, WS>(v, lds, ls, tw, j, vi);
+  if constexpr (F::NST > 1) fft_stage_k<K, N, 1, DIR, V, VAR, WS>(v, lds, ls, tw, j, vi);
+  if constexpr (F::NST > 2) fft_stage_k<K, N, 2, DIR, V, VAR, WS>(v, lds, ls, tw, j, vi);
+  if constexpr (F::NST > 3) fft_stage_k<K, N, 3, DIR, V, VAR, WS>(v, lds, ls, tw, j, vi);
+  if constexpr (F::NST > 4) fft_stage_k<K, N, 4, DIR, V, VAR, WS>(v, lds, ls, tw, j, vi);
+}
+
 // One Stockham stage reading the previous stage's values from `in` and writing this stage's to
 // `out` (two LDS buffers used alternately): no barrier is needed between the reads and the writes
 // of one stage, only after the writes.

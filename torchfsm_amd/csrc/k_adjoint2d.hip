@@ -15,43 +15,68 @@
 //
 // Each launch is one or two rounds of workgroups, as long as one thread's chain of transforms: 4 values
 // per thread (up to 256 points), 1 to 8 transforms.  Burgers 128^2, C = 2, B = 16, one ETDRK2 adjoint step with
-// the gradient of the viscosity: 26 launches and copies, 179 us -> 10 launches, 73 us (rows 10 and 11 us, columns
-// 4.8, 8.0 and 11.7); loading the column pass's operands before its first transform changes nothing.
+// the gradient of the viscosity: 26 launches and copies, 179 us -> 10 launches, 70 us (rows 8.9 and 9.4 us, with the
+// transforms one after the other 9.8 and 11.0; columns 4.8, 8.0 and 12.0; loading the column pass's operands before
+// its first transform changes nothing).
 #include "k_step2d.hpp"
 
 namespace tfsm {
 
-// forward row transform of two real fields (re, im) and their half spectra A, B at this lane's positions
-// (valid up to N1/2)
-template <int N1, int VAR>
-__device__ __forceinline__ void row_fwd_pair(float2 (&v)[(Fft<N1, VAR>::RMAX)], float2 (&A)[(Fft<N1, VAR>::RMAX)],
-                                             float2 (&Bv)[(Fft<N1, VAR>::RMAX)], float2* lds, const float2* s_tw, int j) {
+// K transforms: together (fft_wg_k) with 4 values per thread, otherwise one after the other
+template <int N, int VAR>
+struct Together {
+  static constexpr bool value = Fft<N, VAR>::RMAX <= 4;
+};
+template <int K, int N, int DIR, int V, int VAR, bool WS>
+__device__ __forceinline__ void fft_all(float2 (&z)[K][(Fft<N, VAR>::RMAX)], float2* lds, const float2* s_tw, int j,
+                                        int vi) {
+  if constexpr (Together<N, VAR>::value) {
+    fft_wg_k<K, N, DIR, V, VAR, WS>(z, lds, LdsSize<N, V>::slots, s_tw, j, vi);
+  } else {
+#pragma unroll
+    for (int l = 0; l < K; ++l) fft_wg<N, DIR, V, VAR, WS>(z[l], lds, s_tw, j, vi);
+  }
+}
+
+// v holds forward row transforms of pairs of real fields: their half spectra, the first of pair l in v[l], the
+// second in w[l] (this lane's positions, valid up to N1/2)
+template <int K, int N1, int VAR>
+__device__ __forceinline__ void unpack_pairs(float2 (&v)[K][(Fft<N1, VAR>::RMAX)],
+                                             float2 (&w)[K][(Fft<N1, VAR>::RMAX)], float2* lds, int j) {
   using F = Fft<N1, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
   constexpr bool WS = RowSync<N1, VAR>::WS;
-  fft_wg<N1, -1, 1, VAR, WS>(v, lds, s_tw, j, 0);
+  constexpr int KG = Together<N1, VAR>::value ? K : 1;  // pairs at once
 #pragma unroll
-  for (int m = 0; m < RMAX; ++m) lds[lds_slot<1>(j + m * NT, 0)] = v[m];
-  lds_sync<WS>();
+  for (int l0 = 0; l0 < K; l0 += KG) {
 #pragma unroll
-  for (int m = 0; m < RMAX; ++m) {
-    const int pos = j + m * NT;
-    const float2 zk = v[m];
-    const float2 zm = lds[lds_slot<1>(pos == 0 ? 0 : N1 - pos, 0)];
-    A[m] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-    const float2 d = make_float2(zk.x - zm.x, zk.y + zm.y);
-    Bv[m] = make_float2(0.5f * d.y, -0.5f * d.x);
+    for (int l = 0; l < KG; ++l)
+#pragma unroll
+      for (int m = 0; m < RMAX; ++m) lds[l * LdsSize<N1, 1>::slots + lds_slot<1>(j + m * NT, 0)] = v[l0 + l][m];
+    lds_sync<WS>();
+#pragma unroll
+    for (int l = 0; l < KG; ++l)
+#pragma unroll
+      for (int m = 0; m < RMAX; ++m) {
+        const int pos = j + m * NT;
+        const float2 zk = v[l0 + l][m];
+        const float2 zm = lds[l * LdsSize<N1, 1>::slots + lds_slot<1>(pos == 0 ? 0 : N1 - pos, 0)];
+        const float2 d = make_float2(zk.x - zm.x, zk.y + zm.y);
+        v[l0 + l][m] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
+        w[l0 + l][m] = make_float2(0.5f * d.y, -0.5f * d.x);
+      }
+    lds_sync<WS>();
   }
-  lds_sync<WS>();
 }
 
 template <int N1, int ROWS, int TERM, int VAR, bool NL>
 __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_adj_row(Adj2RowArgs a) {
   using F = Fft<N1, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
-  constexpr int SL = LdsSize<N1, 1>::slots;
   constexpr bool WS = RowSync<N1, VAR>::WS;
   constexpr int NC = Term2<TERM>::NC;
+  constexpr int KI = Term2<TERM>::KR + 1, KF = (TERM == TERM_CONV ? 3 : 2) + (NL ? 1 : 0);  // transforms in, out
+  constexpr int SL = (Together<N1, VAR>::value ? 4 : 1) * LdsSize<N1, 1>::slots;
   __shared__ float2 s_tw[F::tw_size()];
   __shared__ float2 s_buf[ROWS * SL];
   load_twiddles<N1, VAR>(s_tw, a.tw1);
@@ -64,15 +89,15 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_adj_row(Adj2RowA
   const size_t fs = (size_t)a.N0 * a.PF, ps = (size_t)a.N0 * a.P1;
   const float2* gr = a.G + (size_t)b * 4 * fs + (size_t)x * a.PF;
   const float2* pr = a.GP + (size_t)b * NC * ps + (size_t)x * a.P1;
-  float2 z1[RMAX], z2[RMAX], z3[RMAX], zp[RMAX];
+  float2 z[KI][RMAX];
 #pragma unroll
   for (int m = 0; m < RMAX; ++m) {
     const int pos = j + m * NT;
     const bool cj = pos > N1 / 2;
     const int k = cj ? N1 - pos : pos;
     const bool edge = (k == 0) || (k == N1 / 2);
-    const float2 z = make_float2(0.f, 0.f);
-    float2 f0 = z, f1 = z, f2 = z, f3 = z, p0 = z, p1 = z;
+    const float2 o = make_float2(0.f, 0.f);
+    float2 f0 = o, f1 = o, f2 = o, f3 = o, p0 = o, p1 = o;
     float ay = 0.f;
     if (rv) {
       p0 = pr[k];
@@ -85,89 +110,57 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_adj_row(Adj2RowA
       f3 = gr[3 * fs + k];
       ay = a.ay[k];
     }
-    zp[m] = pack_pair(p0, p1, cj, edge);
+    z[0][m] = pack_pair(p0, p1, cj, edge);
     if constexpr (TERM == TERM_VC) {  // fields psi, a_x psi, a_x w, w
-      z1[m] = pack_pair(make_float2(-ay * f0.y, ay * f0.x), make_float2(f1.y, -f1.x), cj, edge);   // psi_y, -psi_x
-      z2[m] = pack_pair(make_float2(-f2.y, f2.x), make_float2(-ay * f3.y, ay * f3.x), cj, edge);   // w_x, w_y
+      z[1][m] = pack_pair(make_float2(-ay * f0.y, ay * f0.x), make_float2(f1.y, -f1.x), cj, edge);  // psi_y, -psi_x
+      z[2][m] = pack_pair(make_float2(-f2.y, f2.x), make_float2(-ay * f3.y, ay * f3.x), cj, edge);  // w_x, w_y
     } else {  // u0, a_x u0, u1, a_x u1
-      z1[m] = pack_pair(f0, f2, cj, edge);
-      z2[m] = pack_pair(make_float2(-f1.y, f1.x), make_float2(-ay * f0.y, ay * f0.x), cj, edge);  // d0u0, d1u0
-      z3[m] = pack_pair(make_float2(-f3.y, f3.x), make_float2(-ay * f2.y, ay * f2.x), cj, edge);  // d0u1, d1u1
+      z[1][m] = pack_pair(f0, f2, cj, edge);
+      z[2][m] = pack_pair(make_float2(-f1.y, f1.x), make_float2(-ay * f0.y, ay * f0.x), cj, edge);  // d0u0, d1u0
+      z[3][m] = pack_pair(make_float2(-f3.y, f3.x), make_float2(-ay * f2.y, ay * f2.x), cj, edge);  // d0u1, d1u1
     }
   }
-  fft_wg<N1, +1, 1, VAR, WS>(zp, lds, s_tw, j, 0);
-  fft_wg<N1, +1, 1, VAR, WS>(z1, lds, s_tw, j, 0);
-  fft_wg<N1, +1, 1, VAR, WS>(z2, lds, s_tw, j, 0);
-  if constexpr (TERM == TERM_CONV) fft_wg<N1, +1, 1, VAR, WS>(z3, lds, s_tw, j, 0);
-  float2 v[RMAX], A[RMAX], Bv[RMAX];
+  fft_all<KI, N1, +1, 1, VAR, WS>(z, lds, s_tw, j, 0);
+  float2 v[KF][RMAX], w[KF][RMAX];
+#pragma unroll
+  for (int m = 0; m < RMAX; ++m) {
+    const float2 p = z[0][m], z1 = z[1][m], z2 = z[2][m];
+    if constexpr (TERM == TERM_VC) {
+      v[0][m] = make_float2(p.x * z2.x, p.x * z2.y);   // p w_x, p w_y
+      v[1][m] = make_float2(p.x * z1.x, -p.x * z1.y);  // p psi_y, p psi_x
+      if constexpr (NL) v[KF - 1][m] = make_float2(z1.x * z2.x + z1.y * z2.y, 0.f);
+    } else {
+      const float2 z3 = z[3][m];
+      v[0][m] = make_float2(p.x * z2.x + p.y * z3.x, p.x * z2.y + p.y * z3.y);  // R_0, R_1
+      v[1][m] = make_float2(p.x * z1.y, p.y * z1.y);                            // S_01, S_11
+      v[2][m] = make_float2(p.x * z1.x, p.y * z1.x);                            // S_00, S_10
+      if constexpr (NL) v[KF - 1][m] = make_float2(z1.x * z2.x + z1.y * z2.y, z1.x * z3.x + z1.y * z3.y);
+    }
+  }
+  fft_all<KF, N1, -1, 1, VAR, WS>(v, lds, s_tw, j, 0);
+  unpack_pairs<KF, N1, VAR>(v, w, lds, j);
+  if (!rv) return;
   float2* q = a.Q + (size_t)b * 4 * fs + (size_t)x * a.PF;
-  if constexpr (NL) {
+  float2* p = a.P + (size_t)b * NC * ps + (size_t)x * a.P1;
 #pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const float n0 = z1[m].x * z2[m].x + z1[m].y * z2[m].y;
-      float n1 = 0.f;
-      if constexpr (TERM == TERM_CONV) n1 = z1[m].x * z3[m].x + z1[m].y * z3[m].y;
-      v[m] = make_float2(n0, n1);
+  for (int m = 0; m < RMAX; ++m) {
+    const int pos = j + m * NT;
+    if (NL && pos <= N1 / 2) {
+      p[pos] = v[KF - 1][m];
+      if constexpr (NC == 2) p[ps + pos] = w[KF - 1][m];
     }
-    row_fwd_pair<N1, VAR>(v, A, Bv, lds, s_tw, j);
-    float2* p = a.P + (size_t)b * NC * ps + (size_t)x * a.P1;
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const int pos = j + m * NT;
-      if (rv && pos <= N1 / 2) {
-        p[pos] = A[m];
-        if constexpr (NC == 2) p[ps + pos] = Bv[m];
-      }
-    }
-  }
-  if constexpr (TERM == TERM_VC) {
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) v[m] = make_float2(zp[m].x * z2[m].x, zp[m].x * z2[m].y);
-    row_fwd_pair<N1, VAR>(v, A, Bv, lds, s_tw, j);
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const int pos = j + m * NT;
-      if (rv && pos <= a.kmax1) {
-        q[pos] = A[m];
-        q[fs + pos] = Bv[m];
-      }
-      v[m] = make_float2(zp[m].x * z1[m].x, -zp[m].x * z1[m].y);
-    }
-    row_fwd_pair<N1, VAR>(v, A, Bv, lds, s_tw, j);
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const int pos = j + m * NT;
-      if (rv && pos <= a.kmax1) {
-        q[2 * fs + pos] = A[m];
-        q[3 * fs + pos] = Bv[m];
-      }
-    }
-  } else {
-    float2 r0[RMAX], r1[RMAX];
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m)  // R_0, R_1
-      v[m] = make_float2(zp[m].x * z2[m].x + zp[m].y * z3[m].x, zp[m].x * z2[m].y + zp[m].y * z3[m].y);
-    row_fwd_pair<N1, VAR>(v, r0, r1, lds, s_tw, j);
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) v[m] = make_float2(zp[m].x * z1[m].y, zp[m].y * z1[m].y);  // S_01, S_11
-    row_fwd_pair<N1, VAR>(v, A, Bv, lds, s_tw, j);
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const int pos = j + m * NT;
-      if (rv && pos <= a.kmax1) {
+    if (pos <= a.kmax1) {
+      if constexpr (TERM == TERM_VC) {
+        q[pos] = v[0][m];
+        q[fs + pos] = w[0][m];
+        q[2 * fs + pos] = v[1][m];
+        q[3 * fs + pos] = w[1][m];
+      } else {
         const float ay = a.ay[pos];
-        q[pos] = make_float2(r0[m].x + ay * A[m].y, r0[m].y - ay * A[m].x);
-        q[fs + pos] = make_float2(r1[m].x + ay * Bv[m].y, r1[m].y - ay * Bv[m].x);
-      }
-      v[m] = make_float2(zp[m].x * z1[m].x, zp[m].y * z1[m].x);  // S_00, S_10
-    }
-    row_fwd_pair<N1, VAR>(v, A, Bv, lds, s_tw, j);
-#pragma unroll
-    for (int m = 0; m < RMAX; ++m) {
-      const int pos = j + m * NT;
-      if (rv && pos <= a.kmax1) {
-        q[2 * fs + pos] = A[m];
-        q[3 * fs + pos] = Bv[m];
+        q[pos] = make_float2(v[0][m].x + ay * v[1][m].y, v[0][m].y - ay * v[1][m].x);
+        q[fs + pos] = make_float2(w[0][m].x + ay * w[1][m].y, w[0][m].y - ay * w[1][m].x);
+        q[2 * fs + pos] = v[2][m];
+        q[3 * fs + pos] = w[2][m];
       }
     }
   }
@@ -178,9 +171,9 @@ template <int N0, int V, int TERM, int VAR, int MODE>
 __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_adj_col(Adj2ColArgs a) {
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
-  constexpr int NC = Term2<TERM>::NC;
+  constexpr int NC = Term2<TERM>::NC, NQ = TERM == TERM_CONV ? 2 : 4;  // channels, planes of Q per channel
   __shared__ float2 s_tw[F::tw_size()];
-  __shared__ float2 s_buf[LdsSize<N0, V>::slots];
+  __shared__ float2 s_buf[(MODE > 0 && Together<N0, VAR>::value ? NQ : 1) * LdsSize<N0, V>::slots];
   load_twiddles<N0, VAR>(s_tw, a.tw0);
   __syncthreads();
   const int vi = threadIdx.x % V, j = threadIdx.x / V;
@@ -218,7 +211,6 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_adj_col(Adj2ColArgs
   if constexpr (MODE > 0) {
     const bool kept = tile * V <= a.kmax1;  // uniform: the tile has kept columns
     const bool kc = ky <= a.kmax1;
-    constexpr int NQ = TERM == TERM_CONV ? 2 : 4;
     float2 q[NQ][RMAX];
     if (kept) {
       const float2* qb = a.Q + (size_t)b * 4 * fs + ky;
@@ -250,8 +242,7 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_adj_col(Adj2ColArgs
       }
     }
     if (kept) {
-#pragma unroll
-      for (int l = 0; l < NQ; ++l) fft_wg<N0, -1, V, VAR>(q[l], s_buf, s_tw, j, vi);
+      fft_all<NQ, N0, -1, V, VAR, false>(q, s_buf, s_tw, j, vi);
       const float ay = TERM == TERM_VC && colv ? a.ay[ky] : 0.f;
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) {

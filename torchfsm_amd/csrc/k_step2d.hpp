@@ -30,27 +30,28 @@ __device__ __forceinline__ float2 pack_pair(float2 A, float2 Bv, bool cj, bool e
   return cj ? make_float2(A.x + Bv.y, Bv.x - A.y) : make_float2(A.x - Bv.y, A.y + Bv.x);
 }
 
+// channels, fields and packed inverse row transforms (KR) of a product
 template <int TERM>
 struct Term2;
 template <>
 struct Term2<TERM_VC> {
-  static constexpr int NC = 1, NF = 4;
+  static constexpr int NC = 1, NF = 4, KR = 2;
 };
 template <>
 struct Term2<TERM_CONV> {
-  static constexpr int NC = 2, NF = 4;
+  static constexpr int NC = 2, NF = 4, KR = 3;
 };
 template <>
 struct Term2<TERM_NSP> {  // velocity-form Navier-Stokes: Convection fields, projected spectrum
-  static constexpr int NC = 2, NF = 4;
+  static constexpr int NC = 2, NF = 4, KR = 3;
 };
 template <>
 struct Term2<TERM_KS> {  // KSConvection: fields phi^, a_x phi^; one product 1/2 |grad phi|^2
-  static constexpr int NC = 1, NF = 2;
+  static constexpr int NC = 1, NF = 2, KR = 1;
 };
 template <>
 struct Term2<TERM_CONS> {  // ConservativeConvection, C = 2: fields u0, u1; product planes per
-  static constexpr int NC = 2, NF = 2;  // channel c: F_y(u0 u_c) and i a_y F_y(u1 u_c)
+  static constexpr int NC = 2, NF = 2, KR = 1;  // channel c: F_y(u0 u_c) and i a_y F_y(u1 u_c)
 };
 
 // Stage combine of one channel's column (see combine_column in engine.hpp): column base ky,
@@ -139,7 +140,7 @@ struct LdsFill {
 
 // Velocity-form Navier-Stokes (NSPressureConvection): both channels' convection spectra are
 // transformed first, projected mode by mode (nsp_project), then channel ch is combined.
-template <int N0, int V, int VAR, bool PP = false>
+template <int N0, int V, int VAR, bool PP = false, bool TOG = false>
 __device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, float2 (&s)[1][Fft<N0, VAR>::RMAX],
                                                 float2* s_buf, const float2* s_tw, int b, int ky, bool colv, int j,
                                                 int vi, int ch) {
@@ -166,8 +167,9 @@ __device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, fl
       const float2 t = a.P[((size_t)b * 2 + c) * plane + (size_t)(j + m * NT) * a.P1 + ky];
       v[c][m] = colv ? t : z;
     }
-    col_fft<N0, -1, V, VAR, PP>(v[c], s_buf, s_tw, j, vi);
+    if constexpr (!TOG) col_fft<N0, -1, V, VAR, PP>(v[c], s_buf, s_tw, j, vi);
   }
+  if constexpr (TOG) fft_wg_k<2, N0, -1, V, VAR>(v, s_buf, LdsSize<N0, V>::slots, s_tw, j, vi);
   // Nyquist-plane parity of nsp_project (N0 is even for every fused size)
   const bool nyy = 2 * ky == a.N1, zy = ky == 0;
 #pragma unroll
@@ -194,9 +196,10 @@ __device__ __forceinline__ void col_nsp_combine(const Col2Args& a, int stage, fl
 // k2_col (and of the column pass of k2_run).  ST >= 0: the stage is a compile-time constant.
 // FILL: the caller has issued the LDS twiddle and wavenumber loads (fill) and this function writes
 // them to LDS, with a barrier, right before its first LDS use; otherwise they are in LDS already.
-// CH: only channel ch (products whose channels meet in the row kernel alone: Convection).
+// CH: only channel ch (products whose channels meet in the row kernel alone: Convection).  TOG: so many
+// fields' inverse transforms together (fft_wg_k), each over its own LDS region.
 template <int N0, int V, int TERM, int VAR, int ST, bool CLAMP = false, bool FILL = false, bool PP = false,
-          bool CH = false>
+          bool CH = false, int TOG = 1>
 __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile, int b, float2* s_buf,
                                           float2* s_tw, float* s_ax, int j, int vi,
                                           const LdsFill<N0, VAR, Fft<N0, VAR>::NT * V>* fill = nullptr, int ch = 0) {
@@ -232,7 +235,7 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
   float2 s[NC][RMAX];
   if constexpr (TERM == TERM_NSP) {
     fill_lds();
-    col_nsp_combine<N0, V, VAR, PP>(a, stage, s, s_buf, s_tw, b, ky, colv, j, vi, ch);
+    col_nsp_combine<N0, V, VAR, PP, (TOG > 1)>(a, stage, s, s_buf, s_tw, b, ky, colv, j, vi, ch);
   } else {
   if constexpr (TERM == TERM_CONS) fill_lds();
 #pragma unroll
@@ -325,9 +328,8 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
   if (tile * V > a.kmax1) return;  // uniform per workgroup: no kept column in this tile
   if (stage == ST_PRO && TERM != TERM_NSP && TERM != TERM_CONS) fill_lds();  // no transform so far
   (void)ay;
-#pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    float2 v[RMAX];
+  // field f of this lane's modes
+  auto field = [&](int f, float2 (&v)[RMAX]) {
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
       const int kx = j + m * NT;
@@ -357,16 +359,35 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
       }
       v[m] = val;
     }
-    col_fft<N0, +1, V, VAR, PP>(v, s_buf, s_tw, j, vi);
+  };
+  auto store = [&](int f, const float2 (&v)[RMAX]) {
     if (ky <= a.kmax1) {  // kept columns only: the row kernel reads no other
       float2* g = a.G + (((size_t)b * NFT + (CH ? ch * NF : 0) + f) * N0) * a.PF + ky;
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.PF] = v[m];
     }
+  };
+  if constexpr (TOG > 1) {
+    static_assert(NF % TOG == 0, "whole groups of fields");
+#pragma unroll
+    for (int g = 0; g < NF; g += TOG) {
+      float2 v[TOG][RMAX];
+#pragma unroll
+      for (int f = 0; f < TOG; ++f) field(g + f, v[f]);
+      fft_wg_k<TOG, N0, +1, V, VAR>(v, s_buf, LdsSize<N0, V>::slots, s_tw, j, vi);
+#pragma unroll
+      for (int f = 0; f < TOG; ++f) store(g + f, v[f]);
+    }
+  } else {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      float2 v[RMAX];
+      field(f, v);
+      col_fft<N0, +1, V, VAR, PP>(v, s_buf, s_tw, j, vi);
+      store(f, v);
+    }
   }
 }
-
-
 
 // Channels of a product taken by different workgroups of the column kernel: those of Convection, whose
 // combine and fields need one channel only, and of NSPressureConvection, where each of the two
@@ -380,6 +401,17 @@ struct ColChannels {
   static constexpr int value = TERM == TERM_CONV || TERM == TERM_NSP ? Term2<TERM>::NC : 1;
 };
 
+// LDS regions of the tiled column kernel: one per field transformed together (plans of 4 values per thread,
+// whose launches are as long as one thread's chain of exchanges), two for ColPP.  256-point vorticity columns
+// go in pairs: four regions hold two workgroups per CU (B = 32 124 us per step against 115, B = 1 57 against 58).
+template <int N0, int V, int TERM, int VAR, int ST>
+struct ColRegions {
+  static constexpr bool PP = ColPP<N0, V, VAR>::value && ST >= 0;
+  static constexpr int NF = Term2<TERM>::NF / ColChannels<TERM>::value;
+  static constexpr int TOG = Fft<N0, VAR>::RMAX > 4 ? 1 : (N0 == 256 && NF > 2 ? 2 : NF);
+  static constexpr int value = PP ? 2 : TOG;
+};
+
 // ST >= 0: the stage is a compile-time constant (only that stage's combine is compiled, which keeps
 // the code a launch executes small); ST = -1: the stage comes at run time.
 template <int N0, int V, int TERM, int VAR, int ST = -1>
@@ -388,9 +420,10 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_col(Col2Args a, int
   using F = Fft<N0, VAR>;
   constexpr int NT = F::NT;
   // (the run-time-stage kernel keeps one buffer: the second one's addressing would make it spill)
-  constexpr bool PP = ColPP<N0, V, VAR>::value && ST >= 0;
+  using Reg = ColRegions<N0, V, TERM, VAR, ST>;
+  constexpr bool PP = Reg::PP;
   __shared__ float2 s_tw[Fft<N0, VAR>::tw_size()];
-  __shared__ float2 s_buf[(PP ? 2 : 1) * LdsSize<N0, V>::slots];
+  __shared__ float2 s_buf[Reg::value * LdsSize<N0, V>::slots];
   __shared__ float s_ax[N0];  // x wavenumbers: read per mode by the field pass without a memory wait
   // the LDS tables' loads go out first; col2_tile writes them to LDS once its own loads are issued
   LdsFill<N0, VAR, NT * V> fill;
@@ -418,8 +451,32 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_col(Col2Args a, int
   }
   const int b = a.b0 + bl / CW;
   if (a.mask.skip(b)) return;  // uniform per workgroup: this sample's steps are done
-  col2_tile<N0, V, TERM, VAR, ST, false, true, PP, (CW > 1)>(a, stage, tile, b, s_buf, s_tw, s_ax, j, vi, &fill,
-                                                             bl % CW);
+  col2_tile<N0, V, TERM, VAR, ST, false, true, PP, (CW > 1), Reg::TOG>(a, stage, tile, b, s_buf, s_tw, s_ax, j, vi,
+                                                                       &fill, bl % CW);
+}
+
+// Inverse transforms of one row's K packed fields: together (fft_wg_k) with 4 values per thread, where the
+// launch is as long as one thread's chain of exchanges, otherwise one after the other.  With the columns'
+// (ColRegions), SETDRK4 us per step: 128^2 B = 16 vorticity 58.7 -> 52.5, NavierStokes 60.3 -> 55.1, Burgers
+// 56.4 -> 53.3; 256^2 B = 1 vorticity 63.6 -> 58, NavierStokes 61.2 -> 54.8, B = 32 172 -> 143.
+template <int N1, int VAR>
+struct RowTogether {
+  static constexpr bool value = Fft<N1, VAR>::RMAX <= 4;
+};
+// LDS slots of a row that transforms K fields
+template <int N1, int VAR, int K>
+constexpr int row_slots() {
+  return (RowTogether<N1, VAR>::value ? K : 1) * LdsSize<N1, 1>::slots;
+}
+template <int K, int N1, int VAR, bool TOG>
+__device__ __forceinline__ void row_fft_k(float2 (&z)[K][(Fft<N1, VAR>::RMAX)], float2* lds, const float2* s_tw, int j) {
+  constexpr bool WS = RowSync<N1, VAR>::WS;
+  if constexpr (TOG) {
+    fft_wg_k<K, N1, +1, 1, VAR, WS>(z, lds, LdsSize<N1, 1>::slots, s_tw, j, 0);
+  } else {
+#pragma unroll
+    for (int l = 0; l < K; ++l) fft_wg<N1, +1, 1, VAR, WS>(z[l], lds, s_tw, j, 0);
+  }
 }
 
 // Row x of sample b (rv false: idle row that only takes part in the transforms' synchronisation):
@@ -429,7 +486,8 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k2_col(Col2Args a, int
 // the other up to their real products p_x, p_x+1, which then share one forward transform,
 // Z = F(p_x + i p_x+1), unpacked as F(p_x)[k] = (Z[k] + conj Z[N-k]) / 2 and
 // F(p_x+1)[k] = (Z[k] - conj Z[N-k]) / (2i): five transforms per two rows instead of six.
-template <int N1, int TERM, int VAR, bool PAIR = false>
+// TOG: the inverse transforms together, over a row region of row_slots.
+template <int N1, int TERM, int VAR, bool PAIR = false, bool TOG = RowTogether<N1, VAR>::value>
 __device__ __forceinline__ void row2_body(const Row2Args& a, int b, int x, bool rv, float2* lds, const float2* s_tw,
                                           int j) {
   using F = Fft<N1, VAR>;
@@ -447,7 +505,8 @@ __device__ __forceinline__ void row2_body(const Row2Args& a, int b, int x, bool 
 #pragma unroll 1
     for (int h = 0; h < (PAIR ? 2 : 1); ++h) {
       const float2* gr = gb + (size_t)h * a.PF;  // row x + h
-      float2 z1[RMAX], z2[RMAX];
+      float2 zz[2][RMAX];
+      auto &z1 = zz[0], &z2 = zz[1];
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) {
         const int pos = j + m * NT;
@@ -471,8 +530,7 @@ __device__ __forceinline__ void row2_body(const Row2Args& a, int b, int x, bool 
         Bv = make_float2(-ay * f3.y, ay * f3.x);
         z2[m] = pack_pair(A, Bv, cj, edge);
       }
-      fft_wg<N1, +1, 1, VAR, WS>(z1, lds, s_tw, j, 0);
-      fft_wg<N1, +1, 1, VAR, WS>(z2, lds, s_tw, j, 0);
+      row_fft_k<2, N1, VAR, TOG>(zz, lds, s_tw, j);
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) {
         const float pr = z1[m].x * z2[m].x + z1[m].y * z2[m].y;
@@ -607,7 +665,8 @@ __device__ __forceinline__ void row2_body(const Row2Args& a, int b, int x, bool 
     }
   } else {
     // Convection, C = D = 2: fields F0 = u0, F1 = kx u0, F2 = u1, F3 = kx u1 (x-inverse done)
-    float2 z1[RMAX], z2[RMAX], z3[RMAX];
+    float2 zz[3][RMAX];
+    auto &z1 = zz[0], &z2 = zz[1], &z3 = zz[2];
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
       const int pos = j + m * NT;
@@ -627,9 +686,7 @@ __device__ __forceinline__ void row2_body(const Row2Args& a, int b, int x, bool 
       z2[m] = pack_pair(make_float2(-f1.y, f1.x), make_float2(-ay * f0.y, ay * f0.x), cj, edge);  // d0u0, d1u0
       z3[m] = pack_pair(make_float2(-f3.y, f3.x), make_float2(-ay * f2.y, ay * f2.x), cj, edge);  // d0u1, d1u1
     }
-    fft_wg<N1, +1, 1, VAR, RowSync<N1, VAR>::WS>(z1, lds, s_tw, j, 0);
-    fft_wg<N1, +1, 1, VAR, RowSync<N1, VAR>::WS>(z2, lds, s_tw, j, 0);
-    fft_wg<N1, +1, 1, VAR, RowSync<N1, VAR>::WS>(z3, lds, s_tw, j, 0);
+    row_fft_k<3, N1, VAR, TOG>(zz, lds, s_tw, j);
     float2 v[RMAX];
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
@@ -673,7 +730,7 @@ template <int N1, int ROWS, int TERM, int VAR>
 __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_row(Row2Args a) {
   using F = Fft<N1, VAR>;
   constexpr int NT = F::NT;
-  constexpr int SL = LdsSize<N1, 1>::slots;
+  constexpr int SL = row_slots<N1, VAR, Term2<TERM>::KR>();
   __shared__ float2 s_tw[Fft<N1, VAR>::tw_size()];
   __shared__ float2 s_buf[ROWS * SL];
   load_twiddles<N1, VAR>(s_tw, a.tw1);
@@ -706,22 +763,29 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * ROWS)) k2_row(Row2Args a) 
 // wider than the pitch, so the column pass clamps its load column (col2_tile<..., CLAMP>).
 // (At 128^2 G and P do not fit LDS; through L2 the stepper took 160 us per SETDRK4 step against
 // 90-130 us for the tiled kernels, and 128^2 keeps them.)
-template <int N, int TERM>
+// WIDE: bands wider than the 2/3 rule's (up to its pitch rounded to 16 columns), transforms one by one.
+template <int N, int TERM, bool WIDE>
 struct Run2Shape {
-  // 4 values per thread (SETDRK4 step, us: 32^2 vorticity 34 -> 27, Convection 51 -> 34, 64^2 Convection 64
-  // -> 60), 8 for the 64-point VorticityConvection (44 against 46)
-  static constexpr int VAR = run2d_var(TERM, N);
+  // 4 values per thread, and fields transformed together: a pass is one chain of exchanges and barriers in one
+  // workgroup (SETDRK4 step, us, 8 values / 4 / 4 and together: 32^2 vorticity 34 / 27 / 25, Convection 51 / 35 /
+  // 32, 64^2 Convection 64 / 61 / 57, vorticity 44 / 46 / 42.5)
+  static constexpr int VAR = RUN2D_VAR;
   using F = Fft<N, VAR>;
   static constexpr int NT = F::NT;               // threads per transform (rows and columns)
   static constexpr int V = N;                    // one column tile holds all N/2 + 1 columns
   static constexpr int THREADS = NT * V;         // 256 (N = 32), 512 or 1024 (N = 64)
   static constexpr int ROWS = THREADS / NT;      // = N: every row in one pass
   static constexpr int PDR = F::PD < 16 ? F::PD : 16;
-  static constexpr int SLR = N + N / PDR + 1;    // LDS slots of one row (padding of lds_slot<1, PD>)
-  static constexpr int COL_SLOTS = LdsSize<N, V>::slots;
+  // fields of a row (all of them, or one by one: three regions of 64 Convection rows exceed the LDS) and of a
+  // column (pairs) transformed together
+  static constexpr bool TOG = !WIDE && (N == 32 || TERM == TERM_VC);
+  static constexpr int TOGC = WIDE ? 1 : 2;
+  static constexpr int SLR = TOG ? Term2<TERM>::KR * LdsSize<N, 1>::slots : N + N / PDR + 1;  // LDS slots of one row
+  static constexpr int COL_SLOTS = TOGC * LdsSize<N, V>::slots;
   static constexpr int SLOTS = COL_SLOTS > ROWS * SLR ? COL_SLOTS : ROWS * SLR;
   static constexpr int P1 = (N / 2 + 1 + 15) / 16 * 16;  // pitch of the half spectrum
-  static constexpr int PF = (N / 3 + 1 + 15) / 16 * 16;  // field pitch at the 2/3 rule (kmax = N/3)
+  // pitch of the fields in LDS: kmax1 + 1 <= N/3 + 1 columns at the 2/3 rule
+  static constexpr int PF = WIDE ? (N / 3 + 1 + 15) / 16 * 16 : (N / 3 + 2) / 2 * 2;
   static constexpr int NF = Term2<TERM>::NF;
   static constexpr int NP = Term2<TERM>::NC;     // product planes: VorticityConvection 1, Convection 2
   static constexpr int G_SLOTS = NF * N * PF;
@@ -729,11 +793,11 @@ struct Run2Shape {
   static_assert(ROWS == N, "every row in one pass");
 };
 
-template <int N, int TERM>
-__global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args ca, Row2Args ra, Run2Args r) {
+template <int N, int TERM, bool WIDE>
+__global__ void __launch_bounds__((Run2Shape<N, TERM, WIDE>::THREADS)) k2_run(Col2Args ca, Row2Args ra, Run2Args r) {
   static_assert(TERM == TERM_VC || TERM == TERM_CONV, "the persistent stepper's column loads are clamped for "
                                                       "Convection and VorticityConvection only");
-  using S = Run2Shape<N, TERM>;
+  using S = Run2Shape<N, TERM, WIDE>;
   constexpr int NT = S::NT, V = S::V;
   __shared__ float2 s_tw[S::F::tw_size()];
   __shared__ float2 s_buf[S::SLOTS];
@@ -757,10 +821,12 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
   c.coef += (size_t)b * ca.coef_bstride;
   if (c.src) c.src += (size_t)b * ca.src_bstride;
   c.G = s_G;
+  c.PF = S::PF;
   c.P = s_P;
   c.b0 = 0;
   Row2Args w = ra;
   w.G = s_G;
+  w.PF = S::PF;
   w.P = s_P;
   w.b0 = 0;
   // rows and columns share the plan: a square mesh with the same radix variant on both axes
@@ -788,10 +854,10 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM>::THREADS)) k2_run(Col2Args
     if (k > 0) {
       __syncthreads();  // fields G of the previous column pass (and the state) complete
       if (e == 0 && r.rec_slot) record((k - 1) / nev);
-      row2_body<N, TERM, S::VAR>(w, 0, g, true, s_buf + g * S::SLR, s_tw, jr);
+      row2_body<N, TERM, S::VAR, false, S::TOG>(w, 0, g, true, s_buf + g * S::SLR, s_tw, jr);
     }
     __syncthreads();  // products P complete; the LDS exchange buffer is reused
-    col2_tile<N, V, TERM, S::VAR, -1, true>(c, k > 0 ? scheme_stage(r.scheme, e) : ST_PRO, 0, 0, s_buf, s_tw, s_ax, jc,
+    col2_tile<N, V, TERM, S::VAR, -1, true, false, false, false, S::TOGC>(c, k > 0 ? scheme_stage(r.scheme, e) : ST_PRO, 0, 0, s_buf, s_tw, s_ax, jc,
                                        vi);
   }
   if (r.rec_slot) {
@@ -879,9 +945,11 @@ inline hipError_t launch_row_t(const Row2Args& a, hipStream_t st) {
 
 template <int N, int TERM>
 inline hipError_t launch_run_t(const Col2Args& ca, const Row2Args& ra, const Run2Args& r, hipStream_t st) {
-  // the kernel's LDS holds G at the field pitch of the 2/3 rule and P at the mesh's pitch
-  if (ca.PF > Run2Shape<N, TERM>::PF || ca.P1 != Run2Shape<N, TERM>::P1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k2_run<N, TERM>), dim3(r.nb), dim3(Run2Shape<N, TERM>::THREADS), 0, st, ca, ra, r);
+  // the kernel's LDS holds the kept columns of G, and P at the mesh's pitch
+  if (ca.kmax1 + 1 > Run2Shape<N, TERM, true>::PF || ca.P1 != Run2Shape<N, TERM, true>::P1) return hipErrorInvalidValue;
+  const dim3 grid(r.nb), block(Run2Shape<N, TERM, true>::THREADS);
+  if (ca.kmax1 + 1 > Run2Shape<N, TERM, false>::PF) hipLaunchKernelGGL((k2_run<N, TERM, true>), grid, block, 0, st, ca, ra, r);
+  else hipLaunchKernelGGL((k2_run<N, TERM, false>), grid, block, 0, st, ca, ra, r);
   return hipGetLastError();
 }
 #define TFSM_RUN_SIZES(X) X(32) X(64)
