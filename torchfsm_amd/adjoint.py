@@ -5,7 +5,8 @@ of every step (_base.py:676-751 with integrator.step, _etdrk.py:72-82, _setdrk_s
 Here the forward pass runs the fused engine and keeps the spectral state every `every` steps
 (checkpoints).  The backward pass walks the segments in reverse: it recomputes the states of one
 segment from its checkpoint and applies tfsm_adjoint_step to each, from the last step back.
-Memory: ceil(steps / every) + every states, instead of the reference's whole graph.
+Memory: ceil(steps / every) + every states, instead of the reference's whole graph (every state, and none
+recomputed, while all of them are small: OperatorLike._integrate_with_adjoint).
 
 Supported: Convection in 1D, 2D and 3D (e.g. Burgers) and VorticityConvection in 2D (e.g.
 NavierStokesVorticity, with explicit sources such as kolm_force), with ETDRK1/2, SETDRK1/2 and
@@ -84,8 +85,8 @@ class IntegrateAdjoint(torch.autograd.Function):
         grad = torch.zeros(plan.batch, dtype=torch.float64, device=plan.device) if want_theta else None
         out = torch.empty_like(ub)
         for _, n, ck in reversed(ctx.ckpts):
-            states = [ck.clone()]
-            u = ck.clone()
+            states = [ck]  # (adjoint_step only reads them)
+            u = ck.clone() if n > 1 else ck
             for _ in range(n - 1):
                 plan.step(u, 1)
                 states.append(u.clone())
