@@ -35,6 +35,13 @@ __device__ __forceinline__ int ky_compress(int ky, int N1, int kmax1) {
   return -1;
 }
 
+// Columns of 4 values per thread run a thread's transforms together (fft_wg_k): NavierStokes SETDRK4 64^3 B = 2
+// 168 -> 158 us per step, 32^3 B = 1 88 -> 82, B = 16 177 -> 165.  Not 256 points: three regions are 104 KB.
+template <int N, int VAR>
+struct Col3Together {
+  static constexpr bool value = Fft<N, VAR>::RMAX <= 4 && N <= 128;
+};
+
 // ---------------------------------------------------------------- x columns (fused combine)
 // Fields f0 = u^_c and f0 + 1 = a_x u^_c of one channel's combined spectrum s (kept modes, scaled),
 // inverse x FFT, stored to G1 at the compressed ky index kyc.
@@ -44,9 +51,7 @@ __device__ __forceinline__ void col3_fields(const Col3Args& a, const float2 (&s)
                                             const float* s_ax, int j, int vi) {
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    float2 v[RMAX];
+  auto field = [&](int h, float2 (&v)[RMAX]) {
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
       const int kx = j + m * NT;
@@ -65,11 +70,28 @@ __device__ __forceinline__ void col3_fields(const Col3Args& a, const float2 (&s)
       }
       v[m] = val;
     }
-    fft_wg<N0, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+  };
+  auto store = [&](int h, const float2 (&v)[RMAX]) {
     if (kz < a.PF2) {
       float2* g = a.G1 + ((((size_t)b * 2 * nc + f0 + h) * N0) * a.K1 + kyc) * a.PF2 + kz;
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.K1 * a.PF2] = v[m];
+    }
+  };
+  if constexpr (Col3Together<N0, VAR>::value) {
+    float2 v[2][RMAX];
+    field(0, v[0]);
+    field(1, v[1]);
+    fft_wg_k<2, N0, +1, V, VAR>(v, s_buf, LdsSize<N0, V>::slots, s_tw, j, vi);
+    store(0, v[0]);
+    store(1, v[1]);
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float2 v[RMAX];
+      field(h, v);
+      fft_wg<N0, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+      store(h, v);
     }
   }
 }
@@ -99,7 +121,8 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k3_col(Col3Args a, int
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
   __shared__ float2 s_tw[Fft<N0, VAR>::tw_size()];
-  __shared__ float2 s_buf[LdsSize<N0, V>::slots];
+  constexpr int REG = Col3Together<N0, VAR>::value ? (TERM == TERM_NSP ? 3 : 2) : 1;
+  __shared__ float2 s_buf[REG * LdsSize<N0, V>::slots];
   __shared__ float s_ax[N0];  // x wavenumbers: read per mode by the field pass without a memory wait
   load_twiddles<N0, VAR>(s_tw, a.tw0);
   for (int i = threadIdx.x; i < N0; i += NT * V) s_ax[i] = a.ax[i];
@@ -155,8 +178,9 @@ __global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k3_col(Col3Args a, int
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       load(a.P, c, v3[c]);
-      fft_wg<N0, -1, V, VAR>(v3[c], s_buf, s_tw, j, vi);
+      if constexpr (REG == 1) fft_wg<N0, -1, V, VAR>(v3[c], s_buf, s_tw, j, vi);
     }
+    if constexpr (REG == 3) fft_wg_k<3, N0, -1, V, VAR>(v3, s_buf, LdsSize<N0, V>::slots, s_tw, j, vi);
     const float ayv = a.ay[ky], azv = colv ? a.az[kz] : 0.f;
     // Nyquist-plane parity of nsp_project (every fused 3D size is even)
     const bool nyy = 2 * ky == a.N1, nyz = 2 * kz == a.N2, oyz = (ky == 0 || nyy) && (kz == 0 || nyz);
@@ -199,7 +223,7 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * V)) k3_yinv(Yinv3Args a) {
   using F = Fft<N1, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
   __shared__ float2 s_tw[Fft<N1, VAR>::tw_size()];
-  __shared__ float2 s_buf[LdsSize<N1, V>::slots];
+  __shared__ float2 s_buf[(Col3Together<N1, VAR>::value ? 3 : 1) * LdsSize<N1, V>::slots];
   load_twiddles<N1, VAR>(s_tw, a.tw1);
   __syncthreads();
   const int vi = threadIdx.x % V, j = threadIdx.x / V;
@@ -223,9 +247,7 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * V)) k3_yinv(Yinv3Args a) {
     f0[m] = ld ? g0[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
     f1[m] = ld ? g1[(size_t)kc * a.PF2] : make_float2(0.f, 0.f);
   }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    float2 v[RMAX];
+  auto field = [&](int k, float2 (&v)[RMAX]) {
 #pragma unroll
     for (int m = 0; m < RMAX; ++m) {
       if (k == 0) v[m] = f0[m];
@@ -235,11 +257,28 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * V)) k3_yinv(Yinv3Args a) {
         v[m] = make_float2(mulr(ay, f0[m].x), mulr(ay, f0[m].y));
       }
     }
-    fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+  };
+  auto store = [&](int k, const float2 (&v)[RMAX]) {
     if (kz < a.PF2) {
       float2* g = a.G2 + ((((size_t)b * 3 * NCH + 3 * c + k) * a.N0 + x) * N1) * a.PF2 + kz;
 #pragma unroll
       for (int m = 0; m < RMAX; ++m) g[(size_t)(j + m * NT) * a.PF2] = v[m];
+    }
+  };
+  if constexpr (Col3Together<N1, VAR>::value) {
+    float2 v[3][RMAX];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) field(k, v[k]);
+    fft_wg_k<3, N1, +1, V, VAR>(v, s_buf, LdsSize<N1, V>::slots, s_tw, j, vi);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) store(k, v[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      float2 v[RMAX];
+      field(k, v);
+      fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+      store(k, v);
     }
   }
 }
