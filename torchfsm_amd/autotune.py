@@ -87,6 +87,10 @@ def autotune(plan, uh, steps=6, log=None, cache_file: Optional[str] = None, fina
     """Pick and apply the fastest launch shape for this plan; returns (tuning, {tuning: ms})."""
     if plan.general:  # the unfused path has no launch shape to choose
         return plan.tuning, {}
+    try:
+        plan.set_tuning(*plan.tuning)
+    except ValueError:  # nor have the long 1D meshes' kernels
+        return plan.tuning, {}
     key = shape_key(plan)
     if cache_file and os.path.exists(cache_file) and key not in _CACHE:
         try:

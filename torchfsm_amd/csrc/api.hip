@@ -1821,7 +1821,8 @@ int64_t tfsm_plan_inverse_scratch_bytes(const tfsm_plan* plan, int32_t nbatch) {
 int tfsm_plan_set_tuning(tfsm_plan* plan, int32_t col_tile, int32_t col_var, int32_t row_var, int32_t row_wg,
                          int32_t sub_batch) {
   if (!plan) return fail(TFSM_E_INVALID, "null plan");
-  if (!plan->fused_ok || plan->l1) return fail(TFSM_E_INVALID, "no fused kernels for this plan: it has no launch shape");
+  if (plan->l1) return fail(TFSM_E_INVALID, "the kernels of long 1D meshes have no launch shape");
+  if (!plan->fused_ok) return fail(TFSM_E_INVALID, "no fixed-size fused kernels for this plan: it has no launch shape");
   if (plan->D == 3 && (row_var < 0 || row_var > 1 || col_var < 0 || col_var > 1))
     return fail(TFSM_E_INVALID, "unsupported 3D tuning");
   if (plan->D == 3 && (col_var == 1 || row_var == 1) &&
