@@ -164,13 +164,20 @@ int tfsm_plan_set_persistent(tfsm_plan* plan, int32_t on);
 int32_t tfsm_plan_persistent(const tfsm_plan* plan);
 
 /* Step through the unfused path (on = 1: separate field, product, transform and stage launches)
- * or the fused kernels (on = 0, TFSM_E_INVALID where none cover the plan).  Plans the fused
- * kernels do not cover start on the unfused path.  Switching grows or shrinks
- * tfsm_plan_workspace_bytes.  (No reference counterpart: choice of kernels.) */
+ * or the fused kernels the plan started with (on = 0, TFSM_E_INVALID where none cover the plan: it
+ * then starts on the unfused path).  Switching changes tfsm_plan_workspace_bytes.
+ * (No reference counterpart: choice of kernels.) */
 int tfsm_plan_set_general(tfsm_plan* plan, int32_t on);
 
-/* 1 if tfsm_step runs the unfused path for this plan, else 0. */
+/* 1 if the fixed-size fused kernels do not step this plan: its mesh or terms have none, or
+ * set_general(1).  It then steps on the run-time-length kernels or unfused (tfsm_plan_path). */
 int32_t tfsm_plan_general(const tfsm_plan* plan);
+
+/* What tfsm_step runs for this plan: fixed-size fused kernels, those of long 1D meshes, fused kernels
+ * of run-time lengths, the unfused path, or linear steps only (no product term).
+ * (No reference counterpart: choice of kernels.) */
+enum { TFSM_PATH_LINEAR = 0, TFSM_PATH_FIXED = 1, TFSM_PATH_LONG1D = 2, TFSM_PATH_RUNTIME = 3, TFSM_PATH_UNFUSED = 4 };
+int32_t tfsm_plan_path(const tfsm_plan* plan);
 
 /* ETD coefficients on the device: SETDRK1-4 as float64 contour means of n_points points on a
  * circle of radius `radius`; ETDRK0-2 with the reference's complex64 closed forms.

@@ -52,3 +52,54 @@ def test_autotune_leaves_long_1d_plans_alone(dev, n):
     assert torch.equal(a, b)
     with pytest.raises(ValueError, match="launch shape"):
         plan.set_tuning(*before)
+
+
+RUNTIME = [("vc", (30, 42), 3), ("conv", (64, 67), 2), ("nsp", (67, 64), 2), ("ks", (48, 60), 2), ("ks_keep_mean", (17, 30), 1),
+           ("conv", (1000,), 2), ("cons", (97,), 3)]
+
+
+@pytest.mark.parametrize("kind,shape,batch", RUNTIME)
+def test_run_time_lengths_against_the_unfused_path(dev, kind, shape, batch):
+    """set_general(True) takes a plan off the run-time-length kernels and set_general(False) puts it back: steps and
+    a single evaluation agree, and the first ones come back bit for bit."""
+    plan = _plan(kind, shape, batch, dev)
+    assert plan.path == "runtime" and plan.general
+    plan.set_scheme("SETDRK4", 1e-3)
+    u = _smooth(plan, dev, sum(shape))
+    h = shape[-1] // 2 + 1
+    res = []
+    for on in (False, True, False):
+        plan.set_general(on)
+        assert plan.path == ("unfused" if on else "runtime") and plan.general
+        uh = plan.forward(u)
+        ev = torch.view_as_real(plan.apply(uh)[..., :h])
+        plan.step(uh, 4)
+        res.append((plan.inverse(uh), ev))
+    assert _rel(res[0][0], res[1][0]) <= TOL and _rel(res[0][1], res[1][1]) <= TOL
+    assert torch.equal(res[0][0], res[2][0]) and torch.equal(res[0][1], res[2][1])
+
+
+@pytest.mark.parametrize("kind,shape,path", [("conv", (256,), "fixed"), ("conv", (8192,), "long1d"), ("vc", (64, 64), "fixed"),
+                                             ("nsp", (32, 32, 32), "fixed"), ("conv", (40, 40, 40), "unfused"),
+                                             ("ks", (1000,), "unfused"), (None, (30, 30), "linear")])
+def test_plan_path(dev, kind, shape, path):
+    """The kernels a plan starts on; a plan with fused ones goes to the unfused path and back."""
+    plan = _plan(kind, shape, 2, dev)
+    assert plan.path == path and plan.general == (path == "unfused")
+    if path == "unfused":
+        with pytest.raises(ValueError):
+            plan.set_general(False)
+    elif path != "linear":
+        plan.set_general(True)
+        assert plan.path == "unfused" and plan.general
+        plan.set_general(False)
+        assert plan.path == path and not plan.general
+
+
+def test_force_takes_a_run_time_length_plan_to_the_unfused_path(dev):
+    plan = _plan("nsp", (30, 34), 2, dev)
+    assert plan.path == "runtime"
+    plan.add_force(torch.ones(1, 2, 30, 34, device=dev), 0.1)
+    assert plan.path == "unfused"
+    with pytest.raises(ValueError):
+        plan.set_general(False)

@@ -68,6 +68,7 @@ SIGNATURES = {
     "tfsm_plan_persistent": (I32, [VP]),
     "tfsm_plan_set_general": (ctypes.c_int, [VP, I32]),
     "tfsm_plan_general": (I32, [VP]),
+    "tfsm_plan_path": (I32, [VP]),
     "tfsm_plan_get_tuning": (ctypes.c_int, [VP, VP]),
     "tfsm_plan_set_scheme": (ctypes.c_int, [VP, I32, ctypes.c_double, I32, ctypes.c_double, VP]),
     "tfsm_plan_coefficients": (ctypes.c_int, [VP, I32, VP, VP]),

@@ -85,7 +85,7 @@ def time_steps_sustained(plan, uh, steps=200) -> float:
 
 def autotune(plan, uh, steps=6, log=None, cache_file: Optional[str] = None, final_steps: int = 200):
     """Pick and apply the fastest launch shape for this plan; returns (tuning, {tuning: ms})."""
-    if plan.general:  # the unfused path has no launch shape to choose
+    if plan.general:  # neither the unfused path nor the run-time-length kernels have a launch shape to choose
         return plan.tuning, {}
     try:
         plan.set_tuning(*plan.tuning)

@@ -156,7 +156,7 @@ struct tfsm_plan {
   int adj_term = -2;       // linear term whose coefficient gets a gradient (-1 none; -2 not prepared)
   int adj_scheme = -1;
   // unfused path (k_general.hip): stepping without the fused kernels
-  bool general = false;    // the plan steps through the unfused path
+  bool general = false;    // no fixed-size fused kernels step the plan (genf: those of run-time lengths; else unfused)
   bool fused_ok = false;   // the fused kernels cover this plan (the unfused path is then optional)
   GAxis gax[3];            // general-length FFT tables of the axes without fixed-size kernels
   float2* gtmp = nullptr;  // four-step scratch of those axes
@@ -164,7 +164,8 @@ struct tfsm_plan {
   int forceB = 0, forceC = 0;
   // general plans that step on the fused kernels of run-time lengths (k_genfused.hip): 2D (gf_row, gf_col: that
   // axis takes the run-time kernel, the other one its fixed-size kernel) or the persistent 1D stepper
-  bool genf = false, gf_row = false, gf_col = false;
+  // (genf: taken now; genf_ok: the plan has them, set_general(1) leaves them aside)
+  bool genf = false, genf_ok = false, gf_row = false, gf_col = false;
   size_t ws_fused = 0;     // workspace of the fused path (the unfused buffers follow it)
   size_t off_gS = 0, off_gF = 0, off_gR = 0, off_gQ = 0;
 
@@ -457,7 +458,7 @@ int build_gaxes(tfsm_plan* p) {
 int plan_genfused(tfsm_plan* p) {
   if (p->cplx || p->force) return TFSM_OK;
   if (p->D == 1) {
-    p->genf = (p->term == TERM_CONV || p->term == TERM_CONS) && p->C == 1 && genfused_axis(p->gax[0]);
+    p->genf = p->genf_ok = (p->term == TERM_CONV || p->term == TERM_CONS) && p->C == 1 && genfused_axis(p->gax[0]);
     return TFSM_OK;
   }
   if (p->D != 2 || p->term == TERM_CONS) return TFSM_OK;
@@ -473,7 +474,7 @@ int plan_genfused(tfsm_plan* p) {
     }
     if (!genfused_axis(p->gax[d])) return TFSM_OK;
   }
-  p->genf = true;
+  p->genf = p->genf_ok = true;
   p->gf_col = gen[0];
   p->gf_row = gen[1];
   p->NF = p->term == TERM_KS ? 2 : 4;
@@ -1856,7 +1857,7 @@ int tfsm_plan_get_tuning(const tfsm_plan* plan, int32_t* out) {
 
 int tfsm_plan_set_persistent(tfsm_plan* plan, int32_t on) {
   if (!plan) return fail(TFSM_E_INVALID, "null plan");
-  if (on && plan->general) return fail(TFSM_E_INVALID, "the plan steps through the unfused path");
+  if (on && plan->general) return fail(TFSM_E_INVALID, "the plan has no fixed-size fused kernels, or set_general(1)");
   if (on && !(plan->D == 2 && run2d_supported(plan->term, plan->n[0], plan->n[1], plan->PF) && !plan->cplx))
     return fail(TFSM_E_INVALID, "the persistent 2D stepper covers square 32^2 and 64^2 meshes with Convection or "
                                 "VorticityConvection (2/3 dealiasing or coarser)");
@@ -1871,7 +1872,13 @@ int tfsm_plan_set_general(tfsm_plan* plan, int32_t on) {
   if (on) {
     if (plan->term == TERM_NONE) return fail(TFSM_E_INVALID, "a plan without a product term has no nonlinear evaluation");
     plan->general = true;
+    plan->genf = false;
     plan->persistent = false;
+    gen_layout(plan);
+    return TFSM_OK;
+  }
+  if (plan->genf_ok) {
+    plan->genf = true;
     gen_layout(plan);
     return TFSM_OK;
   }
@@ -1882,6 +1889,12 @@ int tfsm_plan_set_general(tfsm_plan* plan, int32_t on) {
 }
 
 int32_t tfsm_plan_general(const tfsm_plan* plan) { return plan && plan->general ? 1 : 0; }
+
+int32_t tfsm_plan_path(const tfsm_plan* plan) {
+  if (!plan || plan->term == TERM_NONE) return TFSM_PATH_LINEAR;
+  if (plan->general) return plan->genf ? TFSM_PATH_RUNTIME : TFSM_PATH_UNFUSED;
+  return plan->l1 ? TFSM_PATH_LONG1D : TFSM_PATH_FIXED;
+}
 
 int tfsm_plan_set_streams(tfsm_plan* plan, int32_t nstreams) {
   if (!plan) return fail(TFSM_E_INVALID, "null plan");
@@ -2190,7 +2203,7 @@ int tfsm_plan_add_force(tfsm_plan* p, const float* force, int32_t force_batch, i
   p->persistent = false;
   if (!p->general || p->genf) {
     p->general = true;
-    p->genf = p->gf_row = p->gf_col = false;
+    p->genf = p->genf_ok = p->gf_row = p->gf_col = false;
     gen_layout(p);
   }
   return TFSM_OK;
@@ -2365,7 +2378,7 @@ int tfsm_solve(tfsm_plan* p, const void* uh, void* out, void* stream) {
 
 int tfsm_launch_pass(tfsm_plan* p, void* uh, void* ws, int32_t pass_id, int32_t stage, int32_t sub, void* stream) {
   if (!p || !uh || !ws) return fail(TFSM_E_INVALID, "null argument");
-  if (p->general) return fail(TFSM_E_INVALID, "the plan steps through the unfused path: no fused passes");
+  if (p->general) return fail(TFSM_E_INVALID, "the plan has no fixed-size fused passes");
   hipStream_t st = (hipStream_t)stream;
   // the launches cover sub-batch `sub`, exactly as tfsm_step launches them
   const int sb = (p->sub_batch > 0 && p->sub_batch < p->B) ? p->sub_batch : p->B;

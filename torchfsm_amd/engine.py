@@ -184,12 +184,21 @@ class SpectralPlan:
 
     @property
     def general(self) -> bool:
-        """True when stepping runs the unfused path (separate field, product, transform and stage
-        launches): meshes and terms the fused kernels do not cover, or set_general(True)."""
+        """True when the fixed-size fused kernels do not step the plan: its mesh or terms have none, or
+        set_general(True).  `path` tells what does."""
         return bool(lib.tfsm_plan_general(self._plan))
 
+    PATHS = ("linear", "fixed", "long1d", "runtime", "unfused")
+
+    @property
+    def path(self) -> str:
+        """What stepping runs: fused kernels of "fixed" lengths, of "long1d" meshes or of "runtime" lengths, the
+        "unfused" path (separate field, product, transform and stage launches), or "linear" steps only."""
+        return self.PATHS[lib.tfsm_plan_path(self._plan)]
+
     def set_general(self, on: bool):
-        """Unfused path (True) or the fused kernels (False, where they cover the plan)."""
+        """Unfused path (True) or the fused kernels the plan started with (False; ValueError where none cover
+        it)."""
         self._drop_step_graph()
         check(lib.tfsm_plan_set_general(self._plan, 1 if on else 0), "general")
         ws = int(lib.tfsm_plan_workspace_bytes(self._plan))
