@@ -103,3 +103,24 @@ def test_force_takes_a_run_time_length_plan_to_the_unfused_path(dev):
     assert plan.path == "unfused"
     with pytest.raises(ValueError):
         plan.set_general(False)
+
+
+@pytest.mark.parametrize("kind,scheme", [("conv", "SETDRK4"), ("cons", "SETDRK3")])
+@pytest.mark.parametrize("n,path", [(2049, "unfused"), (2045, "runtime"), (3745, "unfused"), (3750, "runtime"), (3888, "runtime"),
+                                    (4000, "runtime"), (4095, "runtime"), (4097, "unfused")])
+def test_1d_stepper_up_to_4096_points(dev, kind, scheme, n, path):
+    """The persistent 1D stepper takes every mesh whose FFT length (the mesh's own, or Bluestein's) is at most 4096,
+    with its state in global memory where LDS does not hold it: against the unfused path."""
+    plan = _plan(kind, (n,), 2, dev)
+    assert plan.path == path
+    plan.set_scheme(scheme, 0.1 / n)
+    u = _smooth(plan, dev, n)
+    res = []
+    for on in (False, True):
+        if path == "runtime":
+            plan.set_general(on)
+        uh = plan.forward(u)
+        ev = plan.apply(uh)[..., : n // 2 + 1]
+        plan.step(uh, 4)
+        res.append((plan.inverse(uh), torch.view_as_real(ev)))
+    assert _rel(res[0][0], res[1][0]) <= TOL and _rel(res[0][1], res[1][1]) <= TOL

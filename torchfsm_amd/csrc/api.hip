@@ -458,7 +458,7 @@ int build_gaxes(tfsm_plan* p) {
 int plan_genfused(tfsm_plan* p) {
   if (p->cplx || p->force) return TFSM_OK;
   if (p->D == 1) {
-    p->genf = p->genf_ok = (p->term == TERM_CONV || p->term == TERM_CONS) && p->C == 1 && genfused_axis(p->gax[0]);
+    p->genf = p->genf_ok = (p->term == TERM_CONV || p->term == TERM_CONS) && p->C == 1 && genfused_mesh1d(p->gax[0]);
     return TFSM_OK;
   }
   if (p->D != 2 || p->term == TERM_CONS) return TFSM_OK;

@@ -67,8 +67,9 @@ hipError_t gfft_run(const GAxis& a, int mode, int dir, const void* in, const GLi
 struct Col2Args;
 struct Row2Args;
 struct Run1Args;
-// fused kernels of run-time lengths (k_genfused.hip): whether an axis fits them, and their launches
+// fused kernels of run-time lengths (k_genfused.hip): whether a 2D axis or a 1D mesh fits them, and their launches
 bool genfused_axis(const GAxis& ax);
+bool genfused_mesh1d(const GAxis& ax);
 hipError_t launch_g2col(int term, const Col2Args& a, const GAxis& ax, int nb, int stage, hipStream_t st);
 hipError_t launch_g2row(int term, const Row2Args& a, const GAxis& ax, hipStream_t st);
 hipError_t launch_g1run(const Run1Args& a, const GAxis& ax, hipStream_t st);

@@ -614,8 +614,13 @@ GxDev gx_dev(const GAxis& ax, const GxShape& s) {
 
 }  // namespace
 
+// an axis of the 2D passes (two product planes and the wavenumbers beside the buffers), and the 1D stepper's mesh
+// (the stage spectrum beside them: smooth lengths up to 4096)
 bool genfused_axis(const GAxis& ax) {
   return ax.n > 1 && !ax.four && ax.g.L > 1 && lds_bytes(ax, 1, 1, 2, ax.n, false) <= GF_LDS;
+}
+bool genfused_mesh1d(const GAxis& ax) {
+  return ax.n > 1 && !ax.four && ax.g.L > 1 && lds_bytes(ax, 1, 1, 0, (size_t)ax.n / 2 + 1, false) <= GF_LDS;
 }
 
 #define GF_LAUNCH(K, T, ...)                                                            \
