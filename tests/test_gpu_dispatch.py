@@ -124,3 +124,22 @@ def test_1d_stepper_up_to_4096_points(dev, kind, scheme, n, path):
         plan.step(uh, 4)
         res.append((plan.inverse(uh), torch.view_as_real(ev)))
     assert _rel(res[0][0], res[1][0]) <= TOL and _rel(res[0][1], res[1][1]) <= TOL
+
+
+@pytest.mark.parametrize("n", [97, 1000, 4000])
+def test_integrate_on_the_1d_stepper_takes_no_graph(dev, n):
+    """The run-time-length 1D stepper runs every step of integrate() in one launch: no graph of 16 steps is captured
+    around it, and the steps are those of one plan.step call."""
+    import torchfsm_amd as tfa
+    from torchfsm_amd import pde
+
+    op = pde.Burgers(0.01)
+    op.register_mesh(tfa.MeshGrid([(0, 1, n)], device=dev), 1)
+    plan = op._prepare(2, dev, 0.1 / n)
+    assert plan.path == "runtime"
+    u = _smooth(plan, dev, n)
+    out = op.integrate(u, dt=0.1 / n, step=40)
+    assert getattr(plan, "_step_graph", None) is None
+    uh = plan.forward(u)
+    plan.step(uh, 40)
+    assert torch.equal(out, plan.inverse(uh))
