@@ -143,3 +143,40 @@ def test_integrate_on_the_1d_stepper_takes_no_graph(dev, n):
     uh = plan.forward(u)
     plan.step(uh, 40)
     assert torch.equal(out, plan.inverse(uh))
+
+
+@pytest.mark.parametrize("kind,shape,batch,sub,streams", [
+    # narrow meshes: a sub-batch holds about 2M points (one channel of 512 and 1024 points 4M), never a few samples
+    ("conv", (1024, 16), 64, 0, 1), ("conv", (1024, 48), 64, 32, 2), ("nsp", (1024, 48), 32, 0, 1), ("nsp", (1024, 256), 64, 8, 2),
+    ("conv", (512, 48), 64, 0, 1), ("nsp", (512, 64), 128, 64, 2), ("vc", (512, 48), 64, 0, 1), ("vc", (512, 64), 256, 128, 2),
+    ("ks_keep_mean", (512, 128), 64, 0, 1), ("vc", (1024, 256), 64, 16, 2),
+    # ConservativeConvection has two channels
+    ("cons", (512, 48), 64, 0, 1), ("cons", (512, 512), 32, 8, 2), ("cons", (1024, 64), 32, 0, 1), ("cons", (1024, 1024), 8, 2, 2),
+    # square ones
+    ("conv", (512, 512), 32, 16, 2), ("nsp", (512, 1024), 32, 16, 2), ("vc", (512, 512), 64, 16, 2), ("vc", (512, 512), 16, 0, 1),
+    ("conv", (1024, 1024), 8, 4, 2), ("nsp", (1024, 1024), 4, 0, 1), ("vc", (1024, 1024), 8, 0, 1),
+    # nothing to overlap: the batch mean couples the samples, or there is no product term
+    ("ks", (512, 512), 64, 0, 1), (None, (256, 256), 64, 0, 1)])
+def test_2d_sub_batches(dev, kind, shape, batch, sub, streams):
+    """The sub-batches and streams a 2D plan starts with."""
+    plan = _plan(kind, shape, batch, dev)
+    assert (plan.tuning[4], plan.streams) == (sub, streams)
+
+
+@pytest.mark.parametrize("kind,shape,batch", [("conv", (1024, 48), 65), ("cons", (512, 64), 257), ("vc", (512, 64), 257)])
+def test_narrow_sub_batches_equal_the_whole_batch(dev, kind, shape, batch):
+    """The sub-batches of narrow meshes, a shorter last one among them, against one launch over the whole batch: the
+    same kernels, so equal bit for bit."""
+    plan = _plan(kind, shape, batch, dev)
+    assert 0 < plan.tuning[4] < batch and batch % plan.tuning[4] and plan.streams == 2
+    plan.set_scheme("SETDRK4", 1e-4)
+    u = _smooth(plan, dev, batch)
+    res = []
+    for whole in (False, True):
+        if whole:
+            plan.set_tuning(*plan.tuning[:4], 0)
+            plan.set_streams(1)
+        uh = plan.forward(u)
+        plan.step(uh, 3)
+        res.append(plan.inverse(uh))
+    assert torch.equal(res[0], res[1])

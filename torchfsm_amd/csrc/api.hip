@@ -1719,26 +1719,39 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     // shorten the launches (SETDRK4, us per step, one stream / whole batch / two streams: vorticity 128^2
     // B = 256 382 / 184 / 157, 100^2 B = 256 401 / 229 / 228; Burgers 128^2 B = 256 378 / 263 / 221;
     // NavierStokes 256^2 B = 64 338 / 286 / 255).  Other lines where sweeps drew them:
-    const bool pair = term == TERM_CONV || term == TERM_NSP;
-    const size_t pts = (size_t)p->B * n0 * n1, sub_pts = (size_t)1 << 21;
+    const bool pair = term == TERM_CONV || term == TERM_NSP, one = term == TERM_VC || term == TERM_KS;
+    const int B = p->B;
+    const size_t pt = (size_t)n0 * n1, pts = (size_t)B * pt, sub_pts = (size_t)1 << 21;
     int sub = 0, ns = 2;
     if (pts >= sub_pts) {
       const int parts = pts / sub_pts > 2 ? (int)(pts / sub_pts) : 2;
-      sub = (p->B + parts - 1) / parts;
+      sub = (B + parts - 1) / parts;
     }
-    // 512-point one-channel columns: 16 samples (512^2 B = 64: 603 us, against 651 for 32 and 666 for 32 on one
-    // stream; B = 16 as a whole 178, in halves 186); two-channel ones: 16 from B = 32
-    if (n0 == 512 && !pair) sub = p->B >= 32 ? 16 : 0;
-    if (n0 == 512 && pair && p->B >= 32) sub = 16;
-    // 1024-point columns: two-channel products by 4 from B = 8 (Burgers ETDRK2 342 -> 313 us; one channel, or
-    // fewer samples, no gain)
-    if (n0 == 1024) sub = pair && p->B >= 8 ? 4 : 0;
+    // samples of `of` points in all, and no split below two such sub-batches
+    auto of_points = [&](size_t of, int least) {
+      const int lim = (int)(of / pt) > least ? (int)(of / pt) : least;
+      return B >= 2 * lim ? lim : 0;
+    };
+    // 512-point columns.  One channel: 4M points, 16 samples at least (vorticity 512^2 B = 64 614 us, 721 by 2M and
+    // 717 whole; 512 x 64 B = 64 136 whole, 151 in halves; 512 x 128 B = 256 661, 705 by 2M).  Two channels on
+    // rows of 512 points or more: 16 samples from B = 32 (Burgers 512^2 505 us, 555 by 2M; 512 x 256 the reverse)
+    if (n0 == 512 && one) sub = of_points((size_t)1 << 22, 16);
+    if (n0 == 512 && pair && n1 >= 512 && B >= 32) sub = 16;
+    // 1024-point columns.  Two channels on rows of 512 points or more: 4M points (Burgers 1024^2 B = 8 650 us, 840
+    // by 2M; 1024 x 512 B = 16 594, 651 by 2M; 1024 x 256 B = 64 1264 by 2M, 1312).  One channel: 4M points on
+    // shorter rows, 8M on these (vorticity 1024 x 256 B = 64 835 us, 920 whole; 1024^2 B = 16 875, 894 whole,
+    // 1085 by 4M)
+    if (n0 == 1024 && pair && n1 >= 512) sub = of_points((size_t)1 << 22, 1);
+    if (n0 == 1024 && one) sub = of_points((size_t)1 << (n1 < 512 ? 22 : 23), 1);
+    // ConservativeConvection: from 4M points (512^2 B = 32 547 us, 714 whole; 1024 x 256 B = 8, 2M points: 256, 243)
+    if (n0 >= 512 && term == TERM_CONS && pts < 2 * sub_pts) sub = 0;
     // 256^2 up to 95 samples: 16 samples on two streams, on four from B = 48 (Burgers B = 48: 233 -> 180 us)
     if (n0 == 256 && n1 == 256 && term != TERM_NSP && p->B >= 32 && p->B < 96) {
       sub = 16;
       ns = p->B >= 48 ? 4 : 2;
     }
-    if (sub > 0 && sub < p->B && !p->ks_mean && !p->genf) {
+    // (a plan without a product term steps in one elementwise launch)
+    if (sub > 0 && sub < p->B && !p->ks_mean && !p->genf && term != TERM_NONE) {
       p->sub_batch = sub;
       rc = tfsm_plan_set_streams(p, ns);
     }
