@@ -155,6 +155,9 @@ def test_integrate_on_the_1d_stepper_takes_no_graph(dev, n):
     # square ones
     ("conv", (512, 512), 32, 16, 2), ("nsp", (512, 1024), 32, 16, 2), ("vc", (512, 512), 64, 16, 2), ("vc", (512, 512), 16, 0, 1),
     ("conv", (1024, 1024), 8, 4, 2), ("nsp", (1024, 1024), 4, 0, 1), ("vc", (1024, 1024), 8, 0, 1),
+    # KSConvection and long columns of ConservativeConvection from 4M points
+    ("ks_keep_mean", (256, 256), 32, 0, 1), ("ks_keep_mean", (256, 1024), 16, 8, 2), ("cons", (256, 1024), 8, 0, 1),
+    ("cons", (256, 256), 32, 16, 2), ("cons", (128, 1024), 16, 8, 2),
     # nothing to overlap: the batch mean couples the samples, or there is no product term
     ("ks", (512, 512), 64, 0, 1), (None, (256, 256), 64, 0, 1)])
 def test_2d_sub_batches(dev, kind, shape, batch, sub, streams):
@@ -180,3 +183,25 @@ def test_narrow_sub_batches_equal_the_whole_batch(dev, kind, shape, batch):
         plan.step(uh, 3)
         res.append(plan.inverse(uh))
     assert torch.equal(res[0], res[1])
+
+
+@pytest.mark.parametrize("kind", ["ks", "ks_keep_mean", "cons"])
+@pytest.mark.parametrize("shape,batch", [((64, 16), 3), ((128, 48), 2), ((256, 64), 2), ((256, 256), 1)])
+def test_stage_kernels_of_ks_and_conservative_convection(dev, kind, shape, batch):
+    """The column kernels compiled per stage, of 4 values per thread, with a source: every evaluation of the two- and
+    four-stage schemes, the field pass and a single evaluation, against the unfused path."""
+    plan = _plan(kind, shape, batch, dev)
+    assert plan.path == "fixed" and plan.tuning[1] == 1
+    u = _smooth(plan, dev, sum(shape))
+    plan.add_source(u[:1].roll(3, -1).contiguous(), 0.2)
+    h = shape[-1] // 2 + 1
+    for scheme in ("SETDRK2", "ETDRK2", "SETDRK3", "SETDRK4"):
+        plan.set_scheme(scheme, 1e-3)
+        res = []
+        for on in (False, True):
+            plan.set_general(on)
+            uh = plan.forward(u)
+            ev = torch.view_as_real(plan.apply(uh)[..., :h])
+            plan.step(uh, 3)
+            res.append((plan.inverse(uh), ev))
+        assert _rel(res[0][0], res[1][0]) <= TOL and _rel(res[0][1], res[1][1]) <= TOL

@@ -1743,10 +1743,14 @@ int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* s
     // 1085 by 4M)
     if (n0 == 1024 && pair && n1 >= 512) sub = of_points((size_t)1 << 22, 1);
     if (n0 == 1024 && one) sub = of_points((size_t)1 << (n1 < 512 ? 22 : 23), 1);
-    // ConservativeConvection: from 4M points (512^2 B = 32 547 us, 714 whole; 1024 x 256 B = 8, 2M points: 256, 243)
-    if (n0 >= 512 && term == TERM_CONS && pts < 2 * sub_pts) sub = 0;
+    // ConservativeConvection on long columns: from 4M points (512^2 B = 32 547 us, 714 whole; at 2M points 1024 x 256
+    // B = 8 256, 243 whole; 256 x 1024 B = 8 202, 190; 128 x 1024 B = 16 the reverse, 154, 161)
+    if (n0 >= 256 && term == TERM_CONS && pts < 2 * sub_pts) sub = 0;
+    // KSConvection, with two fields instead of four: from 4M points (256 x 1024 B = 8, 2M points: 123 us, 112 whole;
+    // 128^2 B = 128 104, 93; at 4M points 135, 143 whole)
+    if (term == TERM_KS && pts < 2 * sub_pts) sub = 0;
     // 256^2 up to 95 samples: 16 samples on two streams, on four from B = 48 (Burgers B = 48: 233 -> 180 us)
-    if (n0 == 256 && n1 == 256 && term != TERM_NSP && p->B >= 32 && p->B < 96) {
+    if (n0 == 256 && n1 == 256 && term != TERM_NSP && p->B >= (term == TERM_KS ? 64 : 32) && p->B < 96) {
       sub = 16;
       ns = p->B >= 48 ? 4 : 2;
     }

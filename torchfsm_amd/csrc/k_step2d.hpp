@@ -319,7 +319,10 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
         if (a.dc && ky == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
       }
       const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)(CH ? ch : c) * a.src_cstride : nullptr;
-      combine_column2<N0, VAR, (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : 4, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
+      // (two channels in a plan of 4 values: with batches of 4 modes SETDRK4's third evaluation, which loads the
+      // most, holds 147 VGPRs and one 512-thread workgroup per CU: ConservativeConvection 256^2 B = 16 134 -> 127 us)
+      constexpr int BM = (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : (NC > 1 && ST == ST_R4_E2 ? 2 : 4);
+      combine_column2<N0, VAR, BM, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
                                                                                   cko, kl, colv, j, v, s[c], rs,
                                                                                   &pre);
     }
@@ -874,11 +877,11 @@ __global__ void __launch_bounds__((Run2Shape<N, TERM, WIDE>::THREADS)) k2_run(Co
 // state): the 512-point VorticityConvection columns of the Navier-Stokes workloads with 8 values per
 // thread (13-16 KB of code instead of 21 KB, 87-128 VGPRs; with 16 values per thread the stage kernels
 // need 133-164 VGPRs, occupancy 3, and the run-time-stage kernel is kept), and the plans of 4 values
-// per thread, whose short launches spend much of their time in the run-time switch.
+// per thread, whose short launches spend much of their time in the run-time switch (KSConvection 256 x 1024
+// B = 32, SETDRK4: 331 us per step with it, 304 without; 315 with 8 values per thread and the switch).
 template <int N0, int V, int TERM, int VAR>
 struct ColStageKernels {
-  static constexpr bool terms = TERM == TERM_VC || TERM == TERM_CONV || TERM == TERM_NSP;
-  static constexpr bool value = (TERM == TERM_VC && N0 == 512 && VAR == 0) || (terms && VAR == 3);
+  static constexpr bool value = (TERM == TERM_VC && N0 == 512 && VAR == 0) || VAR == 3;
 };
 
 template <int N0, int V, int TERM, int VAR>
