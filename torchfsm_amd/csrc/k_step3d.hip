@@ -114,9 +114,10 @@ struct Col3Channels {
 // ST >= 0: the stage is a compile-time constant (only that stage's combine is compiled, which
 // lowers the register count: 128-point Convection columns 193 -> 133 / 148 VGPRs for ETDRK2's
 // evaluations, three waves per SIMD instead of two); ST = -1: the stage comes at run time.
-// (Holding the stage kernels to 128 VGPRs, four waves, spills a few values and measured slower.)
+// (Holding the stage kernels to 128 VGPRs, four waves, spills a few values and measured slower; at 96 points, where
+// Convection and KSConvection need 129, it spills none: KSConvection 96^3 B = 8 53 -> 47 us per launch.)
 template <int N0, int V, int VAR, int TERM, int ST = -1>
-__global__ void __launch_bounds__((Fft<N0, VAR>::NT * V)) k3_col(Col3Args a, int stage_rt) {
+__global__ void __launch_bounds__((Fft<N0, VAR>::NT * V), (N0 == 96 && TERM != TERM_NSP ? 4 : 1)) k3_col(Col3Args a, int stage_rt) {
   const int stage = ST >= 0 ? ST : stage_rt;
   using F = Fft<N0, VAR>;
   constexpr int RMAX = F::RMAX, NT = F::NT;
@@ -273,13 +274,17 @@ __global__ void __launch_bounds__((Fft<N1, VAR>::NT * V)) k3_yinv(Yinv3Args a) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) store(k, v[k]);
   } else {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float2 v[RMAX];
-      field(k, v);
-      fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
-      store(k, v);
-    }
+    // the second and third field where the first two were loaded (with a copy of each 138 VGPRs at 96 points instead
+    // of 119, one wave per SIMD fewer; 101 instead of 89 at 64)
+    float2 v[RMAX];
+    field(0, v);
+    fft_wg<N1, +1, V, VAR>(v, s_buf, s_tw, j, vi);
+    store(0, v);
+    field(1, f0);
+    fft_wg<N1, +1, V, VAR>(f0, s_buf, s_tw, j, vi);
+    store(1, f0);
+    fft_wg<N1, +1, V, VAR>(f1, s_buf, s_tw, j, vi);
+    store(2, f1);
   }
 }
 
