@@ -1,7 +1,7 @@
 // General-length batched FFTs for the axes the fixed-size kernels do not cover (mesh.py:481-491
 // transforms any length).  A length n that factors into 2, 3, 5, 7, 11 and 13 runs a Stockham FFT with
 // run-time radices 2..16 in one workgroup's LDS (gx_core.hpp); any other n runs Bluestein's algorithm, a
-// circular convolution of the cheapest such length M >= 2n - 1.  Transforms longer than GFFT_LDS_MAX points
+// circular convolution of length M >= 2n - 1 (2^a, 5 2^a or 15 2^a).  Transforms longer than GFFT_LDS_MAX points
 // split L = L1 * L2 into two LDS passes (four-step: L1-point FFTs, twiddles, L2-point FFTs; Bluestein's
 // M is then a power of two).
 //
