@@ -222,3 +222,19 @@ def test_precision_of_transforms_of_any_length(dev):
         ref = np.fft.rfft(u.double().numpy())
         total += float(np.linalg.norm(got - ref) ** 2 / np.linalg.norm(ref) ** 2)
     assert (total / len(ns)) ** 0.5 <= 1.575e-7
+
+
+@pytest.mark.parametrize("shape,batch", [((23,), 1), ((500,), 64), ((1015,), 300), ((2039,), 1), ((2039,), 300), ((4095,), 1), ((4095,), 300),
+                                         ((1017, 9), 2), ((9, 1017), 2), ((17, 1031), 40), ((2050, 34), 1), ((6, 1015, 5), 3)])
+def test_general_transforms_by_launch_shape(dev, shape, batch):
+    """General-length transforms there and back with few workgroups (more threads, tables in LDS) and many (two
+    workgroups per CU), short and long lines, rows and strided columns, against numpy in float64."""
+    import numpy as np
+
+    plan = _plan(None, shape, batch, dev)
+    u = torch.randn(batch, 1, *shape, generator=torch.Generator().manual_seed(sum(shape) + batch))
+    uh = plan.forward(u.to(dev))
+    got = uh[..., : shape[-1] // 2 + 1].cpu().to(torch.complex128).numpy()
+    ref = np.fft.rfftn(u.double().numpy(), axes=tuple(range(2, 2 + len(shape))))
+    assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) <= 1e-6
+    assert _rel(plan.inverse(uh).cpu(), u) <= 1e-6

@@ -59,7 +59,7 @@ __device__ __forceinline__ float2 gtw(const float2* tw, int t, int dir) {
   return dir < 0 ? w : make_float2(w.x, -w.y);
 }
 
-__global__ void __launch_bounds__(512) k_gfft(GLaunch a) {
+__global__ void __launch_bounds__(1024) k_gfft(GLaunch a) {
   extern __shared__ float2 g_lds[];
   const int L = a.g.L, nth = blockDim.x, tid = threadIdx.x;
   GxLines ln;
@@ -174,6 +174,7 @@ __global__ void __launch_bounds__(512) k_gfft(GLaunch a) {
 }
 
 constexpr size_t GX_LDS_BYTES = 150 * 1024;  // of 160 KB
+constexpr size_t GX_LDS_PAIR = 80 * 1024;    // two workgroups per CU
 
 hipError_t launch_g(GLaunch a, hipStream_t st) {
   const long long nlines = a.n_o * a.n_i * a.n_s;
@@ -183,10 +184,16 @@ hipError_t launch_g(GLaunch a, hipStream_t st) {
   const long long din = a.fd == 2 ? a.qs * a.ies : (a.fd == 1 ? a.iis : a.ios);
   const long long dout = a.fd == 2 ? a.rs * a.oes : (a.fd == 1 ? a.ois : a.oos);
   const bool adj = din == 1 || dout == 1;
-  // lines per workgroup: about 4096 points, 16 lines at most; fewer while the launch has under two
-  // workgroups per CU (but 8 where adjacent lines share cache lines)
+  // lines per workgroup: about 4096 points, 16 lines at most, and two workgroups per CU (2048 points two lines at a
+  // time, one workgroup per CU: 1015 points B = 2048 155 us there and back, 112 one line at a time); fewer while the
+  // launch has under two workgroups per CU (but 8 where adjacent lines share cache lines)
+  auto lds_of = [&](int v, bool tables) {
+    return (2 * (size_t)gx_slots(a.g.L, 1 << v) + (tables ? a.g.L : 0)) * sizeof(float2);
+  };
   int vl = 0;
-  while (a.g.L > 1 && vl < 4 && ((long long)a.g.L << (vl + 1)) <= GFFT_LDS_MAX && (1 << vl) < nf) ++vl;
+  while (a.g.L > 1 && vl < 4 && ((long long)a.g.L << (vl + 1)) <= GFFT_LDS_MAX && (1 << vl) < nf &&
+         lds_of(vl + 1, true) <= GX_LDS_PAIR)
+    ++vl;
   const int least = adj ? 3 : 0;
   while (vl > least && outer * ((nf + (1 << vl) - 1) >> vl) < 512) --vl;
   a.vl = vl;
@@ -195,12 +202,15 @@ hipError_t launch_g(GLaunch a, hipStream_t st) {
   a.mgL = (unsigned)((0x100000000ULL + a.g.L - 1) / a.g.L);
   const long long blocks = outer * ((nf + (1 << vl) - 1) >> vl);
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t buf = (size_t)gx_slots(a.g.L, 1 << vl) * sizeof(float2);
-  a.twlds = 2 * buf + a.g.L * sizeof(float2) <= GX_LDS_BYTES ? 1 : 0;
-  const size_t lds = 2 * buf + (a.twlds ? a.g.L * sizeof(float2) : 0);
-  // one butterfly of about 8 values per thread
-  long long nth = ((((long long)a.g.L << vl) / 8 + 63) / 64) * 64;
-  nth = nth < 64 ? 64 : (nth > 512 ? 512 : nth);
+  a.twlds = lds_of(vl, true) <= (blocks > 256 ? GX_LDS_PAIR : GX_LDS_BYTES) ? 1 : 0;
+  const size_t lds = lds_of(vl, a.twlds);
+  // one butterfly of about 4 values per thread, so that a stage is one round of butterflies (with 8 values radices 4
+  // to 6 took two: 500^2 B = 1 there and back 52 us against 42, 57 x 246 57 against 43, 1D 496 points B = 64 35 against
+  // 29), of 2 where a CU has one workgroup at most (unfused KSConvection 1000 points 117 us per step against 112), and
+  // 1024 threads only there (505 x 576 B = 1 55 us against 61; B = 32 the reverse, 1.07)
+  const long long most = blocks > 256 ? 512 : 1024;
+  long long nth = ((((long long)a.g.L << vl) / (blocks > 256 ? 4 : 2) + 63) / 64) * 64;
+  nth = nth < 64 ? 64 : (nth > most ? most : nth);
   hipLaunchKernelGGL(k_gfft, dim3((unsigned)blocks), dim3((unsigned)nth), lds, st, a);
   return hipGetLastError();
 }
