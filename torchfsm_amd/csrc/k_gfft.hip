@@ -215,12 +215,15 @@ hipError_t launch_g(GLaunch a, hipStream_t st) {
   return hipGetLastError();
 }
 
+// (`extra` per stage: Bluestein's sequences take fewer, longer stages, 400 more each: two transforms and the chirps
+// between them make a stage dearer there.  Vorticity 993 x 64 B = 1 SETDRK4 2606 us for 8 steps against 2350, 1D Burgers
+// 767 points 709 against 650, conv 787 x 96 3302 against 2934; errors within 1 %.)
 // The cheapest radix sequence by the time of one butterfly per thread, in cycles: a stage's barrier and LDS
 // latency, plus its LDS traffic, twiddles and index arithmetic (64 per value) and its arithmetic.  The
 // launches that matter are latency bound, so a few stages of radix 4 to 9 beat fewer of radix 15 and 16.
 constexpr int kRadices[] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 15, 16};
 constexpr int kStageCost[] = {670, 760, 820, 1020, 1110, 1350, 1270, 1550, 1720, 2100, 1850, 2500, 2560, 2300};
-void plan_radices(int n, int i, int cost, std::vector<int>& now, std::vector<int>& best, int& bestc) {
+void plan_radices(int n, int i, int cost, int extra, std::vector<int>& now, std::vector<int>& best, int& bestc) {
   if (!best.empty() && cost >= bestc) return;
   if (n == 1) {
     best = now;
@@ -230,18 +233,18 @@ void plan_radices(int n, int i, int cost, std::vector<int>& now, std::vector<int
   for (int k = i; k >= 0; --k)
     if (n % kRadices[k] == 0) {
       now.push_back(kRadices[k]);
-      plan_radices(n / kRadices[k], k, cost + kStageCost[k], now, best, bestc);
+      plan_radices(n / kRadices[k], k, cost + kStageCost[k] + extra, extra, now, best, bestc);
       now.pop_back();
     }
 }
 
-bool radices(int L, GRadix& g) {
+bool radices(int L, GRadix& g, int extra) {
   g = GRadix();
   g.L = L;
   std::vector<int> now, best;
   if (L > 1) {
     int bestc = 0;
-    plan_radices(L, (int)(sizeof(kRadices) / sizeof(int)) - 1, 0, now, best, bestc);
+    plan_radices(L, (int)(sizeof(kRadices) / sizeof(int)) - 1, 0, extra, now, best, bestc);
     if (best.empty() || (int)best.size() > GFFT_MAX_RADICES) return false;
   }
   int ns = 1;
@@ -291,8 +294,8 @@ hipError_t upload(const std::vector<float2>& h, const float2** out, std::vector<
   return e;
 }
 
-hipError_t build_radix(GRadix& g, int L, std::vector<void*>& allocs) {
-  if (!radices(L, g)) return hipErrorInvalidValue;
+hipError_t build_radix(GRadix& g, int L, std::vector<void*>& allocs, int extra = 0) {
+  if (!radices(L, g, extra)) return hipErrorInvalidValue;
   std::vector<float2> h(L);
   for (int t = 0; t < L; ++t) {
     const double ang = -2.0 * M_PI * (double)t / (double)L;
@@ -352,7 +355,7 @@ hipError_t gaxis_build(GAxis& a, int n, std::vector<void*>& allocs) {
   }
   hipError_t e;
   if (a.L <= GFFT_LDS_MAX) {
-    e = build_radix(a.g, a.L, allocs);
+    e = build_radix(a.g, a.L, allocs, a.blu ? 400 : 0);
   } else {
     a.four = true;
     const int l1 = split_four(a.L);
