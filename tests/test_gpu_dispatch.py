@@ -238,3 +238,23 @@ def test_general_transforms_by_launch_shape(dev, shape, batch):
     ref = np.fft.rfftn(u.double().numpy(), axes=tuple(range(2, 2 + len(shape))))
     assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) <= 1e-6
     assert _rel(plan.inverse(uh).cpu(), u) <= 1e-6
+
+
+@pytest.mark.parametrize("kind,shape,batch,path", [("conv", (509, 64), 1, "runtime"), ("nsp", (993, 40), 1, "runtime"), ("vc", (1000, 48), 2, "runtime"),
+                                                   ("ks", (787, 20), 1, "runtime"), ("vc", (2039, 32), 1, "runtime"), ("conv", (2039, 32), 1, "unfused"),
+                                                   ("nsp", (2039, 32), 3, "unfused"), ("conv", (2039, 32), 4, "runtime"), ("conv", (127, 126), 4, "runtime")])
+def test_2d_run_time_lengths_with_few_columns(dev, kind, shape, batch, path):
+    """Meshes with fewer than 64 workgroups' worth of columns, one column and several fields per workgroup, and the long
+    ones that step unfused: against the unfused path."""
+    plan = _plan(kind, shape, batch, dev)
+    assert plan.path == path
+    plan.set_scheme("SETDRK4", 0.02 / max(shape))
+    u = _smooth(plan, dev, sum(shape))
+    res = []
+    for on in (False, True):
+        if path == "runtime":
+            plan.set_general(on)
+        uh = plan.forward(u)
+        plan.step(uh, 3)
+        res.append(plan.inverse(uh))
+    assert _rel(res[0], res[1]) <= TOL and bool(torch.isfinite(res[0]).all())

@@ -474,6 +474,11 @@ int plan_genfused(tfsm_plan* p) {
     }
     if (!genfused_axis(p->gax[d])) return TFSM_OK;
   }
+  // a few columns of over 2048 points of a two-channel product, whose six fields LDS holds one at a time: the unfused
+  // launches spread them (2039 x 32, 8 SETDRK4 steps, us, unfused / fused: Burgers B = 1 3830 / 4256, B = 2 4157 / 4332,
+  // B = 4 4756 / 4445; vorticity B = 1 3676 / 3383)
+  const bool two = p->term == TERM_CONV || p->term == TERM_NSP;
+  if (gen[0] && two && p->gax[0].g.L > 2048 && (size_t)p->H * p->B < 64) return TFSM_OK;
   p->genf = p->genf_ok = true;
   p->gf_col = gen[0];
   p->gf_row = gen[1];

@@ -583,8 +583,12 @@ struct GxShape {
 
 // nfield transforms of `lines` lines: all fields at once if LDS holds them, as many lines as 8192 points in
 // flight allow (16 at most), but no fewer than `least` (adjacent columns share cache lines) unless LDS forces
-// it, and otherwise few enough for two workgroups per CU; about 4 values per thread
+// it, and otherwise few enough for two workgroups per CU; about 4 values per thread.  Where that would leave fewer
+// than 64 workgroups they take single lines with more fields at once (8 SETDRK4 steps, us, B = 1: 509 x 64 Burgers 2587
+// -> 1185, vorticity 2163 -> 987, where the unfused path takes 1940 and 1861; 993 x 256 vorticity 2505 -> 1820; a line of
+// 256 workgroups instead of 64 costs 500^2 B = 4 half again)
 GxShape choose(const GAxis& ax, size_t lines, int nfield, int least, int extra, size_t fixed) {
+  if (lines / least < 64) least = 1;
   GxShape s;
   auto fits = [&](int V, int fg) { return lds_bytes(ax, V, fg, extra, fixed, true) <= GF_LDS; };
   s.fg = nfield;
