@@ -185,17 +185,17 @@ def test_narrow_sub_batches_equal_the_whole_batch(dev, kind, shape, batch):
     assert torch.equal(res[0], res[1])
 
 
-@pytest.mark.parametrize("kind", ["ks", "ks_keep_mean", "cons"])
+@pytest.mark.parametrize("kind", ["ks", "ks_keep_mean", "cons", "vc", "conv", "nsp"])
 @pytest.mark.parametrize("shape,batch", [((64, 16), 3), ((128, 48), 2), ((256, 64), 2), ((256, 256), 1)])
-def test_stage_kernels_of_ks_and_conservative_convection(dev, kind, shape, batch):
-    """The column kernels compiled per stage, of 4 values per thread, with a source: every evaluation of the two- and
-    four-stage schemes, the field pass and a single evaluation, against the unfused path."""
+def test_stage_kernels_of_four_values_per_thread(dev, kind, shape, batch):
+    """The column kernels compiled per stage, of 4 values per thread, with a source: every evaluation of every
+    scheme, the field pass and a single evaluation, against the unfused path."""
     plan = _plan(kind, shape, batch, dev)
     assert plan.path == "fixed" and plan.tuning[1] == 1
     u = _smooth(plan, dev, sum(shape))
     plan.add_source(u[:1].roll(3, -1).contiguous(), 0.2)
     h = shape[-1] // 2 + 1
-    for scheme in ("SETDRK2", "ETDRK2", "SETDRK3", "SETDRK4"):
+    for scheme in ("ETDRK1", "SETDRK1", "SETDRK2", "ETDRK2", "SETDRK3", "SETDRK4"):
         plan.set_scheme(scheme, 1e-3)
         res = []
         for on in (False, True):

@@ -319,9 +319,9 @@ __device__ __forceinline__ void col2_tile(const Col2Args& a, int stage, int tile
         if (a.dc && ky == 0 && j == 0) v[0] = rsub(v[0], a.dc[0]);
       }
       const float2* src = a.src ? a.src + (size_t)b * a.src_bstride + (size_t)(CH ? ch : c) * a.src_cstride : nullptr;
-      // (two channels in a plan of 4 values: with batches of 4 modes SETDRK4's third evaluation, which loads the
-      // most, holds 147 VGPRs and one 512-thread workgroup per CU: ConservativeConvection 256^2 B = 16 134 -> 127 us)
-      constexpr int BM = (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : (NC > 1 && ST == ST_R4_E2 ? 2 : 4);
+      // (two channels in a plan of 4 values: with batches of 4 modes the third evaluations, which load the most, hold
+      // 147 VGPRs and one 512-thread workgroup per CU: ConservativeConvection 256^2 B = 16, SETDRK4 134 -> 127 us)
+      constexpr int BM = (RMAX > 4 && (NC > 1 || RMAX >= 16)) ? 1 : (NC > 1 && (ST == ST_R4_E2 || ST == ST_R3_E2) ? 2 : 4);
       combine_column2<N0, VAR, BM, (ST >= 0), PRE>(a, stage, base, src, cpk, c5b, tb,
                                                                                   cko, kl, colv, j, v, s[c], rs,
                                                                                   &pre);
@@ -895,8 +895,12 @@ inline hipError_t launch_col_t(const Col2Args& a, int nb, int stage, hipStream_t
   if constexpr (ColStageKernels<N0, V, TERM, VAR>::value) {
     if constexpr (VAR == 3) {
       switch (stage) {
+        TFSM_COL_STAGE(ST_R1_E0)
         TFSM_COL_STAGE(ST_R2_E0)
         TFSM_COL_STAGE(ST_R2_E1)
+        TFSM_COL_STAGE(ST_R3_E0)
+        TFSM_COL_STAGE(ST_R3_E1)
+        TFSM_COL_STAGE(ST_R3_E2)
         TFSM_COL_STAGE(ST_EVAL)
         default: break;
       }
