@@ -273,7 +273,11 @@ __global__ void __launch_bounds__(256) k_adj_grad(AdjGradArgs a) {
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
   if ((threadIdx.x & 63) == 0) s_acc[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) a.part[blockIdx.x] = s_acc[0] + s_acc[1] + s_acc[2] + s_acc[3];
+  if (threadIdx.x == 0) {
+    const double g = s_acc[0] + s_acc[1] + s_acc[2] + s_acc[3];
+    if (a.nblk == 1) a.out[b] += g;
+    else a.part[blockIdx.x] = g;
+  }
 }
 
 __global__ void __launch_bounds__(64) k_adj_gsum(const double* __restrict__ part, int nblk, double* __restrict__ out) {
@@ -451,14 +455,18 @@ hipError_t launch_adj_lincomb(const AdjLinArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(k_adj_lincomb, dim3(grid_of((size_t)a.B * a.C * a.modes)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
-hipError_t launch_adj_grad(const AdjGradArgs& a, hipStream_t st) {
+hipError_t launch_adj_grad(const AdjGradArgs& args, hipStream_t st) {
+  // few terms: one workgroup per sample and no second launch (one ETDRK1 step back, us: 1D 64 points B = 9
+  // 35.7 -> 32.8, 1024 points 36.5 -> 34.8; 64^2 vorticity the reverse, 25.1 -> 28.8)
+  AdjGradArgs a = args;
+  if ((size_t)a.nt * a.C * a.modes <= 2048) a.nblk = 1;
   const dim3 grid(a.B * a.nblk), block(256);
   if (a.nt == 2) hipLaunchKernelGGL(k_adj_grad<2>, grid, block, 0, st, a);        // 1-stage schemes
   else if (a.nt == 4) hipLaunchKernelGGL(k_adj_grad<4>, grid, block, 0, st, a);   // 2-stage schemes
   else if (a.nt == ADJ_MAXGT) hipLaunchKernelGGL(k_adj_grad<ADJ_MAXGT>, grid, block, 0, st, a);  // SETDRK4
   else return hipErrorInvalidValue;
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || a.nblk == 1) return e;
   hipLaunchKernelGGL(k_adj_gsum, dim3(a.B), dim3(64), 0, st, (const double*)a.part, a.nblk, a.out);
   return hipGetLastError();
 }
