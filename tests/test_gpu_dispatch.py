@@ -242,7 +242,8 @@ def test_general_transforms_by_launch_shape(dev, shape, batch):
 
 @pytest.mark.parametrize("kind,shape,batch,path", [("conv", (509, 64), 1, "runtime"), ("nsp", (993, 40), 1, "runtime"), ("vc", (1000, 48), 2, "runtime"),
                                                    ("ks", (787, 20), 1, "runtime"), ("vc", (2039, 32), 1, "runtime"), ("conv", (2039, 32), 1, "unfused"),
-                                                   ("nsp", (2039, 32), 3, "unfused"), ("conv", (2039, 32), 4, "runtime"), ("conv", (127, 126), 4, "runtime")])
+                                                   ("nsp", (2039, 32), 3, "unfused"), ("conv", (2039, 32), 4, "runtime"), ("vc", (112, 37), 2, "runtime"),
+                                                   ("nsp", (200, 30), 1, "runtime"), ("conv", (100, 301), 1, "runtime"), ("ks", (100, 37), 60, "runtime"), ("conv", (127, 126), 4, "runtime")])
 def test_2d_run_time_lengths_with_few_columns(dev, kind, shape, batch, path):
     """Meshes with fewer than 64 workgroups' worth of columns, one column and several fields per workgroup, and the long
     ones that step unfused: against the unfused path."""

@@ -464,7 +464,13 @@ int plan_genfused(tfsm_plan* p) {
   if (p->D != 2 || p->term == TERM_CONS) return TFSM_OK;
   // fixed-size columns address whole pitch rows of the y wavenumber table (16 points at least); the paired
   // 512-point vorticity rows need an even number of rows per sample
-  bool gen[2] = {!col2d_supported(p->n[0], 8, 0) || p->n[1] < 16,
+  // where the rows are not of a fixed length: columns of 100, 112 and 200 points, whose fixed-size plans hold 16 and 20
+  // values per thread (k2_col 112 points, 19 columns 28 us a launch), up to 1024 columns (vorticity SETDRK4 against the
+  // unfused path, 112 points, B = 1, 4, 16, 64: fixed 0.97, 0.78, 0.62, 0.52, run-time 0.51, 0.42, 0.40, 0.44; Burgers
+  // at B = 64 the reverse, 0.48, 0.48; an ETDRK2 step back, B = 1: 1.09, 0.74; 48, 96 and 192 points need no such rule)
+  const bool slow_cols = (p->n[0] == 100 || p->n[0] == 112 || p->n[0] == 200) && (size_t)p->H * p->B <= 1024 &&
+                         !row2d_supported(p->n[1], 0, 256);
+  bool gen[2] = {!col2d_supported(p->n[0], 8, 0) || p->n[1] < 16 || slow_cols,
                  !row2d_supported(p->n[1], 0, 256) || (p->n[1] == 512 && p->n[0] % 2 != 0)};
   for (int d = 0; d < 2; ++d) {
     if (!gen[d]) continue;
