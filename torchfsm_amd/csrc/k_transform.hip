@@ -606,27 +606,35 @@ static constexpr int rows_per_wg() {
   return Fft<N>::NT >= 256 ? 1 : 256 / Fft<N>::NT;
 }
 
-#define TFSM_SWITCH_N(n, BODY)  \
+// lengths up to 512 points (rows and strided columns), and the longer ones (rows only)
+#define TFSM_CASES_512(...) \
+    case 16: { constexpr int NN = 16; __VA_ARGS__; } \
+    case 32: { constexpr int NN = 32; __VA_ARGS__; } \
+    case 64: { constexpr int NN = 64; __VA_ARGS__; } \
+    case 128: { constexpr int NN = 128; __VA_ARGS__; } \
+    case 256: { constexpr int NN = 256; __VA_ARGS__; } \
+    case 512: { constexpr int NN = 512; __VA_ARGS__; } \
+    case 48: { constexpr int NN = 48; __VA_ARGS__; } \
+    case 96: { constexpr int NN = 96; __VA_ARGS__; } \
+    case 100: { constexpr int NN = 100; __VA_ARGS__; } \
+    case 112: { constexpr int NN = 112; __VA_ARGS__; } \
+    case 192: { constexpr int NN = 192; __VA_ARGS__; } \
+    case 200: { constexpr int NN = 200; __VA_ARGS__; } \
+    case 384: { constexpr int NN = 384; __VA_ARGS__; } \
+    case 400: { constexpr int NN = 400; __VA_ARGS__; }
+#define TFSM_SWITCH_COLS(n, ...)  \
   switch (n) {                  \
-    case 16: { constexpr int NN = 16; BODY; } \
-    case 32: { constexpr int NN = 32; BODY; } \
-    case 64: { constexpr int NN = 64; BODY; } \
-    case 128: { constexpr int NN = 128; BODY; } \
-    case 256: { constexpr int NN = 256; BODY; } \
-    case 512: { constexpr int NN = 512; BODY; } \
-    case 1024: { constexpr int NN = 1024; BODY; } \
-    case 2048: { constexpr int NN = 2048; BODY; } \
-    case 4096: { constexpr int NN = 4096; BODY; } \
-    case 48: { constexpr int NN = 48; BODY; } \
-    case 96: { constexpr int NN = 96; BODY; } \
-    case 100: { constexpr int NN = 100; BODY; } \
-    case 112: { constexpr int NN = 112; BODY; } \
-    case 192: { constexpr int NN = 192; BODY; } \
-    case 200: { constexpr int NN = 200; BODY; } \
-    case 384: { constexpr int NN = 384; BODY; } \
-    case 400: { constexpr int NN = 400; BODY; } \
-    case 768: { constexpr int NN = 768; BODY; } \
-    case 800: { constexpr int NN = 800; BODY; } \
+    TFSM_CASES_512(__VA_ARGS__) \
+    default: return hipErrorInvalidValue; \
+  }
+#define TFSM_SWITCH_N(n, ...)  \
+  switch (n) {                  \
+    TFSM_CASES_512(__VA_ARGS__) \
+    case 1024: { constexpr int NN = 1024; __VA_ARGS__; } \
+    case 2048: { constexpr int NN = 2048; __VA_ARGS__; } \
+    case 4096: { constexpr int NN = 4096; __VA_ARGS__; } \
+    case 768: { constexpr int NN = 768; __VA_ARGS__; } \
+    case 800: { constexpr int NN = 800; __VA_ARGS__; } \
     default: return hipErrorInvalidValue; \
   }
 
@@ -671,10 +679,9 @@ hipError_t launch_cols_c2c(int n, int dir, const float2* in, float2* out, size_t
                            size_t col_stride, int ninner, float scale, const float2* tw, hipStream_t st,
                            StepMask mask, int b0, size_t outer_per_sample) {
   if (nouter == 0 || ninner <= 0) return hipSuccess;
-  if (n > 512) return hipErrorInvalidValue;
   if (mask.act && (outer_per_sample == 0 || nouter > 0xffffffffu)) return hipErrorInvalidValue;
-  TFSM_SWITCH_N(n, {
-    constexpr int V = (NN > 512) ? 1 : ((Fft<NN>::NT * 16 <= 1024) ? 16 : 8);
+  TFSM_SWITCH_COLS(n, {
+    constexpr int V = Fft<NN>::NT * 16 <= 1024 ? 16 : 8;
     // grid.y is limited to 65535: launch the outer blocks in chunks
     for (size_t o0 = 0; o0 < nouter; o0 += 65535) {
       const size_t no = (nouter - o0) < 65535 ? (nouter - o0) : 65535;
@@ -700,9 +707,8 @@ hipError_t launch_cols_linear(int n, float2* u, size_t nouter, size_t outer_stri
                               const float2* tw, const float* E, const float2* Ec, size_t e_bstride, int C, int nsteps,
                               hipStream_t st) {
   if (nouter == 0 || ninner <= 0) return hipSuccess;
-  if (n > 512) return hipErrorInvalidValue;
-  TFSM_SWITCH_N(n, {
-    constexpr int V = (NN > 512) ? 1 : ((Fft<NN>::NT * 16 <= 1024) ? 16 : 8);
+  TFSM_SWITCH_COLS(n, {
+    constexpr int V = Fft<NN>::NT * 16 <= 1024 ? 16 : 8;
     for (size_t o0 = 0; o0 < nouter; o0 += 65535) {
       const size_t no = (nouter - o0) < 65535 ? (nouter - o0) : 65535;
       const dim3 grid((ninner + V - 1) / V, (unsigned)no);
