@@ -259,3 +259,17 @@ def test_2d_run_time_lengths_with_few_columns(dev, kind, shape, batch, path):
         plan.step(uh, 3)
         res.append(plan.inverse(uh))
     assert _rel(res[0], res[1]) <= TOL and bool(torch.isfinite(res[0]).all())
+
+
+@pytest.mark.parametrize("shape", [(16,), (17,), (100,), (4096,), (64, 48), (30, 34), (1024, 32), (16, 16, 16), (6, 5, 4), (8, 8, 2)])
+def test_forward_writes_its_padding_into_a_given_spectrum(dev, shape):
+    """tfsm_plan_forward_fills: where it says so, forward() overwrites every element of a spectrum full of NaN, the
+    padded columns with zeros; elsewhere it leaves the padded columns alone."""
+    plan = _plan(None, shape, 2, dev)
+    u = torch.randn(2, 1, *shape, generator=torch.Generator().manual_seed(1)).to(dev)
+    out = torch.full((2, 1) + shape[:-1] + (plan.pitch,), complex(float("nan"), float("nan")), dtype=torch.complex64, device=dev)
+    plan.forward(u, out)
+    h = shape[-1] // 2 + 1
+    assert bool(torch.isfinite(torch.view_as_real(out[..., :h])).all())
+    pad = torch.view_as_real(out[..., h:])
+    assert bool((pad == 0).all()) if plan._forward_fills else bool(pad.isnan().all())
