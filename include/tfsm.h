@@ -93,14 +93,16 @@ int tfsm_version(void);
 
 /* Compile an operator on a mesh into a plan: symbols, dealias limits, twiddle tables, L.
  * Any mesh of >= 2 points per axis is accepted (the reference transforms any length,
- * mesh.py:481-491).  The fused step kernels cover 1D powers of two 32..4096 and 48, 96, 100, 112,
+ * mesh.py:481-491).  The fixed-size fused step kernels cover 1D powers of two 32..4096 and 48, 96, 100, 112,
  * 192, 200, 384, 400, 768, 800 points, and 1D products above 4096 of two of those lengths from 64 to
  * 1024 (Convection and ConservativeConvection with a real L); 2D axes of powers of two 16..1024 and 48, 96, 100, 112, 192,
- * 200; 3D axes of powers of two 16..256 and cubic 48, 96, 100 meshes.  Other plans (other sizes,
- * ConservativeConvection in 3D, a complex L with a product term in 2D / 3D, NSPressureConvection
- * with an external force, tfsm_plan_add_force) step through the
- * unfused path: separate field, product and stage launches with general-length FFTs (Stockham with
- * radices 2..7 in LDS, Bluestein for other lengths, four-step beyond 4096 points).
+ * 200; 3D axes of powers of two 16..256 and cubic 48, 96, 100 meshes.  Fused kernels of run-time length cover the
+ * other 1D meshes whose transforms take at most 4096 points (Convection and ConservativeConvection) and, with
+ * a real L, the other 2D meshes whose axes fit the LDS (VorticityConvection, Convection, NSPressureConvection and
+ * KSConvection; about 3700 points per axis, 2048 where a prime factor is beyond 13).  Other plans (other sizes, ConservativeConvection in 3D, a complex L
+ * with a product term in 2D / 3D, NSPressureConvection with an external force, tfsm_plan_add_force) step
+ * through the unfused path: separate field, product and stage launches with general-length FFTs (Stockham with
+ * radices 2..16 in LDS, Bluestein for other lengths, four-step beyond 4096 points).  tfsm_plan_path says which.
  * Replaces OperatorLike.register_mesh + _build_linear_coefs + _build_nonlinear_funcs
  * (_base.py:339-406, 581-624) and the FourierMesh symbol caches (mesh.py:399-461). */
 int tfsm_plan_create(const tfsm_geometry* geom, const tfsm_terms* terms, void* stream, tfsm_plan** out);

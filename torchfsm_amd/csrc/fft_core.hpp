@@ -208,8 +208,8 @@ template <> struct FftPlan<384, 0> { static constexpr int RMAX = 12; static cons
 template <> struct FftPlan<400, 0> { static constexpr int RMAX = 20; static constexpr int NST = 4; static constexpr int R[5] = {4, 4, 5, 5, 0}; };
 template <> struct FftPlan<768, 0> { static constexpr int RMAX = 12; static constexpr int NST = 5; static constexpr int R[5] = {4, 4, 4, 4, 3}; };
 template <> struct FftPlan<800, 0> { static constexpr int RMAX = 20; static constexpr int NST = 5; static constexpr int R[5] = {4, 4, 2, 5, 5}; };
-// VAR 1: twice the elements per thread (half the threads per transform), same radix sequence
-// where possible; lets a column tile of the same width run with half the workgroup size.
+// VAR 1: half the elements per thread of VAR 0 (256, 1024, 2048 and 4096 points: fewer registers, shorter chains),
+// twice at 512 points, where a column tile of the same width then runs with half the workgroup size.
 template <> struct FftPlan<256, 1> { static constexpr int RMAX = 8; static constexpr int NST = 3; static constexpr int R[5] = {8, 8, 4, 0, 0}; };
 template <> struct FftPlan<512, 1> { static constexpr int RMAX = 16; static constexpr int NST = 3; static constexpr int R[5] = {8, 8, 8, 0, 0}; };
 // (1024: half the elements per thread of VAR 0, for 2D columns of 1024 points)

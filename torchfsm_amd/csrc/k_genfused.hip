@@ -12,10 +12,10 @@
 // and FFT stages.  So loads are issued in batches ahead of their use, a stage is a butterfly of a
 // few values per thread, a pass transforms several fields of its lines at once where LDS holds them, and the
 // workgroups are kept small enough to fill the GPU.
-// SETDRK4 step, us, on the unfused path and here: vorticity 225 x 301 B = 1 321 -> 146, B = 4 545 -> 230, B = 32
-// 2210 -> 935; 768^2 B = 4 1057 -> 585; 60 x 72 B = 64 370 -> 116; Burgers 150^2 B = 8 403 -> 133; NSP 172^2 B = 1
-// 306 -> 185; 1D Burgers 1000 B = 1 121 -> 34, 767 B = 15 219 -> 69, 3000 B = 8 235 -> 48.  One field at a time
-// in its workgroup 225 x 301 B = 4 took 267 (columns 32 us against 21) and 172^2 B = 1 350.
+// SETDRK4 step, us, on the unfused path and here: vorticity 225 x 301 B = 1 275 / 135, B = 4 421 / 224, B = 32
+// 1330 / 937; 768^2 B = 4 755 / 585; 60 x 72 B = 64 319 / 117; Burgers 150^2 B = 8 328 / 133; NSP 172^2 B = 1
+// 284 / 167; 1D Burgers 1000 B = 1 102 / 34, 767 B = 15 160 / 64, 3000 B = 8 161 / 48.  With one field at a time
+// in its workgroup columns of 225 x 301 B = 4 took 32 us against 21, a step of 172^2 B = 1 350 against 185.
 #include "engine.hpp"
 #include "gx_core.hpp"
 #include "k_step2d.hpp"

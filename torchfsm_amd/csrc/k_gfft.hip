@@ -10,8 +10,8 @@
 // transforms chain these launches through a scratch buffer.
 //
 // Bound by latency and instruction issue, not bandwidth.  Forward transforms, us, before (radices 2..7, one
-// element's load at a time, 16 adjacent lines or one) and now: 65536 points, B = 16 57 -> 30; 225 x 301,
-// B = 16 65 -> 46; 1000^2, B = 4 89 -> 56; 120^3, B = 3 110 -> 82; 84 x 76 x 96, B = 3 65 -> 52.
+// element's load at a time, 16 adjacent lines or one) and now: 65536 points, B = 16 58 -> 27; 225 x 301,
+// B = 16 65 -> 43; 1000^2, B = 4 94 -> 60; 120^3, B = 3 119 -> 90; 84 x 76 x 96, B = 3 69 -> 51.
 #include <cmath>
 #include <complex>
 #include <vector>

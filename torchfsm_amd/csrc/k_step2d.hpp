@@ -776,7 +776,7 @@ struct Run2Shape {
   using F = Fft<N, VAR>;
   static constexpr int NT = F::NT;               // threads per transform (rows and columns)
   static constexpr int V = N;                    // one column tile holds all N/2 + 1 columns
-  static constexpr int THREADS = NT * V;         // 256 (N = 32), 512 or 1024 (N = 64)
+  static constexpr int THREADS = NT * V;         // 256 (N = 32), 1024 (N = 64)
   static constexpr int ROWS = THREADS / NT;      // = N: every row in one pass
   static constexpr int PDR = F::PD < 16 ? F::PD : 16;
   // fields of a row (all of them, or one by one: three regions of 64 Convection rows exceed the LDS) and of a
